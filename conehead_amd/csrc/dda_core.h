@@ -1,7 +1,8 @@
 // dda_core.h -- FP64 3D-DDA step shared by the trace, plan and TERMA kernels.
 //
 // Same operations as conehead/dda_3d_c.pyx:33-99: step sign from d < 0,
-// |d| in place, t = (s/2)/|d| and dt = s/|d| (1e9 for a zero component),
+// |d| in place, t = (s/2)/|d| and dt = s/|d| (1e9 for a zero component;
+// halving is exact, so t is taken as dt/2, the same bits from one division),
 // then repeated t += dt (never a closed form) and the tie rules
 //   t_x < t_y && t_x < t_z -> x;  t_x < t_y -> z;  t_y < t_z -> y;  else z.
 // Files including this header are compiled with -ffp-contract=off.
@@ -26,11 +27,11 @@ struct Dda {
         d1 = d1 < 0 ? -d1 : d1;
         d2 = d2 < 0 ? -d2 : d2;
         if (d0 == 0.0) { t0 = kBig; dt0 = kBig; }
-        else { t0 = (v0 / 2) / d0; dt0 = v0 / d0; }
+        else { dt0 = v0 / d0; t0 = dt0 / 2; }
         if (d1 == 0.0) { t1 = kBig; dt1 = kBig; }
-        else { t1 = (v1 / 2) / d1; dt1 = v1 / d1; }
+        else { dt1 = v1 / d1; t1 = dt1 / 2; }
         if (d2 == 0.0) { t2 = kBig; dt2 = kBig; }
-        else { t2 = (v2 / 2) / d2; dt2 = v2 / d2; }
+        else { dt2 = v2 / d2; t2 = dt2 / 2; }
     }
 
     // Axis chosen at the current voxel (dda_3d_c.pyx:80-99).

@@ -349,97 +349,123 @@ __device__ __forceinline__ void wave_lds_sync()
 // Radiological depth from voxel (x, y, z) toward the source: the FP64 DDA
 // of conehead/conehead.py:138-166 (the traversal of dda_3d_c.pyx:76-99,
 // the same t-values, voxels and tie rules as ch_dda_3d), each voxel's
-// density times its path length summed in FP32 with Kahan compensation, in
-// path order (conehead.py:249-254).  The step needs no branch.  The tie
+// density times its path length summed in FP64, in path order
+// (conehead.py:249-254).  The step needs no branch.  The tie
 // rules (x if t0 < t1 and t0 < t2, else y if t1 <= t0 and t1 < t2, else z)
 // take the smallest crossing t = min(t0, t1, t2) and, among the axes that
 // reach it, z before y before x: z when t2 == t, else y when t1 == t, else
 // x.  The axis taken advances by t_a = fma(dt_a, 1, t_a), the others by
 // fma(dt_a, 0, t_a) = t_a, both rounded as t_a + dt_a and t_a are.
 // kWalkBatch steps are traversed first and their density loads issued
-// together before the first is used; lanes past the grid exit keep
-// stepping with their sums frozen, their range-checked loads reading 0
-// wherever they land.  Byte offsets are 32-bit (ch_terma requires
-// 4 X Y Z < 2^32).  PACK (every axis of at most kPackMax voxels): the
-// steps left before each axis leaves the grid are one word of three 10-bit
-// fields, field a = 511 - left_a counting up, whose top bit (the guard) is
-// set on the step that takes axis a past the grid, when left_a would go
-// below zero; one select, one add and one test per step instead of three
-// counters.  A field stops at most kWalkBatch - 1 steps past 512, far from
-// carrying into the next.
+// together before the first is used.
+//
+// The walk leaves the grid at the first of the axes' last crossings,
+// t_a + left_a dt_a (left_a: steps until axis a is at its last voxel), so
+// a step is taken while the crossing before it lies below that exit.  The
+// product differs from the repeated sum by at most a few hundred roundings,
+// about 1e-13 of t, so the exit is brought in by 1e-12 of itself: no step
+// past the grid is ever counted, and a last segment that short (a tie at
+// the corner of the grid) adds less than 1e-12 of the depth.  A lane past
+// its exit keeps stepping with a zero density until its wavefront's batch
+// ends, its range-checked loads reading 0 wherever they fall outside the
+// grid.  Byte offsets are 32-bit (ch_terma requires 4 X Y Z < 2^32).
+//
+// 17 VALU instructions per step, against 28 when the steps left were
+// counted per axis and the sum was FP32 with Kahan compensation (FP64 runs
+// at the FP32 rate here, so the FP64 sum needs two instructions where the
+// compensated one needs seven); the 128^3 beam 127.4 -> 125.8 us, 24 MLC
+// beams 4439 -> 4217 us.  What bounds the walk are its loads: each touches
+// one line per (x, y) row the wavefront's lanes stand on.
 constexpr int kWalkBatch = 8;
-constexpr int kPackMax = 512;
+constexpr int kWalkTail = 4;
 
-template <bool PACK>
-__device__ __forceinline__ float depth_walk_t(const float* __restrict__ rho,
-                                              int X, int Y, int Z, int x,
-                                              int y, int z, const Dda& d)
+struct Walk {
+    double t0, t1, t2, dt0, dt1, dt2;   // next crossings and their steps
+    double tprev, exit, depth;
+    uint32_t off;                       // byte offset of the voxel
+};
+
+// N steps (byte strides st0, st1, st2); GUARD: a step past the exit adds
+// nothing.
+template <int N, bool GUARD>
+__device__ __forceinline__ void walk_steps(Walk& w, int32_t st0, int32_t st1,
+                                           int32_t st2,
+                                           __amdgpu_buffer_rsrc_t rsrc)
 {
-    double t0 = d.t0, t1 = d.t1, t2 = d.t2;
-    const double dt0 = d.dt0, dt1 = d.dt1, dt2 = d.dt2;
+    float r[N];
+    double seg[N];
+    bool use[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        use[k] = !GUARD || w.tprev < w.exit;
+        const double t = fmin(fmin(w.t0, w.t1), w.t2);
+        // masks in scalar registers: two compares per step
+        const uint64_t b2 = __builtin_amdgcn_ballot_w64(w.t2 == t);
+        const uint64_t b1 = __builtin_amdgcn_ballot_w64(w.t1 == t) & ~b2;
+        const bool m2 = __builtin_amdgcn_inverse_ballot_w64(b2);
+        const bool m1 = __builtin_amdgcn_inverse_ballot_w64(b1);
+        const bool m0 = __builtin_amdgcn_inverse_ballot_w64(~(b1 | b2));
+        r[k] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+            rsrc, (int)w.off, 0, 0));
+        seg[k] = t - w.tprev;
+        w.tprev = t;
+        w.t0 = fma(w.dt0, m0 ? 1.0 : 0.0, w.t0);
+        w.t1 = fma(w.dt1, m1 ? 1.0 : 0.0, w.t1);
+        w.t2 = fma(w.dt2, m2 ? 1.0 : 0.0, w.t2);
+        w.off += (uint32_t)(m0 ? st0 : (m1 ? st1 : st2));
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        float rho = r[k];
+        if (GUARD) {
+            rho = use[k] ? rho : 0.0f;
+            // keeps the select in one FP32 register
+            asm("" : "+v"(rho));
+        }
+        w.depth = fma((double)rho, seg[k], w.depth);
+    }
+}
+
+__device__ __forceinline__ float depth_walk(const float* __restrict__ rho,
+                                            int X, int Y, int Z, int x, int y,
+                                            int z, const Dda& d)
+{
+    Walk w;
+    w.t0 = d.t0;
+    w.t1 = d.t1;
+    w.t2 = d.t2;
+    w.dt0 = d.dt0;
+    w.dt1 = d.dt1;
+    w.dt2 = d.dt2;
     // steps left before each axis leaves the grid
-    int32_t left0 = d.s0 > 0 ? X - 1 - x : x;
-    int32_t left1 = d.s1 > 0 ? Y - 1 - y : y;
-    int32_t left2 = d.s2 > 0 ? Z - 1 - z : z;
-    constexpr uint32_t kGuards = (1u << 9) | (1u << 19) | (1u << 29);
-    uint32_t pk = PACK ? (511u - (uint32_t)left0) |
-                             ((511u - (uint32_t)left1) << 10) |
-                             ((511u - (uint32_t)left2) << 20)
-                       : 0u;
-    // byte strides and offset
+    const int32_t left0 = d.s0 > 0 ? X - 1 - x : x;
+    const int32_t left1 = d.s1 > 0 ? Y - 1 - y : y;
+    const int32_t left2 = d.s2 > 0 ? Z - 1 - z : z;
+    w.exit = fmin(fmin(fma((double)left0, d.dt0, d.t0),
+                       fma((double)left1, d.dt1, d.t1)),
+                  fma((double)left2, d.dt2, d.t2)) *
+             (1.0 - 1e-12);
     const int32_t st0 = 4 * d.s0 * Y * Z, st1 = 4 * d.s1 * Z, st2 = 4 * d.s2;
-    uint32_t off = 4u * (uint32_t)((x * Y + y) * Z + z);
-    double tprev = 0.0;
-    float de = 0.0f, dc = 0.0f;
-    bool live = true;
-    // range-checked loads: past the grid a read returns 0 (and is not used)
+    w.off = 4u * (uint32_t)((x * Y + y) * Z + z);
+    w.tprev = 0.0;
+    w.depth = 0.0;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void*)rho, (short)0, 4 * X * Y * Z, kBufferFlags);
-    while (live) {
-        uint32_t offs[kWalkBatch];
-        float seg[kWalkBatch];
-        bool use[kWalkBatch];
-#pragma unroll
-        for (int k = 0; k < kWalkBatch; ++k) {
-            use[k] = live;
-            const double t = fmin(fmin(t0, t1), t2);
-            const bool m2 = t2 == t;
-            const bool m1 = !m2 & (t1 == t);
-            const bool m0 = !(m1 | m2);
-            offs[k] = off;
-            seg[k] = (float)(t - tprev);
-            tprev = t;
-            t0 = fma(dt0, m0 ? 1.0 : 0.0, t0);
-            t1 = fma(dt1, m1 ? 1.0 : 0.0, t1);
-            t2 = fma(dt2, m2 ? 1.0 : 0.0, t2);
-            off += (uint32_t)(m0 ? st0 : (m1 ? st1 : st2));
-            if (PACK) {
-                pk += m0 ? 1u : (m1 ? (1u << 10) : (1u << 20));
-                live = live & ((pk & kGuards) == 0u);
-            } else {
-                left0 -= (int32_t)m0;
-                left1 -= (int32_t)m1;
-                left2 -= (int32_t)m2;
-                live = live & ((left0 | left1 | left2) >= 0);
-            }
-        }
-        float r[kWalkBatch];
-#pragma unroll
-        for (int k = 0; k < kWalkBatch; ++k)
-            r[k] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                rsrc, (int)offs[k], 0, 0));
-#pragma unroll
-        for (int k = 0; k < kWalkBatch; ++k) {
-            // a step past the exit adds dc: yk = 0, de keeps its bits (dc
-            // is not used after the walk)
-            const float term = use[k] ? r[k] * seg[k] : dc;
-            const float yk = term - dc;
-            const float tk = de + yk;
-            dc = (tk - de) - yk;
-            de = tk;
-        }
-    }
-    return de;
+    // The last of kWalkBatch steps starts at most `ahead` from here: axis a
+    // crosses at least D / dt_a - 1 times in any distance D, and the axis
+    // of the shortest step D / dt times (its next crossing lies within dt).
+    // Rounded up by far more than FP32 loses.
+    constexpr float kBefore = kWalkBatch - 1;
+    const float i0 = 1.0f / (float)d.dt0, i1 = 1.0f / (float)d.dt1,
+                i2 = 1.0f / (float)d.dt2;
+    const float ahead = 1.00001f * fminf(kBefore / fmaxf(fmaxf(i0, i1), i2),
+                                         (kBefore + 3.0f) / (i0 + i1 + i2));
+    const double safe = w.exit - (double)ahead;
+    while (w.tprev < safe)
+        walk_steps<kWalkBatch, false>(w, st0, st1, st2, rsrc);
+    while (w.tprev < w.exit)
+        walk_steps<kWalkTail, true>(w, st0, st1, st2, rsrc);
+    return (float)w.depth;
 }
 // Sub-sample values staged per wavefront by the compacted hit test.
 constexpr int kSampleBuf = 512;
@@ -686,7 +712,6 @@ __global__ __launch_bounds__(256) void terma_sort_set_kernel(
 // test gave v: hit-test stages 2 and 3, then per voxel the radiological
 // depth, off-axis distance, fluence, softening, horn and the polyenergetic
 // sum (conehead.py:71-377).  Returns the lane's T (0 outside the grid).
-template <bool PACK>
 __device__ __forceinline__ float terma_brick(const TermaParams& P,
                                              const Brick& k, float v, int l,
                                              double* __restrict__ s_samp,
@@ -821,7 +846,7 @@ __device__ __forceinline__ float terma_brick(const TermaParams& P,
             d.init(dir[0], dir[1], dir[2], P.spacing[0], P.spacing[1],
                    P.spacing[2]);
             const float de =
-                depth_walk_t<PACK>(P.density, P.X, P.Y, P.Z, x, y, z, d);
+                depth_walk(P.density, P.X, P.Y, P.Z, x, y, z, d);
 
             // off-axis distance (conehead.py:286-314)
             double oad = 0.0;
@@ -886,7 +911,6 @@ __device__ __forceinline__ float terma_brick(const TermaParams& P,
 // descending cost class, so the longest depth walks are dispatched first
 // and the rest fill in behind them (wavefronts past the last brick exit at
 // once).  Each wavefront writes its support-box partial.
-template <bool PACK>
 __device__ __forceinline__ void terma_wave(const TermaParams& P, int g,
                                            int l, double* __restrict__ s_samp,
                                            int32_t* __restrict__ s_lane,
@@ -957,7 +981,7 @@ __device__ __forceinline__ void terma_wave(const TermaParams& P, int g,
             const float v =
                 (e & 3) == 1 ? 1.0f : ((e & 3) == 2 ? -1.0f : 0.0f);
             bool bad = false;
-            T = terma_brick<PACK>(P, k, v, l, s_samp, s_lane, bad);
+            T = terma_brick(P, k, v, l, s_samp, s_lane, bad);
             if (__ballot(bad) != 0 && l == 0)
                 atomicOr(P.status, 1);
             x = k.x0 + (l >> 4);
@@ -990,16 +1014,14 @@ __device__ __forceinline__ void terma_wave(const TermaParams& P, int g,
     }
 }
 
-// PACK: every axis of the grid has at most kPackMax voxels (depth_walk_t).
-template <bool PACK>
 __global__ __launch_bounds__(256) void terma_kernel(TermaParams P,
                                                     int32_t n_bricks)
 {
     __shared__ double s_samp[4][kSampleBuf];
     __shared__ int32_t s_lane[4][64];
     const int w = threadIdx.x >> 6;
-    terma_wave<PACK>(P, blockIdx.x * 4 + w, threadIdx.x & 63, s_samp[w],
-                     s_lane[w], n_bricks);
+    terma_wave(P, blockIdx.x * 4 + w, threadIdx.x & 63, s_samp[w], s_lane[w],
+               n_bricks);
 }
 
 // Phase 2 of several beams in one launch, beam by beam (the blocks of beam
@@ -1007,7 +1029,6 @@ __global__ __launch_bounds__(256) void terma_kernel(TermaParams P,
 // or two beams, whose rays toward one source cross the same density lines
 // and read one aperture table, so they share the caches; the next beam's
 // longest walks start while the last of the previous beam finish.
-template <bool PACK>
 __global__ __launch_bounds__(256) void terma_set_kernel(
     const TermaParams* __restrict__ tab, int32_t n_bricks,
     int32_t blocks_per_beam)
@@ -1017,7 +1038,7 @@ __global__ __launch_bounds__(256) void terma_set_kernel(
     const int w = threadIdx.x >> 6;
     const int beam = blockIdx.x / blocks_per_beam;
     const int g = (blockIdx.x - beam * blocks_per_beam) * 4 + w;
-    terma_wave<PACK>(tab[beam], g, threadIdx.x & 63, s_samp[w], s_lane[w],
+    terma_wave(tab[beam], g, threadIdx.x & 63, s_samp[w], s_lane[w],
                n_bricks);
 }
 
@@ -1226,8 +1247,6 @@ static ch_status terma_launch(const TermaParams* h, const TermaParams* d_tab,
 {
     const unsigned bpb = (unsigned)((n_bricks + 3) / 4);
     const unsigned spb = (unsigned)sort_blocks(h[0].X, h[0].Y, h[0].Z);
-    const bool pack =
-        h[0].X <= kPackMax && h[0].Y <= kPackMax && h[0].Z <= kPackMax;
     if (clear) {
         const int nc = n * kCounterInts;
         hipLaunchKernelGGL(terma_clear_kernel,
@@ -1237,17 +1256,15 @@ static ch_status terma_launch(const TermaParams* h, const TermaParams* d_tab,
     if (!d_tab) {
         hipExtLaunchKernelGGL(terma_sort_kernel, dim3(spb), dim3(256), 0, s,
                               ev0, nullptr, 0, h[0]);
-        hipExtLaunchKernelGGL(pack ? terma_kernel<true> : terma_kernel<false>,
-                              dim3(bpb), dim3(256), 0, s, nullptr, ev1, 0,
-                              h[0], n_bricks);
+        hipExtLaunchKernelGGL(terma_kernel, dim3(bpb), dim3(256), 0, s,
+                              nullptr, ev1, 0, h[0], n_bricks);
     } else {
         hipExtLaunchKernelGGL(terma_sort_set_kernel, dim3(spb * n),
                               dim3(256), 0, s, ev0, nullptr, 0, d_tab,
                               (int32_t)spb);
-        hipExtLaunchKernelGGL(pack ? terma_set_kernel<true>
-                                   : terma_set_kernel<false>,
-                              dim3(bpb * n), dim3(256), 0, s, nullptr, ev1, 0,
-                              d_tab, n_bricks, (int32_t)bpb);
+        hipExtLaunchKernelGGL(terma_set_kernel, dim3(bpb * n), dim3(256), 0,
+                              s, nullptr, ev1, 0, d_tab, n_bricks,
+                              (int32_t)bpb);
     }
     CH_HIP(hipGetLastError());
     for (int32_t i = 0; i < n; ++i)
