@@ -4,6 +4,7 @@
 // array.  Cell values come from aperture.h, the same functions the TERMA
 // hit test evaluates analytically.
 #include <cstdlib>
+#include <cstring>
 #include <vector>
 
 #include "aperture.h"
@@ -58,7 +59,7 @@ ch_status ch_raster_square(float* d_raster, double length, void* stream)
 
 int32_t ch_mlc_table_len(int32_t n_pairs)
 {
-    return mlc_row_table_start(n_pairs) + 4 * kMlcRows;
+    return mlc_row_table_start(n_pairs) + 5 * kMlcRows;
 }
 
 ch_status ch_mlc_table(int32_t* d_table, int32_t n_pairs,
@@ -81,7 +82,7 @@ ch_status ch_mlc_table(int32_t* d_table, int32_t n_pairs,
                    n, h_a[n], h_b[n]);
     }
     const int rt = mlc_row_table_start(n_pairs);
-    std::vector<int32_t> t(rt + 4 * kMlcRows, 0);
+    std::vector<int32_t> t(rt + 5 * kMlcRows, 0);
     t[0] = n_pairs;
     t[1] = W;
     t[2] = 2000 - W / 2;                         // bank centred on row 2000
@@ -101,14 +102,24 @@ ch_status ch_mlc_table(int32_t* d_table, int32_t n_pairs,
     // whose rows [bound[n] + shift, + width) hold the row (the last pair
     // starting at or before it), or open when none does.
     const int shift = abs(h_bound[0]);
+    auto bits = [](float f) {
+        int32_t v;
+        memcpy(&v, &f, sizeof v);
+        return v;
+    };
+    std::vector<int32_t> pair(kMlcRows);   // -2 closed, -1 open
     for (int row = 0; row < kMlcRows; ++row) {
         int32_t* e = &t[rt + 4 * row];
         const int rr = row - t[2];
+        e[1] = kMlcFar;
         if (rr < 0 || rr >= W || rr < t[5] || rr >= t[6]) {
-            e[0] = kRowClosed;
+            pair[row] = -2;
+            e[0] = kMlcFar;
+            e[2] = bits(1.0f);
             continue;
         }
-        e[0] = kRowOpen;
+        pair[row] = -1;
+        e[0] = -kMlcFar;
         if (h_bound[0] + shift > rr)
             continue;
         int lo = 0;
@@ -117,11 +128,25 @@ ch_status ch_mlc_table(int32_t* d_table, int32_t n_pairs,
         const int rmin = h_bound[lo] + shift;
         const int w = abs(h_bound[lo + 1] - h_bound[lo]);
         if (rr < rmin + w) {
-            e[0] = kRowLeaf;
-            e[1] = 2000 + h_a[lo];
-            e[2] = 2000 + h_b[lo];
-            e[3] = ((rr - rmin) << 16) | w;
+            pair[row] = lo;
+            e[0] = 2000 + h_a[lo];
+            e[1] = 2000 + h_b[lo];
+            e[2] = bits(leaf_edge(rr - rmin, w));
+            e[3] = bits(leaf_edge(w - 1 - (rr - rmin), w));
         }
+    }
+    // run ends, from the last row up
+    int32_t* runs = &t[rt + 4 * kMlcRows];
+    int leaf_end = kMlcRows - 1, same_end = kMlcRows - 1;
+    for (int row = kMlcRows - 1; row >= 0; --row) {
+        const int32_t* e = &t[rt + 4 * row];
+        if (row + 1 < kMlcRows) {
+            if (pair[row] != pair[row + 1])
+                leaf_end = row;
+            if (memcmp(e, e + 4, 4 * sizeof(int32_t)) != 0)
+                same_end = row;
+        }
+        runs[row] = (leaf_end << 16) | same_end;
     }
     if (h_bbox_out) {
         // Every nonzero cell lies inside the bank rows, the Y-jaw rows and

@@ -49,18 +49,23 @@ struct TermaParams {
     int32_t* status;           // geometry error flag
     int32_t accumulate;        // terma += this beam
     // per-launch constants, computed on the host with the kernel's own
-    // operations: sub-sample steps spacing / n, n . source, n^3, and the
-    // blocked fraction of a fully open voxel (1 / n^3 added n^3 times)
+    // operations: sub-sample steps spacing / n, n . source and n^3
     double off[3];
     double ndotn_src;
     double n3;
-    double blocked_one;
-    float inv_n3, inv_ns;
+    float inv_ns;
     float src_vox[3];          // (src - origin) / spacing, for cost classes
     // 100 tr0.src, 100 tr2.src and -100 n.src, for fast_cells, which is
     // used only when |ci_src|, |cj_src| < 1e5 (fast_ok)
     double ci_src, cj_src, k100;
     int32_t fast_ok;
+    // what n.u, tr0.u and tr2.u (u = source - sample) change by per
+    // sub-sample along each axis, and from the first to the last
+    double step_d[3], step_i[3], step_j[3];
+    double span_d[3], span_i[3], span_j[3];
+    // cell coordinates of the source's own image, ci_src + 1999: a cell is
+    // the floor of a coordinate counted from there
+    double ci_cell, cj_cell;
 };
 
 __device__ __forceinline__ double dot3(const double* a, double b0, double b1,
@@ -231,6 +236,11 @@ struct CellBox {
     {
         return (flags & 1) && (flags & 6);
     }
+    // every cell of the box is a raster cell that no index wraps to
+    __device__ __forceinline__ bool inside_raster() const
+    {
+        return ok() && a_i >= 0 && b_i <= 3998 && a_j >= 0 && b_j <= 3998;
+    }
     // The transmission shared by every sub-sample whose image lies in the
     // box, or -1 when it is not one known constant: 0 outside the
     // aperture's bounding cells or the raster, or the leaf table's or the
@@ -242,8 +252,7 @@ struct CellBox {
         if (axis_misses(a_i, b_i, P.ap_bbox[0], P.ap_bbox[1]) ||
             axis_misses(a_j, b_j, P.ap_bbox[2], P.ap_bbox[3]))
             return 0.0f;
-        if (P.ap_kind == CH_APERTURE_RASTER ||
-            !(a_i >= 0 && b_i <= 3998 && a_j >= 0 && b_j <= 3998))
+        if (P.ap_kind == CH_APERTURE_RASTER || !inside_raster())
             return -1.0f;
         return P.ap_kind == CH_APERTURE_MLC
                    ? mlc_block_value(P.ap_table, a_i, b_i, a_j, b_j)
@@ -337,6 +346,72 @@ __device__ __forceinline__ bool fast_cells(const TermaParams& P, double p0,
            ej < 1.0 - kMargin;
 }
 
+// n.u, tr0.u and tr2.u, u = source - sample: affine in the sample's
+// position, so a voxel's sub-samples follow from its first by additions.
+struct Lines {
+    double d, ni, nj;
+};
+
+// At sub-sample (0, 0, 0) of voxel (x, y, z).
+__device__ __forceinline__ Lines lines_at(const TermaParams& P, int x, int y,
+                                          int z)
+{
+    const double u0 = P.src[0] - sample_pos(P, 0, x, P.off[0], 0),
+                 u1 = P.src[1] - sample_pos(P, 1, y, P.off[1], 0),
+                 u2 = P.src[2] - sample_pos(P, 2, z, P.off[2], 0);
+    Lines L;
+    L.d = fma(P.vy[2], u2, fma(P.vy[1], u1, P.vy[0] * u0));
+    L.ni = fma(P.tr0[2], u2, fma(P.tr0[1], u1, P.tr0[0] * u0));
+    L.nj = fma(P.tr2[2], u2, fma(P.tr2[1], u1, P.tr2[0] * u0));
+    return L;
+}
+
+// -100 n.src / (n.u), the quotient from a reciprocal refined by one Newton
+// step (fast_cells).
+__device__ __forceinline__ double plane_scale(const TermaParams& P, double d)
+{
+    double r = __builtin_amdgcn_rcp(d);
+    r = r * fma(-d, r, 2.0);
+    return P.k100 * r;
+}
+
+// Cell box of the images of a voxel's 8 extreme sub-samples, by fast_cells'
+// evaluation (within 1e-8 cell of plane_image's while every |n.u| >= 1 cm,
+// which the box requires; the box is widened by 1e-6 cell).  As in
+// brick_value it then holds the image of every sub-sample.  The cells are
+// monotone in the coordinate, so the extremes are taken first and floored
+// once: 120 instructions where 8 separate corner images take 370.
+__device__ __forceinline__ void voxel_box(const TermaParams& P,
+                                          const Lines& L, CellBox& b)
+{
+    double dlo = 0, dhi = 0, ilo = 0, ihi = 0, jlo = 0, jhi = 0;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        double d = L.d, ni = L.ni, nj = L.nj;
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            if (c & (1 << a)) {
+                d += P.span_d[a];
+                ni += P.span_i[a];
+                nj += P.span_j[a];
+            }
+        const double s = plane_scale(P, d);
+        const double ci = fma(s, ni, P.ci_src), cj = fma(s, nj, P.cj_src);
+        dlo = c ? fmin(dlo, d) : d;
+        dhi = c ? fmax(dhi, d) : d;
+        ilo = c ? fmin(ilo, ci) : ci;
+        ihi = c ? fmax(ihi, ci) : ci;
+        jlo = c ? fmin(jlo, cj) : cj;
+        jhi = c ? fmax(jhi, cj) : cj;
+    }
+    b.a_i = cell_of(ilo - 1e-6);
+    b.b_i = cell_of(ihi + 1e-6);
+    b.a_j = cell_of(jlo - 1e-6);
+    b.b_j = cell_of(jhi + 1e-6);
+    // CellBox::ok needs bit 0 and one of the sign bits
+    b.flags = P.fast_ok && (dlo >= 1.0 || dhi <= -1.0) ? 3 : 0;
+}
+
 // LDS of one wavefront exchanged between its own lanes: the writes are
 // complete and visible once every lane has passed this point.
 __device__ __forceinline__ void wave_lds_sync()
@@ -344,6 +419,102 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The aperture's value at a cell inside the raster.
+__device__ __forceinline__ float cell_value(const TermaParams& P, int i,
+                                            int j)
+{
+    if (P.ap_kind == CH_APERTURE_MLC)
+        return mlc_value(P.ap_table, i, j);
+    if (P.ap_kind == CH_APERTURE_RECTS)
+        return rects_value(P.ap_table, P.ap_n, i, j);
+    return P.raster[i * 4000 + j];
+}
+
+// Brick of 4 x 4 x 4 voxels.
+struct Brick {
+    int x0, y0, z0;
+};
+
+// Sums of the n^3 sub-sample transmissions of the brick's voxels whose lane
+// is set in todo (mine: this lane's bit), L their Lines; every sample's
+// cell lies inside the raster and |n.u| >= 1 cm (voxel_box).  Every lane of
+// the wavefront calls it.  Where n lanes per voxel are there, one takes each
+// plane of a voxel's samples, so a brick on an edge of the field costs a
+// third of one with every voxel open.  Each sample's lines come from the
+// first's by one addition per axis, its cells as fast_cells certifies them;
+// a cell within 1e-6 of an integer is decided by plane_image.  The
+// transmissions are FP32 values of at most 1 on a grid of 2^-24, so their
+// FP64 sum is exact in any order.  33 instructions per sample against about
+// 100 with each sample's own dot products, quotient and range checks.
+__device__ __forceinline__ double sample_sums(const TermaParams& P,
+                                              const Brick& k, const Lines& L,
+                                              bool mine, uint64_t todo, int l,
+                                              int32_t* __restrict__ s_lane)
+{
+    const int ns = P.samples;
+    const int n = __popcll(todo);
+    const int rank = __popcll(todo & ((1ull << l) - 1ull));
+    const bool split = n * ns <= 64;
+    // the voxel (lane) this lane works for and its planes [ix0, ix1)
+    int src = l, ix0 = 0, ix1 = mine ? ns : 0;
+    Lines W = L;
+    if (split) {
+        if (mine)
+            s_lane[rank] = l;
+        wave_lds_sync();
+        // l / ns by a float reciprocal, exact for l < 64
+        const int q = (int)(((float)l + 0.5f) * P.inv_ns);
+        const bool work = q < n;
+        src = work ? s_lane[q] : l;
+        wave_lds_sync();
+        ix0 = l - q * ns;
+        ix1 = work ? ix0 + 1 : ix0;
+        W.d = __shfl(L.d, src, 64);
+        W.ni = __shfl(L.ni, src, 64);
+        W.nj = __shfl(L.nj, src, 64);
+    }
+    double sum = 0.0;
+    for (int ix = ix0; ix < ix1; ++ix) {
+        for (int iy = 0; iy < ns; ++iy) {
+            const double fx = ix, fy = iy;
+            double d = fma(fy, P.step_d[1], fma(fx, P.step_d[0], W.d));
+            double ni = fma(fy, P.step_i[1], fma(fx, P.step_i[0], W.ni));
+            double nj = fma(fy, P.step_j[1], fma(fx, P.step_j[0], W.nj));
+            for (int iz = 0; iz < ns; ++iz) {
+                const double s = plane_scale(P, d);
+                const double ci = fma(s, ni, P.ci_cell),
+                             cj = fma(s, nj, P.cj_cell);
+                // both are positive: truncation is the floor
+                int i = (int)ci, j = (int)cj;
+                const double e =
+                    fmax(fabs(__builtin_amdgcn_fract(ci) - 0.5),
+                         fabs(__builtin_amdgcn_fract(cj) - 0.5));
+                if (e >= 0.5 - 1e-6) {
+                    const PlaneImage c = plane_image(
+                        P, sample_pos(P, 0, k.x0 + (src >> 4), P.off[0], ix),
+                        sample_pos(P, 1, k.y0 + ((src >> 2) & 3), P.off[1],
+                                   iy),
+                        sample_pos(P, 2, k.z0 + (src & 3), P.off[2], iz),
+                        P.ndotn_src);
+                    i = (int)(floor(c.ci) + 1999.0);
+                    j = (int)(floor(c.cj) + 1999.0);
+                }
+                sum = sum + (double)cell_value(P, i, j);
+                d += P.step_d[2];
+                ni += P.step_i[2];
+                nj += P.step_j[2];
+            }
+        }
+    }
+    if (split) {
+        double all = 0.0;
+        for (int i = 0; i < ns; ++i)
+            all = all + __shfl(sum, (rank * ns + i) & 63, 64);
+        sum = all;
+    }
+    return sum;
 }
 
 // Radiological depth from voxel (x, y, z) toward the source: the FP64 DDA
@@ -467,9 +638,6 @@ __device__ __forceinline__ float depth_walk(const float* __restrict__ rho,
         walk_steps<kWalkTail, true>(w, st0, st1, st2, rsrc);
     return (float)w.depth;
 }
-// Sub-sample values staged per wavefront by the compacted hit test.
-constexpr int kSampleBuf = 512;
-
 // TERMA in two phases.  The hit test (conehead.py:78-120) runs in three
 // stages that each give the exact blocked fraction of the loop over n^3
 // sub-samples: (1) the brick of 64 voxels at once (brick_value), (2) each
@@ -486,9 +654,6 @@ constexpr int kSampleBuf = 512;
 // Bricks of 4 x 4 x 4 voxels (one per wavefront in phase 2), indexed z
 // fastest: the corner voxel of brick b, and lane l's voxel (x0 + l / 16,
 // y0 + l / 4 % 4, z0 + l % 4).
-struct Brick {
-    int x0, y0, z0;
-};
 __device__ __forceinline__ Brick brick_of(const TermaParams& P, int b)
 {
     const int nbz = (P.Z + 3) / 4, nby = (P.Y + 3) / 4;
@@ -663,10 +828,12 @@ __device__ __forceinline__ void sort_block(const TermaParams& P, int blk,
             }
         }
         if (in && !zero && (l & 7) == 0) {
-            q = brick_cost_class(P, k, v < 0.0f);
-            // entry: brick index and stage-1 value (0 -> 0, 1 -> 1, -1 -> 2)
+            const bool edge = v != 0.0f && v != 1.0f;
+            q = brick_cost_class(P, k, edge);
+            // entry: brick index and stage-1 value (0 -> 0, 1 -> 1, any
+            // other -> 2)
             const int b = (bx * g.nby + by) * g.nbz + bz;
-            entry = b * 4 + (v > 0.0f ? 1 : (v < 0.0f ? 2 : 0));
+            entry = b * 4 + (edge ? 2 : (v != 0.0f ? 1 : 0));
             rank = atomicAdd(&s_cnt[q], 1);
         }
     }
@@ -714,7 +881,6 @@ __global__ __launch_bounds__(256) void terma_sort_set_kernel(
 // sum (conehead.py:71-377).  Returns the lane's T (0 outside the grid).
 __device__ __forceinline__ float terma_brick(const TermaParams& P,
                                              const Brick& k, float v, int l,
-                                             double* __restrict__ s_samp,
                                              int32_t* __restrict__ s_lane,
                                              bool& bad)
 {
@@ -725,94 +891,36 @@ __device__ __forceinline__ float terma_brick(const TermaParams& P,
     const int z = z0 + (l & 3);
     const bool inside = x < P.X && y < P.Y && z < P.Z;
     const int ns = P.samples;
-    const int n3i = ns * ns * ns;
     const double n3 = P.n3;
     const double* off = P.off;
     const double ndotn_src = P.ndotn_src;
     float T = 0.0f;
         // 2. the voxel's own corners
+        Lines L;
+        bool inner = false;
         if (v < 0.0f && inside) {
+            L = lines_at(P, x, y, z);
             CellBox b;
-            for (int k = 0; k < 8; ++k) {
-                const int s0 = (k & 1) ? ns - 1 : 0;
-                const int s1 = (k & 2) ? ns - 1 : 0;
-                const int s2 = (k & 4) ? ns - 1 : 0;
-                CellBox c;
-                c.init(corner_image(P, sample_pos(P, 0, x, off[0], s0),
-                                    sample_pos(P, 1, y, off[1], s1),
-                                    sample_pos(P, 2, z, off[2], s2)));
-                if (k == 0)
-                    b = c;
-                else
-                    b.add(c);
-                if (!b.ok())
-                    break;
-            }
+            voxel_box(P, L, b);
             v = b.value(P);
+            inner = b.inside_raster();
         }
-        // box values are 0, 1 or unknown (-1): a known box adds v / n^3
-        // n^3 times, which is 0 or the open fraction
-        double blocked = v > 0.0f ? P.blocked_one : 0.0;
+        // a known box has one value for every sub-sample
+        double blocked = v > 0.0f ? (double)v : 0.0;
 
-        // 3. the sub-samples of the voxels still open: spread over the
-        // lanes when at most two rounds of voxels need them, else each lane
-        // loops over its own (more voxels than that fill the lanes anyway)
+        // 3. the sub-samples of the voxels still open
         const bool need = inside && v < 0.0f;
-        const uint64_t need_mask = __ballot(need);
-        const int n_need = __popcll(need_mask);
-        const int G = n3i <= kSampleBuf ? kSampleBuf / n3i : 0;
-        if (n_need > 0 && n_need <= 2 * G) {
-            double* buf = s_samp;
-            int32_t* lanes = s_lane;
-            const int rank = __popcll(need_mask & ((1ull << l) - 1ull));
-            if (need)
-                lanes[rank] = l;
-            wave_lds_sync();
-            // k / n3 and s / ns by float reciprocals: for k, s < 512 and
-            // divisors <= 512 the product (k + 0.5) / d is off by
-            // < 512 * 2^-23 < 0.5 / 512, less than its distance to an
-            // integer, so the truncation is the integer quotient
-            const float inv_n3 = P.inv_n3;
-            const float inv_ns = P.inv_ns;
-            for (int g0 = 0; g0 < n_need; g0 += G) {
-                const int gn = min(G, n_need - g0);
-                for (int k = l; k < gn * n3i; k += 64) {
-                    const int j = (int)(((float)k + 0.5f) * inv_n3);
-                    const int smp = k - j * n3i;
-                    const int q = (int)(((float)smp + 0.5f) * inv_ns);
-                    const int iz = smp - q * ns;
-                    const int ix = (int)(((float)q + 0.5f) * inv_ns);
-                    const int iy = q - ix * ns;
-                    const int src = lanes[g0 + j];
-                    const double p0 =
-                        sample_pos(P, 0, x0 + (src >> 4), off[0], ix);
-                    const double p1 =
-                        sample_pos(P, 1, y0 + ((src >> 2) & 3), off[1], iy);
-                    const double p2 =
-                        sample_pos(P, 2, z0 + (src & 3), off[2], iz);
-                    double tv = 0.0;  // a sample in the source plane adds 0
-                    double fi, fj;
-                    if (fast_cells(P, p0, p1, p2, fi, fj)) {
-                        tv = (double)transmission_at(P, fi, fj) / n3;
-                    } else {
-                        const PlaneImage c =
-                            plane_image(P, p0, p1, p2, ndotn_src);
-                        if (fabs(c.ndotu) < 1e-6)
-                            bad = true;
-                        else
-                            tv = (double)transmission(P, c.ci, c.cj) / n3;
-                    }
-                    buf[k] = tv;
-                }
-                wave_lds_sync();
-                if (need && rank >= g0 && rank < g0 + gn) {
-                    const double* mine = buf + (rank - g0) * n3i;
-                    for (int smp = 0; smp < n3i; ++smp)
-                        blocked = blocked + mine[smp];
-                }
-                wave_lds_sync();
-            }
-        } else if (need) {
+        const uint64_t todo = __ballot(need && inner);
+        if (todo != 0) {
+            const double sum = sample_sums(P, k, L, need && inner, todo, l,
+                                           s_lane);
+            if (need && inner)
+                blocked = sum / n3;
+        }
+        if (need && !inner) {
+            // the box reaches past the raster or the source plane: each
+            // sample by the definition's own evaluation where it has to be
+            double sum = 0.0;
             for (int ix = 0; ix < ns; ++ix)
                 for (int iy = 0; iy < ns; ++iy)
                     for (int iz = 0; iz < ns; ++iz) {
@@ -821,8 +929,7 @@ __device__ __forceinline__ float terma_brick(const TermaParams& P,
                         const double p2 = sample_pos(P, 2, z, off[2], iz);
                         double fi, fj;
                         if (fast_cells(P, p0, p1, p2, fi, fj)) {
-                            blocked = blocked +
-                                      (double)transmission_at(P, fi, fj) / n3;
+                            sum = sum + (double)transmission_at(P, fi, fj);
                             continue;
                         }
                         const PlaneImage c =
@@ -831,9 +938,9 @@ __device__ __forceinline__ float terma_brick(const TermaParams& P,
                             bad = true;
                             continue;
                         }
-                        blocked = blocked +
-                                  (double)transmission(P, c.ci, c.cj) / n3;
+                        sum = sum + (double)transmission(P, c.ci, c.cj);
                     }
+            blocked = sum / n3;
         }
 
         const bool dbg = P.debug != nullptr;
@@ -912,8 +1019,7 @@ __device__ __forceinline__ float terma_brick(const TermaParams& P,
 // and the rest fill in behind them (wavefronts past the last brick exit at
 // once).  Each wavefront writes its support-box partial.
 __device__ __forceinline__ void terma_wave(const TermaParams& P, int g,
-                                           int l, double* __restrict__ s_samp,
-                                           int32_t* __restrict__ s_lane,
+                                           int l, int32_t* __restrict__ s_lane,
                                            int32_t n_bricks)
 {
     const int32_t* __restrict__ list = P.list;
@@ -981,7 +1087,7 @@ __device__ __forceinline__ void terma_wave(const TermaParams& P, int g,
             const float v =
                 (e & 3) == 1 ? 1.0f : ((e & 3) == 2 ? -1.0f : 0.0f);
             bool bad = false;
-            T = terma_brick(P, k, v, l, s_samp, s_lane, bad);
+            T = terma_brick(P, k, v, l, s_lane, bad);
             if (__ballot(bad) != 0 && l == 0)
                 atomicOr(P.status, 1);
             x = k.x0 + (l >> 4);
@@ -1017,11 +1123,9 @@ __device__ __forceinline__ void terma_wave(const TermaParams& P, int g,
 __global__ __launch_bounds__(256) void terma_kernel(TermaParams P,
                                                     int32_t n_bricks)
 {
-    __shared__ double s_samp[4][kSampleBuf];
     __shared__ int32_t s_lane[4][64];
     const int w = threadIdx.x >> 6;
-    terma_wave(P, blockIdx.x * 4 + w, threadIdx.x & 63, s_samp[w], s_lane[w],
-               n_bricks);
+    terma_wave(P, blockIdx.x * 4 + w, threadIdx.x & 63, s_lane[w], n_bricks);
 }
 
 // Phase 2 of several beams in one launch, beam by beam (the blocks of beam
@@ -1033,13 +1137,11 @@ __global__ __launch_bounds__(256) void terma_set_kernel(
     const TermaParams* __restrict__ tab, int32_t n_bricks,
     int32_t blocks_per_beam)
 {
-    __shared__ double s_samp[4][kSampleBuf];
     __shared__ int32_t s_lane[4][64];
     const int w = threadIdx.x >> 6;
     const int beam = blockIdx.x / blocks_per_beam;
     const int g = (blockIdx.x - beam * blocks_per_beam) * 4 + w;
-    terma_wave(tab[beam], g, threadIdx.x & 63, s_samp[w], s_lane[w],
-               n_bricks);
+    terma_wave(tab[beam], g, threadIdx.x & 63, s_lane[w], n_bricks);
 }
 
 __global__ __launch_bounds__(64) void terma_prep_kernel(int32_t* status)
@@ -1100,13 +1202,6 @@ static TermaParams make_params(const ch_beam& B, const int32_t* h_shape,
         P.off[a] = P.spacing[a] / ns;
     P.ndotn_src = P.vy[0] * P.src[0] + P.vy[1] * P.src[1] + P.vy[2] * P.src[2];
     P.n3 = (double)(ns * ns * ns);
-    // the hit test's loop adds (double)v / n^3 n^3 times, here for v = 1
-    const double inc = 1.0 / P.n3;
-    double one = 0.0;
-    for (int k = 0; k < ns * ns * ns; ++k)
-        one = one + inc;
-    P.blocked_one = one;
-    P.inv_n3 = 1.0f / (float)(ns * ns * ns);
     P.inv_ns = 1.0f / (float)ns;
     for (int a = 0; a < 3; ++a)
         P.src_vox[a] = (float)((P.src[a] - P.origin[a]) / P.spacing[a]);
@@ -1116,6 +1211,16 @@ static TermaParams make_params(const ch_beam& B, const int32_t* h_shape,
                         P.tr2[2] * P.src[2]);
     P.k100 = -100.0 * P.ndotn_src;
     P.fast_ok = fabs(P.ci_src) < 1e5 && fabs(P.cj_src) < 1e5;
+    P.ci_cell = P.ci_src + 1999.0;
+    P.cj_cell = P.cj_src + 1999.0;
+    for (int a = 0; a < 3; ++a) {
+        P.step_d[a] = -P.vy[a] * P.off[a];
+        P.step_i[a] = -P.tr0[a] * P.off[a];
+        P.step_j[a] = -P.tr2[a] * P.off[a];
+        P.span_d[a] = P.step_d[a] * (ns - 1);
+        P.span_i[a] = P.step_i[a] * (ns - 1);
+        P.span_j[a] = P.step_j[a] * (ns - 1);
+    }
     return P;
 }
 
