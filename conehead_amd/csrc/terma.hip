@@ -4,10 +4,9 @@
 //
 // The reference runs these as six kernels with a host round trip after each
 // (conehead/conehead.py:536-682).  Geometry (sub-sample positions, plane
-// hits, ray directions, DDA alphas) is FP64 with contraction off so that the
-// traversal and the aperture lookups match the FP64 oracle bit for bit; the
-// depth integral uses FP32 with Kahan compensation and the fluence and TERMA
-// arithmetic is FP32.
+// hits, ray directions, DDA alphas) and the depth integral are FP64 with
+// contraction off, so that the traversal and the aperture lookups match the
+// FP64 oracle bit for bit; the fluence and TERMA arithmetic is FP32.
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -432,7 +431,23 @@ __device__ __forceinline__ float cell_value(const TermaParams& P, int i,
     return P.raster[i * 4000 + j];
 }
 
-// Brick of 4 x 4 x 4 voxels.
+// Bricks of 4 x 2 x 8 voxels, one per wavefront in phase 2, lane l's voxel
+// (x0 + lane_x, y0 + lane_y, z0 + lane_z).  A density load of the walk
+// touches one line per (x, y) row of the brick, and 64 lanes in 8 rows of
+// 8 voxels keep the rays side by side: the walk of the 200 x 200 x 160 beam
+// took 232 us against 291 with 4 x 4 x 4 (16 rows), and 241 to 306 with
+// z runs of 16 and 64 (rays that drift apart in z leave a long row's lanes
+// on different rows, and the field's edge cuts more of them off); the
+// 128^3 beam 41 us against 46.
+constexpr int kBX = 4, kBY = 2, kBZ = 8;
+static_assert(kBX * kBY * kBZ == 64, "one voxel per lane");
+__device__ __forceinline__ int lane_x(int l) { return l / (kBY * kBZ); }
+__device__ __forceinline__ int lane_y(int l) { return (l / kBZ) % kBY; }
+__device__ __forceinline__ int lane_z(int l) { return l % kBZ; }
+__host__ __device__ __forceinline__ int ceil_div(int a, int b)
+{
+    return (a + b - 1) / b;
+}
 struct Brick {
     int x0, y0, z0;
 };
@@ -445,8 +460,8 @@ struct Brick {
 // third of one with every voxel open.  Each sample's lines come from the
 // first's by one addition per axis, its cells as fast_cells certifies them;
 // a cell within 1e-6 of an integer is decided by plane_image.  The
-// transmissions are FP32 values of at most 1 on a grid of 2^-24, so their
-// FP64 sum is exact in any order.  33 instructions per sample against about
+// transmissions are FP32 values; those of squares and leaves lie on a grid of
+// 2^-24, so their FP64 sum is exact in any order.  33 instructions per sample against about
 // 100 with each sample's own dot products, quotient and range checks.
 __device__ __forceinline__ double sample_sums(const TermaParams& P,
                                               const Brick& k, const Lines& L,
@@ -493,10 +508,9 @@ __device__ __forceinline__ double sample_sums(const TermaParams& P,
                          fabs(__builtin_amdgcn_fract(cj) - 0.5));
                 if (e >= 0.5 - 1e-6) {
                     const PlaneImage c = plane_image(
-                        P, sample_pos(P, 0, k.x0 + (src >> 4), P.off[0], ix),
-                        sample_pos(P, 1, k.y0 + ((src >> 2) & 3), P.off[1],
-                                   iy),
-                        sample_pos(P, 2, k.z0 + (src & 3), P.off[2], iz),
+                        P, sample_pos(P, 0, k.x0 + lane_x(src), P.off[0], ix),
+                        sample_pos(P, 1, k.y0 + lane_y(src), P.off[1], iy),
+                        sample_pos(P, 2, k.z0 + lane_z(src), P.off[2], iz),
                         P.ndotn_src);
                     i = (int)(floor(c.ci) + 1999.0);
                     j = (int)(floor(c.cj) + 1999.0);
@@ -641,26 +655,21 @@ __device__ __forceinline__ float depth_walk(const float* __restrict__ rho,
 // TERMA in two phases.  The hit test (conehead.py:78-120) runs in three
 // stages that each give the exact blocked fraction of the loop over n^3
 // sub-samples: (1) the brick of 64 voxels at once (brick_value), (2) each
-// voxel's own 8 corners by the same argument, (3) the sub-samples of the
-// voxels still open, spread over all 64 lanes (a few voxels at a time),
-// each lane evaluating one sub-sample into LDS; each voxel then sums its
-// own values in the loop's order, so the result is bitwise that of the
-// loop (when most of the lanes need samples the loop runs on each lane).
+// voxel's own 8 corners by the same argument (voxel_box), (3) the
+// sub-samples of the voxels still open (sample_sums).
 // Phase 1 sorts the bricks by stage 1: those outside the aperture are done
 // there; the rest -- the voxels the beam reaches, a seventh of a 128^3 grid
 // for a 10 x 10 cm field -- go to phase 2 in order of their estimated cost,
 // the longest depth walks first, so they start together and the cheaper
 // ones fill in behind them.
-// Bricks of 4 x 4 x 4 voxels (one per wavefront in phase 2), indexed z
-// fastest: the corner voxel of brick b, and lane l's voxel (x0 + l / 16,
-// y0 + l / 4 % 4, z0 + l % 4).
+// The corner voxel of brick b (bricks indexed z fastest).
 __device__ __forceinline__ Brick brick_of(const TermaParams& P, int b)
 {
-    const int nbz = (P.Z + 3) / 4, nby = (P.Y + 3) / 4;
+    const int nbz = ceil_div(P.Z, kBZ), nby = ceil_div(P.Y, kBY);
     Brick k;
-    k.z0 = (b % nbz) * 4;
-    k.y0 = ((b / nbz) % nby) * 4;
-    k.x0 = (b / nbz / nby) * 4;
+    k.z0 = (b % nbz) * kBZ;
+    k.y0 = ((b / nbz) % nby) * kBY;
+    k.x0 = (b / nbz / nby) * kBX;
     return k;
 }
 
@@ -677,9 +686,9 @@ __device__ __forceinline__ float brick_value(const TermaParams& P,
 {
     const int ns = P.samples;
     const int c = l & 7;
-    const int xa = (c & 1) ? min(k.x0 + 3, P.X - 1) : k.x0;
-    const int ya = (c & 2) ? min(k.y0 + 3, P.Y - 1) : k.y0;
-    const int za = (c & 4) ? min(k.z0 + 3, P.Z - 1) : k.z0;
+    const int xa = (c & 1) ? min(k.x0 + kBX - 1, P.X - 1) : k.x0;
+    const int ya = (c & 2) ? min(k.y0 + kBY - 1, P.Y - 1) : k.y0;
+    const int za = (c & 4) ? min(k.z0 + kBZ - 1, P.Z - 1) : k.z0;
     const int s0 = (c & 1) ? ns - 1 : 0;
     const int s1 = (c & 2) ? ns - 1 : 0;
     const int s2 = (c & 4) ? ns - 1 : 0;
@@ -720,7 +729,8 @@ constexpr int kCounterInts = 3 * kCounters + 64;    // 256-byte multiple
 __device__ __forceinline__ int brick_cost_class(const TermaParams& P,
                                                 const Brick& k, bool edge)
 {
-    const float c[3] = {k.x0 + 1.5f, k.y0 + 1.5f, k.z0 + 1.5f};
+    const float c[3] = {k.x0 + 0.5f * (kBX - 1), k.y0 + 0.5f * (kBY - 1),
+                        k.z0 + 0.5f * (kBZ - 1)};
     const int n[3] = {P.X, P.Y, P.Z};
     float d[3], t = 3.0e38f;
     for (int a = 0; a < 3; ++a) {
@@ -755,17 +765,16 @@ struct SuperGrid {
 __device__ __forceinline__ SuperGrid super_grid(const TermaParams& P)
 {
     SuperGrid g;
-    g.nbx = (P.X + 3) / 4;
-    g.nby = (P.Y + 3) / 4;
-    g.nbz = (P.Z + 3) / 4;
+    g.nbx = ceil_div(P.X, kBX);
+    g.nby = ceil_div(P.Y, kBY);
+    g.nbz = ceil_div(P.Z, kBZ);
     g.sby = (g.nby + 1) / 2;
     g.sbz = (g.nbz + 1) / 2;
     return g;
 }
 __host__ __device__ __forceinline__ int32_t super_bricks(int X, int Y, int Z)
 {
-    return (((X + 3) / 4 + 1) / 2) * (((Y + 3) / 4 + 1) / 2) *
-           (((Z + 3) / 4 + 1) / 2);
+    return ceil_div(X, 2 * kBX) * ceil_div(Y, 2 * kBY) * ceil_div(Z, 2 * kBZ);
 }
 constexpr int kSortSupers = 4;                   // super-bricks per workgroup
 constexpr int kSortBricks = 8 * kSortSupers;     // bricks per workgroup
@@ -807,22 +816,22 @@ __device__ __forceinline__ void sort_block(const TermaParams& P, int blk,
                   bz = 2 * sz + (c & 1);
         const bool in = bx < g.nbx && by < g.nby && bz < g.nbz;
         Brick k;
-        k.x0 = 4 * min(bx, g.nbx - 1);
-        k.y0 = 4 * min(by, g.nby - 1);
-        k.z0 = 4 * min(bz, g.nbz - 1);
+        k.x0 = kBX * min(bx, g.nbx - 1);
+        k.y0 = kBY * min(by, g.nby - 1);
+        k.z0 = kBZ * min(bz, g.nbz - 1);
         const float v = brick_value(P, k, l);
         const bool zero = in && v == 0.0f && P.debug == nullptr;
         // bit 8 c set when child c reads 0: lane l writes voxel l of each
         const uint64_t zmask = __ballot(zero) & 0x0101010101010101ull;
         if (zmask != 0 && !P.accumulate) {
-            const int dx = l >> 4, dy = (l >> 2) & 3, dz = l & 3;
+            const int dx = lane_x(l), dy = lane_y(l), dz = lane_z(l);
 #pragma unroll
             for (int cc = 0; cc < 8; ++cc) {
                 if (!((zmask >> (8 * cc)) & 1))
                     continue;  // wavefront-uniform
-                const int x = 4 * (2 * sx + (cc >> 2)) + dx,
-                          y = 4 * (2 * sy + ((cc >> 1) & 1)) + dy,
-                          z = 4 * (2 * sz + (cc & 1)) + dz;
+                const int x = kBX * (2 * sx + (cc >> 2)) + dx,
+                          y = kBY * (2 * sy + ((cc >> 1) & 1)) + dy,
+                          z = kBZ * (2 * sz + (cc & 1)) + dz;
                 if (x < P.X && y < P.Y && z < P.Z)
                     P.terma[((int64_t)x * P.Y + y) * P.Z + z] = 0.0f;
             }
@@ -886,9 +895,9 @@ __device__ __forceinline__ float terma_brick(const TermaParams& P,
 {
     const int64_t nv = (int64_t)P.X * P.Y * P.Z;
     const int x0 = k.x0, y0 = k.y0, z0 = k.z0;
-    const int x = x0 + (l >> 4);
-    const int y = y0 + ((l >> 2) & 3);
-    const int z = z0 + (l & 3);
+    const int x = x0 + lane_x(l);
+    const int y = y0 + lane_y(l);
+    const int z = z0 + lane_z(l);
     const bool inside = x < P.X && y < P.Y && z < P.Z;
     const int ns = P.samples;
     const double n3 = P.n3;
@@ -1090,9 +1099,9 @@ __device__ __forceinline__ void terma_wave(const TermaParams& P, int g,
             T = terma_brick(P, k, v, l, s_lane, bad);
             if (__ballot(bad) != 0 && l == 0)
                 atomicOr(P.status, 1);
-            x = k.x0 + (l >> 4);
-            y = k.y0 + ((l >> 2) & 3);
-            z = k.z0 + (l & 3);
+            x = k.x0 + lane_x(l);
+            y = k.y0 + lane_y(l);
+            z = k.z0 + lane_z(l);
         }
     }
     if (P.box) {
@@ -1230,8 +1239,8 @@ static TermaParams make_params(const ch_beam& B, const int32_t* h_shape,
 // phase-2 wavefront.
 inline int32_t terma_bricks(const int32_t* shape)
 {
-    return ((shape[0] + 3) / 4) * ((shape[1] + 3) / 4) *
-           ((shape[2] + 3) / 4);
+    return ceil_div(shape[0], kBX) * ceil_div(shape[1], kBY) *
+           ceil_div(shape[2], kBZ);
 }
 inline size_t terma_list_ints(const int32_t* shape)
 {
@@ -1397,7 +1406,26 @@ static ch_status terma_grid_ok(const char* fn, const int32_t* shape,
 // The allocation-free variant's scratch: one array per device, resolved to
 // a device address per device once (hipGetSymbolAddress) and used only
 // through that address.
-constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
+// It takes the grids whose lists and boxes for bricks of 4 x 4 x 4 voxels
+// fit kNoAllocLimit (noalloc_need), so the limit does not move with the
+// brick shape; those of kBX x kBY x kBZ bricks are at most twice that (the
+// largest ratio, on grids of one to eight layers in z).
+constexpr size_t kNoAllocLimit = (size_t)16 << 20;
+constexpr size_t kNoAllocScratchBytes = 2 * kNoAllocLimit;
+static size_t noalloc_need(const int32_t* n)
+{
+    const size_t supers = (size_t)ceil_div(n[0], 8) * ceil_div(n[1], 8) *
+                          ceil_div(n[2], 8);
+    const size_t bricks = (size_t)ceil_div(n[0], 4) * ceil_div(n[1], 4) *
+                          ceil_div(n[2], 4);
+    const size_t blocks = (supers + kSortSupers - 1) / kSortSupers;
+    const size_t list = (blocks + kShards - 1) / kShards * kSortBricks;
+    size_t cap = kSortBricks;
+    while (cap < list)
+        cap *= 2;
+    return terma_counter_bytes(1) + (size_t)kCounters * cap * sizeof(int32_t) +
+           (bricks + 3) / 4 * 4 * kBoxStride * sizeof(int32_t);
+}
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 constexpr int kMaxDevices = 64;
 static void* g_scratch_ptr[kMaxDevices];
@@ -1614,13 +1642,14 @@ ch_status ch_terma_noalloc(int32_t n_beams, const ch_beam* h_beams,
     if (st != CH_OK)
         return st;
     const int32_t n_bricks = terma_bricks(h_shape);
-    const size_t need = terma_counter_bytes(1) + terma_list_bytes(1, h_shape) +
-                        terma_box_bytes(1, n_bricks);
-    CH_REQUIRE(need <= kNoAllocScratchBytes,
+    const size_t need = noalloc_need(h_shape);
+    CH_REQUIRE(need <= kNoAllocLimit &&
+                   terma_counter_bytes(1) + terma_list_bytes(1, h_shape) +
+                           terma_box_bytes(1, n_bricks) <=
+                       kNoAllocScratchBytes,
                "ch_terma_noalloc: a %d x %d x %d grid needs %zu bytes of "
                "scratch, more than its %zu (use ch_terma)",
-               h_shape[0], h_shape[1], h_shape[2], need,
-               kNoAllocScratchBytes);
+               h_shape[0], h_shape[1], h_shape[2], need, kNoAllocLimit);
     for (int32_t b = 0; b < n_beams; ++b)
         CH_REQUIRE(h_beams[b].d_status,
                    "ch_terma_noalloc: beam %d has no d_status (the geometry "

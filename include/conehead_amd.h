@@ -448,9 +448,9 @@ ch_status ch_terma(int32_t n_beams, const ch_beam* h_beams,
  * reference.  Same arguments, kernels and results as ch_terma, except:
  * every beam must carry d_status (its geometry flag, an output the caller
  * zeroes; ch_terma_check does not see these calls), and the launch scratch
- * (cost-class lists and support-box partials) is a fixed 16 MiB array per
- * GPU, held until the process ends, so grids needing more (about 11 M
- * voxels and beyond) are refused with CH_ERR_ARG.  Calls that overlap on
+ * (cost-class lists and support-box partials) is a fixed 32 MiB array per
+ * GPU, held until the process ends, so large grids (about 11 M voxels and
+ * beyond) are refused with CH_ERR_ARG.  Calls that overlap on
  * one GPU (on different streams or threads) share that array and race;
  * calls queued on one stream do not. */
 ch_status ch_terma_noalloc(int32_t n_beams, const ch_beam* h_beams,

@@ -256,3 +256,45 @@ def test_repeated_calls_keep_their_counters(engine):
     g.close()
     s.sync()
     s.close()
+
+
+@pytest.mark.parametrize("shape,samples,aperture,gantry", [
+    ((4, 2, 8), 3, "square", 0.0),        # one whole brick
+    ((5, 3, 9), 1, "square", 0.0),        # one voxel past it on every axis
+    ((3, 1, 7), 2, "square", 200.0),      # less than one
+    ((17, 9, 33), 4, "mlc", 61.0),        # ragged bricks, 64 samples
+    ((24, 21, 40), 3, "mlc", 118.0),
+    ((24, 21, 40), 5, "mlc", 90.0),       # more lanes than a wavefront holds
+    ((20, 22, 24), 2, "narrow", 305.0),   # closed leaf interiors, thin leaves
+    ((33, 18, 30), 3, "two", 17.0),       # two rectangles
+])
+def test_brick_remainders_and_sample_counts(oracle, engine, shape, samples,
+                                            aperture, gantry):
+    """Grids that end inside a brick, sub-sample counts on both sides of
+    one lane per plane of a voxel's samples, and leaf tables whose rows are
+    open, closed, interior and edge: the blocked fraction stays bitwise the
+    oracle's and the raster gives the same TERMA as the analytic aperture
+    (compare)."""
+    rng = np.random.default_rng(sum(shape) + samples)
+    s = 0.45
+    origin = np.array([-(n - 1) / 2 * s for n in shape])
+    dens = (1.0 + 0.3 * rng.standard_normal(shape)).clip(0.1, None)
+    blk = Block()
+    if aperture == "square":
+        blk.set_square(1.7 if min(shape) < 8 else 6.0)
+    elif aperture == "two":
+        blk.set_square(3.1)
+        blk.set_square(9.3)
+    elif aperture == "mlc":
+        bound = np.arange(-100, 101, 10.0)
+        a = rng.uniform(-60, 5, 20)
+        blk.set_mlc(bound, a, a + rng.uniform(0, 60, 20), (-70.5, 66.2),
+                    (-55, 48.3))
+    else:
+        # 0.4 to 1.2 mm leaves, most of them closed
+        bound = np.cumsum(np.r_[-30.0, np.tile([0.4, 0.8, 1.2], 25)])
+        a = rng.uniform(-30, 30, 75)
+        blk.set_mlc(bound, a, a + np.where(rng.random(75) < 0.3, 25.0, 0.0),
+                    (-60, 60), (-28, 28))
+    compare(oracle, engine, shape, [s] * 3, origin, dens.astype(np.float32),
+            gantry, blk, settings=dict(SETTINGS, fluenceResampling=samples))
