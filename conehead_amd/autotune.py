@@ -151,8 +151,8 @@ timings = 0          # candidates timed by tune_fft / tune_pipeline so far
 
 
 def fft_key(plan, n_beams):
-    # "fft2": the choices reach 16 lines wherever 16 frames fit 4096 points
-    return "fft2/%dx%dx%d/%d/%d" % (plan.shape + (plan.n_cones, n_beams))
+    # "fft3": frames of 72 to 400 points take the two-stage passes
+    return "fft3/%dx%dx%d/%d/%d" % (plan.shape + (plan.n_cones, n_beams))
 
 
 def tune_fft(plan, n_beams=1, reps=3, stream=None, use_cache=True):

@@ -36,22 +36,31 @@ PAD_Y = 32   # kYPad of the padded TERMA copy (ch_internal.h)
 PAD_Z = 80   # kZPad
 
 
-def _smooth_at_least(n):
-    m = max(int(n), 1)
+# Frame lengths of the two-stage FFT passes (csrc/fft_pair.h).
+PAIR_FRAMES = (72, 80, 90, 96, 100, 108, 120, 128, 144, 150, 160, 162, 180,
+               192, 200, 216, 240, 256, 270, 288, 300, 320, 324, 360, 384,
+               400)
+
+
+def frame_len(n):
+    """Frame length of an axis of n voxels, as ch_plan_spectrum picks it:
+    the smallest 2, 3, 5-smooth length >= 2 n - 1; between 64 and 400 the
+    smallest of the two-stage passes' lengths."""
+    m = max(2 * int(n) - 1, 1)
     while True:
         k = m
         for q in (2, 3, 5):
             while k % q == 0:
                 k //= q
-        if k == 1:
+        if m in PAIR_FRAMES if 64 < m <= 400 else k == 1:
             return m
         m += 1
 
 
 def spectral_frame(shape):
-    """Frame lengths (smallest 2, 3, 5-smooth F >= 2 n - 1 per axis) and
-    half-spectrum pitch of the FFT form, as ch_plan_spectrum picks them."""
-    frame = tuple(_smooth_at_least(2 * int(n) - 1) for n in shape)
+    """Frame lengths (frame_len per axis) and half-spectrum pitch of the FFT
+    form, as ch_plan_spectrum picks them."""
+    frame = tuple(frame_len(n) for n in shape)
     kz = frame[2] // 2 + 1
     return frame, (kz + 15) // 16 * 16
 

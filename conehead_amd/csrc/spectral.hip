@@ -19,13 +19,16 @@
 //   col     x transforms, times K^, inverse x transforms, rows x < X kept;
 //   col     inverse y transforms, rows y < Y kept;
 //   z_inv   two half spectra per complex inverse FFT into the dose lines.
-// The transforms are mixed-radix (2, 3, 4, 5, 8, 16) Stockham FFTs in LDS,
-// W lines per workgroup; frame lengths are products of 2, 3 and 5.  Where
-// the frame is at least twice the grid, half of every forward transform's
-// input is padding and half of every inverse transform's output is cropped:
-// the first stage then skips those rows (half_in) and the last stage those
-// outputs (half_out), when its radix is even.
-#include "ch_internal.h"
+// Frame lengths are products of 2, 3 and 5.  Those from 72 to 400 take the
+// two-stage passes of fft_pair.h; the others, and K^'s own transforms, the
+// general passes here: mixed-radix (2, 3, 4, 5, 8, 16) Stockham FFTs in LDS,
+// W lines per workgroup.  Where the frame is at least twice the grid, half of
+// every forward transform's input is padding and half of every inverse
+// transform's output is cropped: the first stage then skips those rows
+// (half_in) and the last stage those outputs (half_out), when its radix is
+// even.
+#include "fft_core.h"
+#include "fft_pair.h"
 
 #include <algorithm>
 #include <cmath>
@@ -61,195 +64,6 @@ struct FftLen {
     int32_t nfac;
     int32_t fac[12];
 };
-
-__device__ __forceinline__ float2 cmul(float2 a, float2 b)
-{
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ float2 cadd(float2 a, float2 b)
-{
-    return make_float2(a.x + b.x, a.y + b.y);
-}
-__device__ __forceinline__ float2 csub(float2 a, float2 b)
-{
-    return make_float2(a.x - b.x, a.y - b.y);
-}
-__device__ __forceinline__ float2 cscale(float2 a, float s)
-{
-    return make_float2(a.x * s, a.y * s);
-}
-// -i * a for the forward transform, +i * a for the inverse
-template <bool INV>
-__device__ __forceinline__ float2 rot(float2 a)
-{
-    return INV ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
-}
-
-template <bool INV>
-__device__ __forceinline__ void dft2(float2& a, float2& b)
-{
-    const float2 t = a;
-    a = cadd(t, b);
-    b = csub(t, b);
-}
-
-template <bool INV>
-__device__ __forceinline__ void dft4(float2& a, float2& b, float2& c,
-                                     float2& d)
-{
-    const float2 t0 = cadd(a, c), t1 = csub(a, c);
-    const float2 t2 = cadd(b, d), t3 = rot<INV>(csub(b, d));
-    a = cadd(t0, t2);
-    c = csub(t0, t2);
-    b = cadd(t1, t3);
-    d = csub(t1, t3);
-}
-
-// dft4 of (a, b, 0, 0), c and d not read: a + c and b + d are a and b, so
-// every nonzero output has the bits dft4 gives it (only the sign of an
-// exact zero may differ).
-template <bool INV>
-__device__ __forceinline__ void dft4h(float2& a, float2& b, float2& c,
-                                      float2& d)
-{
-    const float2 t3 = rot<INV>(b);
-    c = csub(a, b);
-    d = csub(a, t3);
-    const float2 a0 = a;
-    a = cadd(a0, b);
-    b = cadd(a0, t3);
-}
-
-// dft<INV, H>: the DFT of v in place.  H: the upper half v[R/2 ..] of an
-// even-length v is zero and not read (the first layer of each
-// decomposition drops its zero terms, as in dft4h).
-template <bool INV, bool H = false>
-__device__ __forceinline__ void dft(float2 (&v)[2])
-{
-    if (H)
-        v[1] = v[0];
-    else
-        dft2<INV>(v[0], v[1]);
-}
-
-template <bool INV, bool H = false>
-__device__ __forceinline__ void dft(float2 (&v)[4])
-{
-    if (H)
-        dft4h<INV>(v[0], v[1], v[2], v[3]);
-    else
-        dft4<INV>(v[0], v[1], v[2], v[3]);
-}
-
-template <bool INV, bool H = false>
-__device__ __forceinline__ void dft(float2 (&v)[8])
-{
-    // even and odd halves, then X[k] = E[k] + w^k O[k], X[k+4] = E - w^k O
-    float2 e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6];
-    float2 o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
-    if (H) {
-        dft4h<INV>(e0, e1, e2, e3);
-        dft4h<INV>(o0, o1, o2, o3);
-    } else {
-        dft4<INV>(e0, e1, e2, e3);
-        dft4<INV>(o0, o1, o2, o3);
-    }
-    const float h = 0.70710678118654752f;
-    // w^1 = (h, -h) forward, (h, h) inverse; w^3 = (-h, -h) / (-h, h)
-    const float2 w1o = INV ? make_float2(h * (o1.x - o1.y), h * (o1.x + o1.y))
-                           : make_float2(h * (o1.x + o1.y), h * (o1.y - o1.x));
-    const float2 w2o = rot<INV>(o2);
-    const float2 w3o = INV
-                           ? make_float2(-h * (o3.x + o3.y), h * (o3.x - o3.y))
-                           : make_float2(h * (o3.y - o3.x), -h * (o3.x + o3.y));
-    v[0] = cadd(e0, o0);
-    v[4] = csub(e0, o0);
-    v[1] = cadd(e1, w1o);
-    v[5] = csub(e1, w1o);
-    v[2] = cadd(e2, w2o);
-    v[6] = csub(e2, w2o);
-    v[3] = cadd(e3, w3o);
-    v[7] = csub(e3, w3o);
-}
-
-template <bool INV, bool H = false>
-__device__ __forceinline__ void dft(float2 (&v)[3])
-{
-    static_assert(!H, "odd length");
-    const float s3 = 0.86602540378443865f;  // sin(pi / 3)
-    const float2 t1 = cadd(v[1], v[2]);
-    const float2 t2 = csub(v[0], cscale(t1, 0.5f));
-    const float2 t3 = rot<INV>(cscale(csub(v[1], v[2]), s3));
-    v[0] = cadd(v[0], t1);
-    v[1] = cadd(t2, t3);
-    v[2] = csub(t2, t3);
-}
-
-template <bool INV, bool H = false>
-__device__ __forceinline__ void dft(float2 (&v)[5])
-{
-    static_assert(!H, "odd length");
-    const float c1 = 0.30901699437494742f;   // cos(2 pi / 5)
-    const float c2 = -0.80901699437494742f;  // cos(4 pi / 5)
-    const float s1 = 0.95105651629515357f;   // sin(2 pi / 5)
-    const float s2 = 0.58778525229247313f;   // sin(4 pi / 5)
-    const float2 a = v[0];
-    const float2 sbe = cadd(v[1], v[4]), dbe = csub(v[1], v[4]);
-    const float2 scd = cadd(v[2], v[3]), dcd = csub(v[2], v[3]);
-    const float2 a1 = cadd(a, cadd(cscale(sbe, c1), cscale(scd, c2)));
-    const float2 a2 = cadd(a, cadd(cscale(sbe, c2), cscale(scd, c1)));
-    const float2 b1 = rot<INV>(cadd(cscale(dbe, s1), cscale(dcd, s2)));
-    const float2 b2 = rot<INV>(csub(cscale(dbe, s2), cscale(dcd, s1)));
-    v[0] = cadd(a, cadd(sbe, scd));
-    v[1] = cadd(a1, b1);
-    v[4] = csub(a1, b1);
-    v[2] = cadd(a2, b2);
-    v[3] = csub(a2, b2);
-}
-
-template <bool INV, bool H = false>
-__device__ __forceinline__ void dft(float2 (&v)[16])
-{
-    // 4 x 4: DFT4 over n1 of x[4 n1 + n2], twiddle W16^(n2 k1), DFT4 over
-    // n2, output k1 + 4 k2
-    const float c8 = 0.92387953251128674f, s8 = 0.38268343236508977f;
-    const float h = 0.70710678118654752f;
-    const float sg = INV ? 1.0f : -1.0f;
-#pragma unroll
-    for (int n2 = 0; n2 < 4; ++n2) {
-        if (H)
-            dft4h<INV>(v[n2], v[4 + n2], v[8 + n2], v[12 + n2]);
-        else
-            dft4<INV>(v[n2], v[4 + n2], v[8 + n2], v[12 + n2]);
-    }
-    // after this v[n2 + 4 k1] holds y[n2][k1]; W16^m = (cos, sg sin)
-    const float2 w1 = make_float2(c8, sg * s8), w2 = make_float2(h, sg * h),
-                 w3 = make_float2(s8, sg * c8), w6 = make_float2(-h, sg * h),
-                 w9 = make_float2(-c8, -sg * s8);
-    v[1 + 4] = cmul(v[1 + 4], w1);
-    v[1 + 8] = cmul(v[1 + 8], w2);
-    v[1 + 12] = cmul(v[1 + 12], w3);
-    v[2 + 4] = cmul(v[2 + 4], w2);
-    v[2 + 8] = rot<INV>(v[2 + 8]);
-    v[2 + 12] = cmul(v[2 + 12], w6);
-    v[3 + 4] = cmul(v[3 + 4], w3);
-    v[3 + 8] = cmul(v[3 + 8], w6);
-    v[3 + 12] = cmul(v[3 + 12], w9);
-    float2 o[16];
-#pragma unroll
-    for (int k1 = 0; k1 < 4; ++k1) {
-        float2 a = v[4 * k1], b = v[4 * k1 + 1], c = v[4 * k1 + 2],
-               d = v[4 * k1 + 3];
-        dft4<INV>(a, b, c, d);
-        o[k1] = a;
-        o[k1 + 4] = b;
-        o[k1 + 8] = c;
-        o[k1 + 12] = d;
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        v[i] = o[i];
-}
 
 // One Stockham stage of radix R over W lines of length F in LDS, element
 // (n, w) at n * W + w.  Sub-transforms of length Ns are done; this stage
@@ -639,52 +453,6 @@ __device__ __forceinline__ void load_twiddles(float2* s_tw, const float2* g,
         s_tw[i] = g[i];
 }
 
-// The beams of one launch: TERMA and dose grids from device tables (a
-// batch) or one pointer each (a single beam); work grid b at a_beam * b.
-// Workgroups take blockIdx.x = group * n_beams + beam, so consecutive
-// workgroups are the same columns of different beams (K^ chunks are read
-// once per launch from HBM and then from L2).
-struct BeamIO {
-    const float* t;
-    float* d;
-    const float* const* t_tab;
-    float* const* d_tab;
-    const int32_t* acc_tab;
-    int32_t accumulate;
-    int32_t n_beams;
-    int64_t a_beam;
-};
-
-__device__ __forceinline__ int beam_of_block(const BeamIO& io)
-{
-    return (int)(blockIdx.x % (unsigned)io.n_beams);
-}
-__device__ __forceinline__ int group_of_block(const BeamIO& io)
-{
-    return (int)(blockIdx.x / (unsigned)io.n_beams);
-}
-
-// Workgroups go to the 8 XCDs round-robin by linear id, and each XCD has
-// its own L2.  The y passes take their work in XCD-major order instead:
-// XCD k runs a contiguous range of logical blocks, so the two halves of a
-// 128-byte line (neighbouring 8-column groups) meet in one L2.  The work
-// per block is uniform, so the ranges stay balanced.
-constexpr unsigned kXcds = 8;
-struct BlockXY {
-    unsigned x, y;
-};
-__device__ __forceinline__ BlockXY xcd_major_block(bool on)
-{
-    const unsigned nx = gridDim.x, total = gridDim.x * gridDim.y;
-    unsigned l = blockIdx.x + nx * blockIdx.y;
-    if (on && total % kXcds == 0)
-        l = (l % kXcds) * (total / kXcds) + l / kXcds;
-    BlockXY b;
-    b.x = l % nx;
-    b.y = l / nx;
-    return b;
-}
-
 // The forward y pass (an even number of column groups per beam) puts the
 // two halves of a 128-byte line (column groups 2 gp and 2 gp + 1 of one
 // beam and slab) on one XCD, as consecutive blocks there, and deals these
@@ -706,47 +474,6 @@ __device__ __forceinline__ BlockXY paired_block(unsigned n_beams)
     b.x = (2 * (rest % pairs) + (j & 1)) * n_beams + beam;
     b.y = rest / pairs;
     return b;
-}
-
-// Line pair w of a z-pass workgroup: lines (x, y) and (x, y + 1) of the
-// grid, y even; valid = false past the last pair.
-struct LinePair {
-    int64_t x;
-    int32_t y;
-    bool valid;
-};
-__device__ __forceinline__ LinePair line_pair(int64_t p, int32_t X,
-                                              int32_t Y)
-{
-    const int Yp = (Y + 1) / 2;
-    LinePair lp;
-    lp.valid = p < (int64_t)X * Yp;
-    lp.x = lp.valid ? p / Yp : 0;
-    lp.y = lp.valid ? 2 * (int)(p - lp.x * Yp) : 0;
-    return lp;
-}
-
-// Zero support of a beam's work grid, so the forward passes skip what is
-// zero: z_fwd records per line pair whether it holds a nonzero value (and
-// writes the pair's spectra only then); the forward y pass reads those
-// flags, skips a slab whose pairs are all zero (recording it in the slab
-// flags) and reads only the nonzero rows of the others; the convolution
-// pass reads only the rows x of nonzero slabs.  The flags are int32 at
-// `off` (complex points after the beam's work grid): X * yp pair flags
-// (pair p = x * yp + y / 2), then X slab flags at xyp = X * yp.  off < 0:
-// no flags (every row is read).
-struct Support {
-    int64_t off;
-    int32_t yp, xyp;
-};
-constexpr int kMaxFlagRows = 512;   // pairs per slab and slabs (X) with flags
-
-__host__ __device__ __forceinline__ Support no_support()
-{
-    Support sp;
-    sp.off = -1;
-    sp.yp = sp.xyp = 0;
-    return sp;
 }
 
 // Whether any thread of line pair w (threads tid % W == w) loaded a
@@ -1276,6 +1003,51 @@ bool fft_factor(int n, FftLen& L)
     return m == 1;
 }
 
+// Frame length of an axis of n voxels: the smallest length >= 2 n - 1 whose
+// prime factors are 2, 3 and 5 (1 for one voxel); between 64 and 400, where
+// the two-stage passes have their lengths, the smallest of those.  They skip
+// the odd lengths, which could not halve their end stages (the convolution
+// pass of three 112 x 104 x 110 beams took 158 us at 225 points against 57
+// at 240), and 250, whose radix 25 leaves too few registers (three 125 x 129
+// x 76 beams: 194 us at 250 against 56 at 256).
+int32_t frame_len(int32_t n)
+{
+    for (int32_t m = std::max(2 * n - 1, 1);; ++m) {
+        PairFns fns;
+        if (m > 64 && m <= 400) {
+            if (fft_pair(m, &fns))
+                return m;
+            continue;
+        }
+        int32_t k = m;
+        for (int32_t q : {2, 3, 5})
+            while (k % q == 0)
+                k /= q;
+        if (k == 1)
+            return m;
+    }
+}
+
+// Lines per workgroup of plan p's five passes.  The two-stage passes hold
+// 16 lines of any of their lengths; the general ones what fits their LDS
+// limits.
+void pass_lines(const ch_plan* p, int32_t lines[5])
+{
+    const int axis[5] = {2, 1, 0, 1, 2};
+    for (int k = 0; k < 5; ++k) {
+        const int a = axis[k], want = p->fft_lines[k];
+        const int F = p->fft_n[a] ? p->fft_n[a]
+                                  : frame_len(p->shape[a]);
+        PairFns fns;
+        if (fft_pair(F, &fns))
+            lines[k] = want == 2 || want == 4 || want == 8 ? want
+                                                           : kPairLines;
+        else
+            lines[k] = lines_per_group(
+                F, k == 2 ? kFftLdsElemsConv : kFftLdsElems, want);
+    }
+}
+
 FftLen plan_len(const ch_plan* p, int a)
 {
     FftLen L;
@@ -1468,19 +1240,6 @@ BeamIO single_beam(const float* t, float* d, int32_t accumulate)
     return io;
 }
 
-// Smallest n' >= n whose prime factors are 2, 3 and 5.
-int32_t smooth_at_least(int32_t n)
-{
-    for (int32_t m = std::max(n, 1);; ++m) {
-        int32_t k = m;
-        for (int32_t q : {2, 3, 5})
-            while (k % q == 0)
-                k /= q;
-        if (k == 1)
-            return m;
-    }
-}
-
 // The support flags of a beam's work grid (after its complex points), or
 // none when a slab or its line pairs exceed the flag rows of the kernels.
 Support plan_support(const ch_plan* p)
@@ -1519,27 +1278,47 @@ ch_status spectral_passes(const ch_plan* p, BeamIO io, float2* A,
     const int64_t slab = (int64_t)Fy * kp;
     const int32_t* W = p->fft_lines;
     const Support sp = plan_support(p);
+    // each pass by the two-stage kernels where its frame has a pair of
+    // radices (such a frame is even, so at least twice the grid), else by
+    // the general ones
+    PairFns fx, fy, fz;
+    const bool px = fft_pair(Lx.n, &fx), py = fft_pair(Ly.n, &fy),
+               pz = fft_pair(Lz.n, &fz);
+    int32_t lines[5];
+    pass_lines(p, lines);
     ch_status st =
-        z_fwd(io, A, X, Y, Z, Fy, kp, Lz, p->d_tw[2], s, W[0], sp);
+        pz ? fz.z_fwd(io, A, X, Y, Z, Fy, kp, p->d_tw[2], s, lines[0], sp)
+           : z_fwd(io, A, X, Y, Z, Fy, kp, Lz, p->d_tw[2], s, W[0], sp);
     if (st == CH_OK)
-        st = col<kColFwd>(io, A, kp, slab, X, kz, Y, Fy, Ly, p->d_tw[1],
-                          nullptr, 0, 0, s, W[1], nullptr, sp);
+        st = py ? fy.y_fwd(io, A, (uint32_t)kp, slab, X, kz, Y, p->d_tw[1], s,
+                           lines[1], sp)
+                : col<kColFwd>(io, A, kp, slab, X, kz, Y, Fy, Ly, p->d_tw[1],
+                               nullptr, 0, 0, s, W[1], nullptr, sp);
     if (st == CH_OK) {
+        auto conv = [&](LaunchTimer* timer) {
+            return px ? fx.conv(io, A, (uint32_t)slab, kp, Fy, kz, X,
+                                p->d_tw[0], p->d_khat, (uint32_t)slab, kp, s,
+                                lines[2], timer, sp)
+                      : col<kColConv>(io, A, slab, kp, Fy, kz, X, X, Lx,
+                                      p->d_tw[0], p->d_khat, slab, kp, s,
+                                      W[2], timer, sp);
+        };
         if (time_conv) {
             LaunchTimer timer(s);
-            st = col<kColConv>(io, A, slab, kp, Fy, kz, X, X, Lx, p->d_tw[0],
-                               p->d_khat, slab, kp, s, W[2], &timer, sp);
+            st = conv(&timer);
             timer.stop();
         } else {
-            st = col<kColConv>(io, A, slab, kp, Fy, kz, X, X, Lx, p->d_tw[0],
-                               p->d_khat, slab, kp, s, W[2], nullptr, sp);
+            st = conv(nullptr);
         }
     }
     if (st == CH_OK)
-        st = col<kColInv>(io, A, kp, slab, X, kz, Fy, Y, Ly, p->d_tw[1],
-                          nullptr, 0, 0, s, W[3]);
+        st = py ? fy.y_inv(io, A, (uint32_t)kp, slab, X, kz, Y, p->d_tw[1], s,
+                           lines[3])
+                : col<kColInv>(io, A, kp, slab, X, kz, Fy, Y, Ly, p->d_tw[1],
+                               nullptr, 0, 0, s, W[3]);
     if (st == CH_OK)
-        st = z_inv(io, A, X, Y, Z, Fy, kp, Lz, p->d_tw[2], s, W[4]);
+        st = pz ? fz.z_inv(io, A, X, Y, Z, Fy, kp, p->d_tw[2], s, lines[4])
+                : z_inv(io, A, X, Y, Z, Fy, kp, Lz, p->d_tw[2], s, W[4]);
     return st;
 }
 
@@ -1626,6 +1405,40 @@ static BeamIO table_io(void* d, int32_t nb)
 }
 
 }  // namespace
+
+bool fft_pair(int F, PairFns* out)
+{
+    switch (F) {
+    case 72: *out = pair_fns_72(); return true;
+    case 80: *out = pair_fns_80(); return true;
+    case 90: *out = pair_fns_90(); return true;
+    case 96: *out = pair_fns_96(); return true;
+    case 100: *out = pair_fns_100(); return true;
+    case 108: *out = pair_fns_108(); return true;
+    case 120: *out = pair_fns_120(); return true;
+    case 128: *out = pair_fns_128(); return true;
+    case 144: *out = pair_fns_144(); return true;
+    case 150: *out = pair_fns_150(); return true;
+    case 160: *out = pair_fns_160(); return true;
+    case 162: *out = pair_fns_162(); return true;
+    case 180: *out = pair_fns_180(); return true;
+    case 192: *out = pair_fns_192(); return true;
+    case 200: *out = pair_fns_200(); return true;
+    case 216: *out = pair_fns_216(); return true;
+    case 240: *out = pair_fns_240(); return true;
+    case 256: *out = pair_fns_256(); return true;
+    case 270: *out = pair_fns_270(); return true;
+    case 288: *out = pair_fns_288(); return true;
+    case 300: *out = pair_fns_300(); return true;
+    case 320: *out = pair_fns_320(); return true;
+    case 324: *out = pair_fns_324(); return true;
+    case 360: *out = pair_fns_360(); return true;
+    case 384: *out = pair_fns_384(); return true;
+    case 400: *out = pair_fns_400(); return true;
+    default: return false;
+    }
+}
+
 }  // namespace ch
 
 using namespace ch;
@@ -1669,7 +1482,7 @@ ch_status ch_plan_spectrum(ch_plan* plan, void* stream)
                               "spectrum before capturing");
     int32_t F[3];
     for (int a = 0; a < 3; ++a) {
-        F[a] = smooth_at_least(2 * plan->shape[a] - 1);
+        F[a] = frame_len(plan->shape[a]);
         CH_REQUIRE(F[a] <= kFftMax,
                    "ch_plan_spectrum: axis %d of %d voxels needs a %d-point "
                    "transform (at most %d)", a, plan->shape[a], F[a], kFftMax);
@@ -1963,16 +1776,7 @@ ch_status ch_plan_set_fft_lines(ch_plan* plan, const int32_t lines[5])
 ch_status ch_plan_get_fft_lines(const ch_plan* plan, int32_t lines[5])
 {
     CH_REQUIRE(plan && lines, "ch_plan_get_fft_lines: null pointer");
-    int32_t F[3];
-    for (int a = 0; a < 3; ++a)
-        F[a] = plan->fft_n[a] ? plan->fft_n[a]
-                              : smooth_at_least(2 * plan->shape[a] - 1);
-    const int* W = plan->fft_lines;
-    lines[0] = lines_per_group(F[2], kFftLdsElems, W[0]);
-    lines[1] = lines_per_group(F[1], kFftLdsElems, W[1]);
-    lines[2] = lines_per_group(F[0], kFftLdsElemsConv, W[2]);
-    lines[3] = lines_per_group(F[1], kFftLdsElems, W[3]);
-    lines[4] = lines_per_group(F[2], kFftLdsElems, W[4]);
+    pass_lines(plan, lines);
     return CH_OK;
 }
 

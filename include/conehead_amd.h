@@ -268,12 +268,13 @@ ch_status ch_plan_get_tile(const ch_plan* plan, int32_t* tx, int32_t* ty,
                            int32_t* tz);
 /* Lines per workgroup of the FFT form's five passes (z forward, y
  * forward, x convolution, y inverse, z inverse); set by the autotuner.
- * Each value is 0 (the default: the most lines, up to 16, whose frames fit
- * 2048 points, 4096 for the convolution pass) or 2, 4, 8 or 16, taken when
- * its frames fit 4096 points; a value whose frames do not fit falls back to
- * the default.  Every choice computes the same butterflies
- * on every line, so the dose does not depend on it.  get returns the
- * values the passes use. */
+ * Each value is 0 (the default) or 2, 4, 8 or 16.  Passes over frames of 72
+ * to 400 points take any of them, 16 by default; the others the most lines,
+ * up to 16, whose frames fit 2048 points by default (4096 for the
+ * convolution pass) and a value whose frames fit 4096 points; one whose
+ * frames do not falls back to the default.  Every choice computes the same
+ * butterflies on every line, so the dose does not depend on it.  get returns
+ * the values the passes use. */
 ch_status ch_plan_set_fft_lines(ch_plan* plan, const int32_t lines[5]);
 ch_status ch_plan_get_fft_lines(const ch_plan* plan, int32_t lines[5]);
 /* Accumulation mode: 0 = Kahan per tap, 1 = plain per cone line with Kahan

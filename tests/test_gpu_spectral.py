@@ -19,6 +19,7 @@ import numpy as np
 import pytest
 
 from conehead_amd import engine as E
+from conehead_amd.batch import PAIR_FRAMES, frame_len, spectral_frame
 from conehead_amd.cones import ConeSet, default_thetas
 from conehead_amd.device import DeviceArray
 from conehead_amd.kernel2 import PolyenergeticKernel, merged_kernel
@@ -309,3 +310,50 @@ def test_spectrum_budget(engine, kern):
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
     tight.close()
+
+
+@pytest.mark.parametrize("frame", PAIR_FRAMES)
+def test_two_stage_passes(engine, kern, frame):
+    """Every frame length of the two-stage passes on every axis, at the
+    largest grid of the frame (half of it) and the smallest, against the
+    gather.  The other axes have one radix or an odd extent (an unpaired z
+    line, a partly filled group of lines or columns), T has zero slabs and
+    zero lines, and every count of lines per workgroup gives the same bits,
+    alone and as one of three beams.  Both forms sum FP32 products: their
+    errors of a few 1e-7 of Dmax stay far inside the 1e-5 of this file."""
+    small = next(n for n in range(1, frame) if frame_len(n) == frame)
+    rng = np.random.default_rng(frame)
+    cs = cone_set(kern, 6, 4)
+    for axis in range(3):
+        for n in (frame // 2, small):
+            shape = [9, 11, 7]
+            shape[axis] = n
+            shape = tuple(shape)
+            assert spectral_frame(shape)[0][axis] == frame
+            plan = E.Plan(shape, (0.3, 0.3, 0.3), cs)
+            plan.spectrum()
+            T = rng.random(shape).astype(np.float32)
+            T[: shape[0] // 3] = 0.0
+            T[:, shape[1] // 2] = 0.0
+            d_t = DeviceArray.from_host(T)
+            d_g = DeviceArray(shape, np.float32)
+            E.convolve(plan, d_t, d_g)
+            ref = run_fft(plan, T)
+            assert rel_err(ref, d_g.download()) < TOL, (axis, n)
+            outs = [DeviceArray(shape, np.float32) for _ in range(3)]
+            for w in (2, 4, 8, 16):
+                plan.set_fft_lines((w,) * 5)
+                E.convolve_fft_batch([(plan, d_t, d, None, False)
+                                      for d in outs])
+                for d in outs:
+                    assert np.array_equal(d.download(), ref), (axis, n, w)
+
+
+def test_frame_lengths_agree(engine, kern):
+    """The frame of ch_plan_spectrum is spectral_frame's, from one voxel
+    past the two-stage lengths."""
+    cs = cone_set(kern, 3, 4)
+    for n in list(range(1, 70, 3)) + [32, 33, 36, 37, 41, 63, 68, 113, 122,
+                                      125, 126, 188, 200, 201, 260]:
+        plan = E.Plan((n, 3, 2), (0.3, 0.3, 0.3), cs)
+        assert plan.spectrum()[0] == spectral_frame((n, 3, 2))[0], n
