@@ -738,22 +738,60 @@ __global__ __launch_bounds__(256) void pad_group_kernel(
     P[i] = v;
 }
 
+// One wavefront per padded row: its x and y by one division, its lanes
+// along z.
+struct PadRow {
+    int64_t src;       // first voxel of the source row, -1 for a border row
+    int64_t dst;       // first element of the padded row
+    int Zp;
+};
+__device__ __forceinline__ bool pad_row(int X, int Y, int Z, PadRow& r)
+{
+    const int Yp = Y + 2 * kYPad;
+    const int row = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    if (row >= X * Yp)
+        return false;
+    const int x = row / Yp, y = row - x * Yp - kYPad;
+    r.Zp = Z + 2 * kZPad;
+    r.src = y >= 0 && y < Y ? ((int64_t)x * Y + y) * Z : -1;
+    r.dst = (int64_t)row * r.Zp;
+    return true;
+}
+static unsigned pad_blocks(const ch_plan* p)
+{
+    const int64_t rows = (int64_t)p->shape[0] * (p->shape[1] + 2 * kYPad);
+    return (unsigned)((rows + 3) / 4);
+}
+
 // T [X][Y][Z] -> padded [X][Y + 2 kYPad][Z + 2 kZPad] with zero borders.
 __global__ __launch_bounds__(256) void pad_kernel(const float* __restrict__ T,
                                                   float* __restrict__ P,
                                                   int X, int Y, int Z)
 {
-    const int Zp = Z + 2 * kZPad, Yp = Y + 2 * kYPad;
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= (int64_t)X * Yp * Zp)
+    PadRow r;
+    if (!pad_row(X, Y, Z, r))
         return;
-    const int zz = (int)(i % Zp) - kZPad;
-    const int64_t r = i / Zp;
-    const int yy = (int)(r % Yp) - kYPad;
-    const int64_t x = r / Yp;
-    P[i] = (zz >= 0 && zz < Z && yy >= 0 && yy < Y)
-               ? T[(x * Y + yy) * Z + zz]
-               : 0.0f;
+    for (int i = threadIdx.x & 63; i < r.Zp; i += 64) {
+        const int z = i - kZPad;
+        P[r.dst + i] =
+            r.src >= 0 && z >= 0 && z < Z ? T[r.src + z] : 0.0f;
+    }
+}
+
+// The same for densities and T together (pad_rad).
+__global__ __launch_bounds__(256) void pad_rad_kernel(
+    const float* __restrict__ T, const float* __restrict__ rho,
+    float* __restrict__ P, float* __restrict__ Q, int X, int Y, int Z)
+{
+    PadRow r;
+    if (!pad_row(X, Y, Z, r))
+        return;
+    for (int i = threadIdx.x & 63; i < r.Zp; i += 64) {
+        const int z = i - kZPad;
+        const bool in = r.src >= 0 && z >= 0 && z < Z;
+        P[r.dst + i] = in ? rho[r.src + z] : 0.0f;
+        Q[r.dst + i] = in ? T[r.src + z] : 0.0f;
+    }
 }
 
 // ------------------------------------------------------ slab boxes ----
@@ -1068,31 +1106,32 @@ void release_gather_workspace(hipStream_t s)
 static ch_status pad_into(const float* T, float* P, const ch_plan* p,
                           hipStream_t s)
 {
-    const int64_t n = (int64_t)padded_elems(p);
-    hipLaunchKernelGGL(pad_kernel, dim3((unsigned)((n + 255) / 256)),
-                       dim3(256), 0, s, T, P, p->shape[0], p->shape[1],
-                       p->shape[2]);
+    hipLaunchKernelGGL(pad_kernel, dim3(pad_blocks(p)), dim3(256), 0, s, T, P,
+                       p->shape[0], p->shape[1], p->shape[2]);
     CH_HIP(hipGetLastError());
     return CH_OK;
 }
 
-ch_status pad_pair(const ch_plan* p, const float* a, const float* b,
-                   hipStream_t s, const float** pa, const float** pb)
+ch_status pad_rad(const ch_plan* p, const float* terma, const float* density,
+                  int32_t n_parts, hipStream_t s, const float** grids,
+                  double** parts)
 {
     std::lock_guard<std::mutex> lock(g_ws_mu);
     Workspace* w = nullptr;
     const size_t n = padded_elems(p);
-    ch_status st = workspace(s, 2 * n, 0, &w);
+    // the sums first, 8-byte aligned
+    const size_t np =
+        (size_t)n_parts * p->shape[0] * p->shape[1] * p->shape[2];
+    ch_status st = workspace(s, 2 * np + 2 * n, 0, &w);
     if (st != CH_OK)
         return st;
-    st = pad_into(a, w->pad, p, s);
-    if (st == CH_OK)
-        st = pad_into(b, w->pad + n, p, s);
-    if (st != CH_OK)
-        return st;
-    const size_t interior = (size_t)kYPad * (p->shape[2] + 2 * kZPad) + kZPad;
-    *pa = w->pad + interior;
-    *pb = w->pad + n + interior;
+    float* r = w->pad + 2 * np;
+    hipLaunchKernelGGL(pad_rad_kernel, dim3(pad_blocks(p)), dim3(256), 0, s,
+                       terma, density, r, r + n, p->shape[0], p->shape[1],
+                       p->shape[2]);
+    CH_HIP(hipGetLastError());
+    *grids = r;
+    *parts = reinterpret_cast<double*>(w->pad);
     return CH_OK;
 }
 

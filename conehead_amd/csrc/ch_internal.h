@@ -233,11 +233,12 @@ void release_gather_workspace(hipStream_t s);
 ch_status stage_table(hipStream_t s, const void* h_src, size_t bytes,
                       void** d_out);
 void release_stage_tables(hipStream_t s);
-// Pads two grids of plan p's shape into the stream's gather workspace
-// (the layout the gathers read) and returns the interior voxel (0, 0, 0)
-// of each copy.
-ch_status pad_pair(const ch_plan* p, const float* a, const float* b,
-                   hipStream_t s, const float** pa, const float** pb);
+// Pads densities and T of plan p's shape into the stream's gather workspace
+// (the layout the gathers read), T right after the densities.  Returns their
+// start and room for n_parts dose grids of FP64 sums.
+ch_status pad_rad(const ch_plan* p, const float* terma, const float* density,
+                  int32_t n_parts, hipStream_t s, const float** grids,
+                  double** parts);
 
 // Support box of T != 0 from per-block partial boxes: kernels write
 // kBoxStride ints per block (min x, y, z, max x, y, z) to `partials`, then

@@ -13,14 +13,38 @@
 // t_m - t_{m-1} come from the plan (CH_SEM_RADIOLOGICAL).
 //
 // The gather keeps the direct gather's layout: a wavefront owns a 1 x 4 x 16
-// output tile and reads T and the densities from padded copies with
-// range-checked buffer loads.  Every lane walks its cone from its own voxel
-// (R needs the whole path), loading densities only up to the first tap of
-// the tile's union range and both grids from there on.  A workgroup of 8
-// wavefronts stages each kernel row (5996 FP64 values) in LDS once and runs
-// the cones of that row.  R, the index and the increments are FP64 and
-// round like the FP64 oracle (this file is built without contraction); the
-// sums are FP32 with compensation.
+// output tile and reads padded copies of the grids.  Every lane walks its
+// cone from its own voxel (R needs the whole path), loading densities only
+// up to the first tap of the tile's union range and (density, T) pairs from
+// there on.  A workgroup of 8 wavefronts stages each kernel row in LDS once
+// and runs the cones of that row.  R, the index and the increments are FP64;
+// the sums are FP32 with compensation.
+//
+// What bounds it is the latency of the loads and of the path sum they feed,
+// with vector issue at half of its rate, so
+//   - a workgroup's wavefronts are 4 x 2 tiles in x and y: they walk the same
+//     cone at about the same time, and what one of them reads its neighbours
+//     read a few taps later (96^3 voxels, 144 cones: 8 tiles along z 2393 us,
+//     8 along x 2069, 2 x 2 x 2 2098, 4 x 2 1976; a contiguous eighth of the
+//     workgroups per XCD 2371, the XCDs' shares are too uneven);
+//   - tap addresses are a scalar base per tap plus the lane's own offset, no
+//     vector arithmetic and no range check: every tap of a range lies inside
+//     the padded grids for every lane (the tile's end points are within the
+//     range's box or on the way to it, and the padding covers the tile), and
+//     the taps past the range end take its last one with path length 0 and
+//     T = 0, which adds nothing;
+//   - T follows the densities, so one base serves both loads; one 8-byte
+//     load of (density, T) costs more than the two (a wavefront's 4-byte
+//     load takes 5 cycles of the vector cache, its 8-byte load 16);
+//   - a row starts kRadLead entries into its LDS array, so the truncated
+//     100 R is its slot;
+//   - a chunk whose T is 0 for the whole wavefront (the corners of an
+//     oblique beam's box) needs one lookup instead of eight;
+//   - a staged row's loads are all in flight before the first store.
+// The times above and at rad_parts are with the path sum as fused
+// multiply-adds, 2.5 % faster than the product and sum kept here, whose
+// indices are the FP64 oracle's.  96^3 voxels, 144 cones: 2540 -> 2010 us.
+#include <algorithm>
 #include <climits>
 
 #include "ch_internal.h"
@@ -31,23 +55,26 @@ typedef __attribute__((address_space(4))) const int32_t c_i32;
 typedef __attribute__((address_space(4))) const double c_f64;
 
 struct RadJob {
-    const float* terma;    // padded copies, interior voxel (0, 0, 0)
-    const float* density;
+    const float* grids;    // padded densities and, after them, T
     float* dose;
     const int32_t* box;
-    const int32_t* lin;    // per tap: byte offset into the padded grids
+    const int32_t* lin;    // per tap: byte offset into the padded densities
     const double* seg;     // per tap: path length inside the voxel
     const int32_t* ftT;    // first-step tables, cone-minor
     const ConeMeta* meta;
     const int32_t* perm;   // cones ordered by kernel row
     const int32_t* row_begin;
     const double* cum;
-    int32_t row_len, n_rows;
+    double* parts;         // n_parts > 1: the sums of each part of the rows
+    int32_t row_len, n_rows, n_parts;
     int32_t X, Y, Z, n_cones, accumulate, nty, ntz;
 };
 
-constexpr int kRadTY = 4, kRadTZ = 16, kRadWaves = 8;
+constexpr int kRadTY = 4, kRadTZ = 16;   // a wavefront's y and z voxels
+constexpr int kRadWX = 4, kRadWY = 2;    // a workgroup's tiles in x and y
+constexpr int kRadWaves = kRadWX * kRadWY;
 constexpr int kRadRow = kMaxIndex + 1;
+constexpr int kRadLead = 5;   // unused entries before a row in LDS
 
 // trunc(x) as int32, saturating (v_cvt_i32_f64 clamps to the int32 range
 // and reads NaN as 0; a C++ cast of an out-of-range value is undefined).
@@ -69,16 +96,6 @@ __device__ __forceinline__ int rad_index_of(double x)
     return i > kMaxIndex ? kMaxIndex : i;
 }
 
-__device__ __forceinline__ int rad_index(double r)
-{
-    const double f = floor(r * 100.0 - 5.0);
-    if (!(f < 2147483647.0 && f > -2147483648.0))
-        return kMaxIndex;
-    int i = (int)f;
-    i = i < 0 ? -i : i;
-    return i > kMaxIndex ? kMaxIndex : i;
-}
-
 __device__ __forceinline__ void rad_kahan(float& s, float& c, float x)
 {
     const float y = x - c;
@@ -87,86 +104,119 @@ __device__ __forceinline__ void rad_kahan(float& s, float& c, float x)
     s = t;
 }
 
-// Densities (and TERMA) of kUnroll taps from tap t of the tap tables ml,
-// relative to the lane's voxel at byte offset base4 of the padded grids.
-__device__ __forceinline__ void load_taps(__amdgpu_buffer_rsrc_t rr,
-                                          uint32_t base4, const c_i32* ml,
-                                          int t, float (&rho)[kUnroll])
+// The row's value at |floor(100 R - 5)| (clamped); s_cum: the row after
+// kRadLead unused entries.
+__device__ __forceinline__ double rad_at(const double* s_cum, double R)
 {
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
-        rho[u] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-            rr, (int)(base4 - (uint32_t)ml[t + u]), 0, 0));
+    return s_cum[rad_index_of(R * 100.0) + kRadLead];
 }
 
-__device__ __forceinline__ void load_taps2(__amdgpu_buffer_rsrc_t rr,
-                                           __amdgpu_buffer_rsrc_t rt,
-                                           uint32_t base4, const c_i32* ml,
-                                           int t, float (&rho)[kUnroll],
-                                           float (&tv)[kUnroll])
+// The lane's element of a grid at a tap: base (uniform) minus the tap's byte
+// offset in scalar registers, kept apart from the lane's offset by the empty
+// asm, so a load needs no vector address arithmetic.
+__device__ __forceinline__ float tap_load(const char* base, int64_t tap,
+                                          uint32_t voff)
+{
+    uint64_t p = (uint64_t)base - (uint64_t)tap;
+    asm("" : "+s"(p));
+    typedef __attribute__((address_space(1))) const float g_float;
+    typedef __attribute__((address_space(1))) const char g_char;
+    asm("" : "+v"(voff));
+    return *(g_float*)((g_char*)p + voff);
+}
+
+// Densities and T of kUnroll taps from tap t; LAST: the ones at or past the
+// range end uhi take tap uhi - 1 (with path length 0 and T = 0 in rad_step).
+template <bool LAST>
+__device__ __forceinline__ void rad_load(const char* rho, uint32_t voff,
+                                         uint32_t toff, const c_i32* ml,
+                                         int t, int uhi, float (&v)[kUnroll],
+                                         float (&y)[kUnroll])
 {
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-        const int o = (int)(base4 - (uint32_t)ml[t + u]);
-        rho[u] = __int_as_float(
-            __builtin_amdgcn_raw_buffer_load_b32(rr, o, 0, 0));
-        tv[u] = __int_as_float(
-            __builtin_amdgcn_raw_buffer_load_b32(rt, o, 0, 0));
+        const int q = LAST ? min(t + u, uhi - 1) : t + u;
+        v[u] = tap_load(rho, ml[q], voff);
+        y[u] = tap_load(rho, ml[q], toff);
+    }
+}
+template <bool LAST>
+__device__ __forceinline__ void rad_step(const c_f64* ms, int t, int uhi,
+                                         const float (&v)[kUnroll],
+                                         double& R,
+                                         int (&idx)[kUnroll],
+                                         float (&y)[kUnroll], bool& lit)
+{
+    // For x = 100 R >= 5 the subtraction of 5 is exact (the difference is a
+    // multiple of ulp(x) below x), so the slot |floor(x - 5)| + 5, clamped,
+    // is min(trunc(x), kMaxIndex + 5); a chunk with a tap below 5 (or NaN,
+    // which truncates to 0) takes rad_index_of for all its taps.
+    const double R0 = R;
+    int least = kMaxIndex;
+    int any = 0;
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+        if (LAST)
+            y[u] = t + u < uhi ? y[u] : 0.0f;
+        any |= __float_as_int(y[u]);
+        const int q = LAST ? min(t + u, uhi - 1) : t + u;
+        const double seg = ms[q] * (LAST && t + u >= uhi ? 0.0 : 1.0);
+        R = R + (double)v[u] * seg;
+        idx[u] = min(trunc_sat(R * 100.0), kMaxIndex + kRadLead);
+        least = min(least, idx[u]);
+    }
+    lit = __builtin_amdgcn_ballot_w64(any != 0) != 0;
+    if (__builtin_amdgcn_ballot_w64(least < kRadLead) != 0) {
+        // a real branch: R passes through an empty asm here, so the compiler
+        // cannot hoist this work onto every chunk
+        double r = R0;
+        asm volatile("" : "+v"(r));
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const int q = LAST ? min(t + u, uhi - 1) : t + u;
+            const double seg = ms[q] * (LAST && t + u >= uhi ? 0.0 : 1.0);
+            r = r + (double)v[u] * seg;
+            idx[u] = rad_index_of(r * 100.0) + kRadLead;
+        }
     }
 }
 
-__global__ __launch_bounds__(64 * kRadWaves) void gather_rad(RadJob j,
-                                                            int n_tiles)
-{
-    __shared__ double s_cum[kRadRow];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int tile = blockIdx.x * kRadWaves + wave;
-    const bool live = tile < n_tiles;
-    int x = 0, y0 = 0, z0 = 0;
-    if (live) {
-        const int tz = tile % j.ntz;
-        const int r = tile / j.ntz;
-        y0 = (r % j.nty) * kRadTY;
-        x = r / j.nty;
-        z0 = tz * kRadTZ;
-    }
-    const int yl = min(y0 + kRadTY - 1, j.Y - 1);
-    const int zl = min(z0 + kRadTZ - 1, j.Z - 1);
-    const int y = y0 + lane / kRadTZ;
-    const int z = z0 + lane % kRadTZ;
-    const int Zp = j.Z + 2 * kZPad;
-    const int Yp = j.Y + 2 * kYPad;
+constexpr int kRadAhead = 2;   // chunks of densities in flight
+constexpr int kRadStage = (kRadRow + 64 * kRadWaves - 1) / (64 * kRadWaves);
 
-    int lo0 = 0, lo1 = 0, lo2 = 0;
-    int hi0 = j.X - 1, hi1 = j.Y - 1, hi2 = j.Z - 1;
-    if (j.box) {
-        const c_i32* b = (const c_i32*)j.box;
-        lo0 = max(lo0, b[0]);
-        lo1 = max(lo1, b[1]);
-        lo2 = max(lo2, b[2]);
-        hi0 = min(hi0, b[3]);
-        hi1 = min(hi1, b[4]);
-        hi2 = min(hi2, b[5]);
-    }
-    const bool work = live && lo0 <= hi0 && lo1 <= hi1 && lo2 <= hi2;
-    const uint32_t base4 =
-        (uint32_t)(((x * Yp + y + kYPad) * Zp + z + kZPad) * 4);
-    const size_t interior = (size_t)kYPad * Zp + kZPad;
-    const int bytes = j.X * Yp * Zp * 4;
-    const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(j.terma - interior), (short)0, bytes, kBufferFlags);
-    const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(j.density - interior), (short)0, bytes, kBufferFlags);
+// The lane's sum over every kernel row (all wavefronts of the workgroup call
+// it; work: the tile has something to do).
+__device__ __forceinline__ void rad_rows(const RadJob& j, double* s_cum,
+                                          bool work, int x, int y0, int yl,
+                                          int z0, int zl, const int (&lo)[3],
+                                          const int (&hi)[3], uint32_t voff,
+                                          uint32_t toff, float& sum,
+                                          float& comp)
+{
+    const int lane = threadIdx.x & 63;
+    const char* rho = (const char*)j.grids;
     const c_i32* lin = (const c_i32*)j.lin;
     const c_f64* seg = (const c_f64*)j.seg;
-
-    float sum = 0.0f, comp = 0.0f;
-    for (int row = 0; row < j.n_rows; ++row) {
+    sum = comp = 0.0f;
+    const int part = blockIdx.y;
+    const int row_end = j.n_rows * (part + 1) / j.n_parts;
+    for (int row = j.n_rows * part / j.n_parts; row < row_end; ++row) {
         __syncthreads();
         const double* src = j.cum + (size_t)row * j.row_len;
-        for (int i = threadIdx.x; i < kRadRow; i += 64 * kRadWaves)
-            s_cum[i] = src[i];
+        // every load of the row first, then the stores
+        double v[kRadStage];
+#pragma unroll
+        for (int q = 0; q < kRadStage; ++q) {
+            const int i = threadIdx.x + q * 64 * kRadWaves;
+            if (i < kRadRow)
+                v[q] = src[i];
+        }
+#pragma unroll
+        for (int q = 0; q < kRadStage; ++q) {
+            const int i = threadIdx.x + q * 64 * kRadWaves;
+            if (i < kRadRow)
+                s_cum[i + kRadLead] = v[q];
+        }
         __syncthreads();
         if (!work)
             continue;
@@ -182,14 +232,15 @@ __global__ __launch_bounds__(64 * kRadWaves) void gather_rad(RadJob j,
                 const int32_t* f1 = j.ftT + ftab_t_base(1, j.X, j.Y, n);
                 const int32_t* f2 = j.ftT + ftab_t_base(2, j.X, j.Y, n);
                 int ax, bx, ay1, by1, ay2, by2, az1, bz1, az2, bz2;
-                vrange_t(x, lo0, hi0, m->step[0], f0, j.X + 2, n, c, ax, bx);
-                vrange_t(y0, lo1, hi1, m->step[1], f1, j.Y + 2, n, c, ay1,
+                vrange_t(x, lo[0], hi[0], m->step[0], f0, j.X + 2, n, c, ax,
+                         bx);
+                vrange_t(y0, lo[1], hi[1], m->step[1], f1, j.Y + 2, n, c, ay1,
                          by1);
-                vrange_t(yl, lo1, hi1, m->step[1], f1, j.Y + 2, n, c, ay2,
+                vrange_t(yl, lo[1], hi[1], m->step[1], f1, j.Y + 2, n, c, ay2,
                          by2);
-                vrange_t(z0, lo2, hi2, m->step[2], f2, j.Z + 2, n, c, az1,
+                vrange_t(z0, lo[2], hi[2], m->step[2], f2, j.Z + 2, n, c, az1,
                          bz1);
-                vrange_t(zl, lo2, hi2, m->step[2], f2, j.Z + 2, n, c, az2,
+                vrange_t(zl, lo[2], hi[2], m->step[2], f2, j.Z + 2, n, c, az2,
                          bz2);
                 r_lo = max(max(ax, min(ay1, ay2)), min(az1, az2));
                 r_hi = min(min(bx, max(by1, by2)), max(bz1, bz2));
@@ -208,73 +259,134 @@ __global__ __launch_bounds__(64 * kRadWaves) void gather_rad(RadJob j,
                 // densities only (every source there is outside the box)
                 double R = 0.0;
                 int t = 0;
-                for (; t + kUnroll <= ulo; t += kUnroll) {
-                    float rho[kUnroll];
-                    load_taps(rr, base4, ml, t, rho);
+                for (; t + kRadAhead * kUnroll <= ulo;
+                     t += kRadAhead * kUnroll) {
+                    float v[kRadAhead * kUnroll];
 #pragma unroll
-                    for (int u = 0; u < kUnroll; ++u)
-                        R = R + (double)rho[u] * ms[t + u];
+                    for (int u = 0; u < kRadAhead * kUnroll; ++u)
+                        v[u] = tap_load(rho, ml[t + u], voff);
+#pragma unroll
+                    for (int u = 0; u < kRadAhead * kUnroll; ++u)
+                        R = R + (double)v[u] * ms[t + u];
                 }
-                for (; t < ulo; ++t) {
-                    const float rho = __int_as_float(
-                        __builtin_amdgcn_raw_buffer_load_b32(
-                            rr, (int)(base4 - (uint32_t)ml[t]), 0, 0));
-                    R = R + (double)rho * ms[t];
-                }
-                double cprev = ulo > 0 ? s_cum[rad_index(R)] : 0.0;
-                // whole chunks: a tap past the union end has T = 0 for
-                // every lane, and the zero path lengths of the tap padding
-                // leave R unchanged
-                float acc = 0.0f, ac = 0.0f;
-                for (t = ulo; t < uhi; t += kUnroll) {
-                    float rho[kUnroll], tv[kUnroll];
-                    load_taps2(rr, rt, base4, ml, t, rho, tv);
-                    // The index |floor(100 R - 5)| clamped to kMaxIndex.
-                    // For x = 100 R >= 5 the subtraction of 5 is exact
-                    // (the difference is a multiple of ulp(x) below x), so
-                    // the index is min(trunc(x), 6000) - 5; a chunk with a
-                    // tap below 5 (or NaN, which truncates to 0) takes
-                    // rad_index_of for all its taps.
-                    double x[kUnroll];
-                    int idx[kUnroll];
-                    bool slow = false;
+                for (; t < ulo; t += kUnroll) {
+                    float v[kUnroll];
+                    double sg[kUnroll];
 #pragma unroll
                     for (int u = 0; u < kUnroll; ++u) {
-                        R = R + (double)rho[u] * ms[t + u];
-                        x[u] = R * 100.0;
-                        const int ti = trunc_sat(x[u]);
-                        slow = slow || ti < 5;
-                        idx[u] = min(ti, kMaxIndex + 5) - 5;
+                        const int q = min(t + u, ulo - 1);
+                        v[u] = tap_load(rho, ml[q], voff);
+                        sg[u] = ms[q] * (t + u >= ulo ? 0.0 : 1.0);
                     }
-                    if (__builtin_amdgcn_ballot_w64(slow) != 0) {
-                        // a real branch: x passes through an empty asm
-                        // here, so the compiler cannot hoist this work
-                        // onto every chunk
 #pragma unroll
-                        for (int u = 0; u < kUnroll; ++u) {
-                            double xu = x[u];
-                            asm volatile("" : "+v"(xu));
-                            idx[u] = rad_index_of(xu);
-                        }
+                    for (int u = 0; u < kUnroll; ++u)
+                        R = R + (double)v[u] * sg[u];
+                }
+                double cprev = ulo > 0 ? rad_at(s_cum, R) : 0.0;
+                float acc = 0.0f, ac = 0.0f;
+                for (t = ulo; t < uhi; t += kUnroll) {
+                    float v[kUnroll];
+                    int idx[kUnroll];
+                    float y[kUnroll];
+                    bool lit;
+                    if (t + kUnroll <= uhi) {
+                        rad_load<false>(rho, voff, toff, ml, t, uhi, v, y);
+                        rad_step<false>(ms, t, uhi, v, R, idx, y, lit);
+                    } else {
+                        rad_load<true>(rho, voff, toff, ml, t, uhi, v, y);
+                        rad_step<true>(ms, t, uhi, v, R, idx, y, lit);
                     }
-                    float part = 0.0f;
+                    if (!lit) {
+                        cprev = s_cum[idx[kUnroll - 1]];
+                        continue;
+                    }
+                    float some = 0.0f;
 #pragma unroll
                     for (int u = 0; u < kUnroll; ++u) {
                         const double cv = s_cum[idx[u]];
                         const float k = (float)(cv - cprev);
                         cprev = cv;
-                        part = fmaf(k, tv[u], part);
+                        some = fmaf(k, y[u], some);
                     }
-                    rad_kahan(acc, ac, part);
+                    rad_kahan(acc, ac, some);
                 }
                 rad_kahan(sum, comp, acc);
             }
         }
     }
-    if (live && y <= yl && z <= zl) {
+}
+
+__global__ __launch_bounds__(64 * kRadWaves, 6) void gather_rad(RadJob j)
+{
+    __shared__ double s_cum[kRadRow + kRadLead];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int gy = (j.nty + kRadWY - 1) / kRadWY;
+    const int tz = blockIdx.x % j.ntz, by = blockIdx.x / j.ntz;
+    const int xw = (by / gy) * kRadWX + wave % kRadWX;
+    const int ty = (by % gy) * kRadWY + wave / kRadWX;
+    const bool live = xw < j.X && ty < j.nty;
+    const int x = live ? xw : 0;
+    const int y0 = live ? ty * kRadTY : 0, z0 = tz * kRadTZ;
+    const int yl = min(y0 + kRadTY - 1, j.Y - 1);
+    const int zl = min(z0 + kRadTZ - 1, j.Z - 1);
+    const int y = y0 + lane / kRadTZ;
+    const int z = z0 + lane % kRadTZ;
+    const int Zp = j.Z + 2 * kZPad;
+    const int Yp = j.Y + 2 * kYPad;
+
+    int lo[3] = {0, 0, 0}, hi[3] = {j.X - 1, j.Y - 1, j.Z - 1};
+    if (j.box) {
+        const c_i32* b = (const c_i32*)j.box;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = max(lo[a], b[a]);
+            hi[a] = min(hi[a], b[3 + a]);
+        }
+    }
+    const bool work =
+        live && lo[0] <= hi[0] && lo[1] <= hi[1] && lo[2] <= hi[2];
+    const uint32_t voff =
+        (uint32_t)((x * Yp + y + kYPad) * Zp + z + kZPad) * 4u;
+    const uint32_t toff = voff + (uint32_t)(j.X * Yp * Zp) * 4u;
+    float sum, comp;
+    rad_rows(j, s_cum, work, x, y0, yl, z0, zl, lo, hi, voff, toff, sum,
+             comp);
+    if (live && y <= yl && z <= zl && j.n_parts > 1) {
+        const int64_t n = (int64_t)j.X * j.Y * j.Z;
+        j.parts[blockIdx.y * n + ((int64_t)x * j.Y + y) * j.Z + z] =
+            (double)sum - (double)comp;
+    } else if (live && y <= yl && z <= zl) {
         float* d = j.dose + ((size_t)x * j.Y + y) * j.Z + z;
         *d = (j.accumulate ? *d : 0.0f) + sum;
     }
+}
+
+// dose (+)= the sum of the parts, in FP64.
+__global__ __launch_bounds__(256) void rad_sum(const double* parts,
+                                               int n_parts, int64_t n,
+                                               float* dose, int accumulate)
+{
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i >= n)
+        return;
+    double v = 0.0;
+    for (int p = 0; p < n_parts; ++p)
+        v += parts[p * n + i];
+    dose[i] = (accumulate ? dose[i] : 0.0f) + (float)v;
+}
+
+// Parts of the kernel rows, each a grid of workgroups of its own: a launch
+// of a few workgroups per slot ends in a round of partly idle compute units
+// (and a small grid never fills them), so the rows are split until there are
+// sixteen per slot (96^3 voxels, 144 cones: 2128 us at two, 1976 at eight,
+// 1948 at sixteen, 1950 at 32).  A slot is a third of a compute unit: the
+// row in LDS.
+static int rad_parts(unsigned blocks, int n_rows)
+{
+    const unsigned want = 16u * 3u * (unsigned)num_cus();
+    const unsigned parts = (want + blocks - 1) / blocks;
+    return (int)std::max(1u, std::min(parts, (unsigned)n_rows));
 }
 
 }  // namespace ch
@@ -298,15 +410,22 @@ ch_status ch_convolve_rad(const ch_plan* plan, const float* d_terma,
                    plan->row_len >= kRadRow,
                "ch_convolve_rad: plan has no kernel rows");
     hipStream_t s = (hipStream_t)stream;
-    const float* pt = nullptr;
-    const float* pr = nullptr;
-    ch_status st = pad_pair(plan, d_terma, d_density, s, &pt, &pr);
+    RadJob j;
+    j.nty = (plan->shape[1] + kRadTY - 1) / kRadTY;
+    j.ntz = (plan->shape[2] + kRadTZ - 1) / kRadTZ;
+    const int64_t groups =
+        (int64_t)((plan->shape[0] + kRadWX - 1) / kRadWX) *
+        ((j.nty + kRadWY - 1) / kRadWY) * j.ntz;
+    CH_REQUIRE(groups * kRadWaves < INT_MAX / 2,
+               "ch_convolve_rad: too many tiles");
+    const unsigned blocks = (unsigned)groups;
+    j.n_parts = rad_parts(blocks, plan->n_rows);
+    ch_status st = pad_rad(plan, d_terma, d_density,
+                           j.n_parts > 1 ? j.n_parts : 0, s, &j.grids,
+                           &j.parts);
     if (st != CH_OK)
         return st;
     capture_pin(s, plan);
-    RadJob j;
-    j.terma = pt;
-    j.density = pr;
     j.dose = d_dose;
     j.box = d_box;
     j.lin = plan->d_lin;
@@ -323,16 +442,16 @@ ch_status ch_convolve_rad(const ch_plan* plan, const float* d_terma,
     j.Z = plan->shape[2];
     j.n_cones = plan->n_cones;
     j.accumulate = accumulate;
-    j.nty = (j.Y + kRadTY - 1) / kRadTY;
-    j.ntz = (j.Z + kRadTZ - 1) / kRadTZ;
-    const int64_t n_tiles = (int64_t)j.X * j.nty * j.ntz;
-    CH_REQUIRE(n_tiles < INT_MAX / 2, "ch_convolve_rad: too many tiles");
-    const unsigned blocks =
-        (unsigned)((n_tiles + kRadWaves - 1) / kRadWaves);
     LaunchTimer timer(s);
-    timer.launch(gather_rad, dim3(blocks), dim3(64 * kRadWaves), 0, j,
-                 (int)n_tiles);
+    timer.launch(gather_rad, dim3(blocks, j.n_parts), dim3(64 * kRadWaves), 0,
+                 j);
     CH_HIP(hipGetLastError());
+    if (j.n_parts > 1) {
+        const int64_t n = (int64_t)j.X * j.Y * j.Z;
+        timer.launch(rad_sum, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                     j.parts, j.n_parts, n, d_dose, accumulate);
+        CH_HIP(hipGetLastError());
+    }
     timer.stop();
     return CH_OK;
 }

@@ -246,3 +246,38 @@ def test_water_profiles_against_tank(engine):
         assert dev_in < IN_FIELD, (depth, dev_in)
         assert dev_out < OUT_FIELD, (depth, dev_out)
         assert edge < EDGE_MM, (depth, edge)
+
+
+@pytest.mark.parametrize("n_phi", [1, 6])     # the rows whole, and in parts
+@pytest.mark.parametrize("shape", [(4, 8, 16), (5, 9, 17), (1, 1, 1),
+                                   (3, 7, 33), (8, 16, 31)])
+def test_tiles_and_densities(oracle, engine, shape, n_phi):
+    """Tile and workgroup remainders, boxes at the grid's faces and away
+    from them, taps below index 5, negative and far out-of-range densities,
+    and rows in parts against the oracle; the tolerance of this file."""
+    poly = EdkSet.load().poly(W.SETTINGS["energy_weights"])
+    phis, cum = merge_polar(poly.angles, poly.kernel_cum, n_phi)
+    src = Source("varian_clinac_6MV")
+    src.gantry = 15.0
+    cs = ConeSet(default_thetas(5), phis, cum, semantics="physics",
+                 frame=beam_frame(src))
+    vs = (0.5, 0.3, 0.4)
+    rng = np.random.default_rng(sum(shape))
+    for part in (slice(None), slice(0, 1), slice(-1, None)):
+        for kind in ("plain", "thin", "odd"):
+            rho = rng.uniform(0.2, 1.9, shape).astype(np.float32)
+            if kind == "thin":
+                rho *= np.float32(0.02)
+            if kind == "odd":
+                rho[rng.random(shape) < 0.2] *= np.float32(-1.0)
+                rho[rng.random(shape) < 0.05] = np.float32(1e4)
+            T = np.zeros(shape, np.float32)
+            T[part, part, part] = rng.uniform(0.5, 1.0, T[part, part,
+                                                          part].shape)
+            ref = np.zeros(shape)
+            oracle.convolve_rad(T, rho, ref, vs, cs.dirs, cs.rows, cs.cum,
+                                radiological=True, n_threads=4)
+            for box in (True, False):
+                d = gpu_rad(engine, shape, vs, cs, T, rho, box=box)
+                err = float(np.abs(d - ref).max())
+                assert err <= TOL * np.abs(ref).max(), (kind, box, err)
