@@ -5,8 +5,7 @@
 // linspace(o_a, o_a + n_a s_a, n_a) (conehead/conehead.py:525-533) and
 // evaluates it at the dose grid's axes built the same way, laid out by
 // np.meshgrid with indexing 'xy' (:562-567), so output[i][j][k] is the
-// value at (x_j, y_i, z_k).  One thread per output voxel.  The arithmetic
-// follows numpy and scipy in FP64 without contraction: linspace nodes are
+// value at (x_j, y_i, z_k).  The arithmetic follows numpy and scipy in FP64 without contraction: linspace nodes are
 // k * step + start with the last node equal to stop, the cell of a
 // coordinate is searchsorted(nodes, x) - 1 clamped to [0, n - 2], points
 // outside [node_0, node_{n-1}] give 0, and the eight corner weights are
@@ -20,7 +19,7 @@
 namespace ch {
 
 struct Axis {
-    double start, stop;
+    double start, stop, step;   // step = (stop - start) / (n - 1)
     int n;
 };
 
@@ -31,21 +30,21 @@ __device__ __forceinline__ double node(const Axis& a, int k)
         return a.start;
     if (k == a.n - 1)
         return a.stop;
-    const double step = (a.stop - a.start) / (double)(a.n - 1);
-    return (double)k * step + a.start;
+    return (double)k * a.step + a.start;
 }
 
-// Cell index and fraction of x on the axis; false when x is outside.
-__device__ __forceinline__ bool locate(const Axis& a, double x, int& i,
+// Cell index (-1 when x is outside the axis) and fraction of x.
+__device__ __forceinline__ void locate(const Axis& a, double x, int& i,
                                        double& t)
 {
     const double first = node(a, 0), last = node(a, a.n - 1);
+    i = -1;
+    t = 0.0;
     if (!(x >= first && x <= last))
-        return false;
+        return;
     if (a.n == 1) {
         i = 0;
-        t = 0.0;
-        return true;
+        return;
     }
     // searchsorted(side='left'): first k with node(k) >= x
     int lo = 0, hi = a.n;
@@ -60,47 +59,65 @@ __device__ __forceinline__ bool locate(const Axis& a, double x, int& i,
     i = i < 0 ? 0 : (i > a.n - 2 ? a.n - 2 : i);
     const double g0 = node(a, i), g1 = node(a, i + 1);
     t = (x - g0) / (g1 - g0);
-    return true;
 }
+
+// A voxel's three searches and divisions cost far more than its eight loads,
+// so they are shared: a wavefront's lanes lie along z, `width` of them on a
+// row, and take kRows rows one after the other.  A lane finds its own z once;
+// lane r finds x and y of the wavefront's r-th row, and the others fetch them
+// from it.  The width is 64, or 32 or 16 for dose grids of few slices, where
+// the lanes of a wavefront lie on two or four rows at a time.
+// 512 x 512 x 120 onto 160 x 160 x 128: 82 -> 19 us.
+constexpr int kRows = 8;
 
 __global__ __launch_bounds__(256) void resample_kernel(
     const float* __restrict__ src, int sx, int sy, int sz, Axis ax, Axis ay,
     Axis az, float* __restrict__ dst, int dx, int dy, int dz, Axis bx,
-    Axis by, Axis bz, int swap)
+    Axis by, Axis bz, int swap, int width, int z_groups)
 {
-    const int64_t li = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (li >= (int64_t)dx * dy * dz)
+    const int lane = threadIdx.x & 63;
+    const int64_t rows = (int64_t)dx * dy;
+    const int per = kRows * (64 / width);         // rows of a wavefront, <= 64
+    const int zg = (int)(blockIdx.x % (unsigned)z_groups);
+    const int64_t first = ((int64_t)(blockIdx.x / (unsigned)z_groups) * 4 +
+                           (threadIdx.x >> 6)) * per;
+    if (first >= rows)
         return;
-    const int c = (int)(li % dz);
-    const int b = (int)((li / dz) % dy);
-    const int a = (int)(li / ((int64_t)dz * dy));
-    // output index (a, b, c) -> sample point
-    const double x = swap ? node(bx, b) : node(bx, a);
-    const double y = swap ? node(by, a) : node(by, b);
-    const double z = node(bz, c);
-    int i0, i1, i2;
-    double t0, t1, t2;
-    float out = 0.0f;
-    if (locate(ax, x, i0, t0) && locate(ay, y, i1, t1) &&
-        locate(az, z, i2, t2)) {
-        double v = 0.0;
-        for (int e0 = 0; e0 < 2; ++e0)
-            for (int e1 = 0; e1 < 2; ++e1)
-                for (int e2 = 0; e2 < 2; ++e2) {
-                    double w = 1.0;
-                    w = w * (e0 ? t0 : 1.0 - t0);
-                    w = w * (e1 ? t1 : 1.0 - t1);
-                    w = w * (e2 ? t2 : 1.0 - t2);
-                    const int j0 = sx == 1 ? 0 : i0 + e0;
-                    const int j1 = sy == 1 ? 0 : i1 + e1;
-                    const int j2 = sz == 1 ? 0 : i2 + e2;
-                    const double val =
-                        (double)src[((int64_t)j0 * sy + j1) * sz + j2];
-                    v = v + val * w;
-                }
-        out = (float)v;
+    const int64_t mine = min(first + (lane & (per - 1)), rows - 1);
+    const int a = (int)(mine / dy), b = (int)(mine % dy);
+    int ix, iy, i2;
+    double tx, ty, t2;
+    locate(ax, swap ? node(bx, b) : node(bx, a), ix, tx);
+    locate(ay, swap ? node(by, a) : node(by, b), iy, ty);
+    const int c = zg * width + (lane & (width - 1));
+    locate(az, node(bz, min(c, dz - 1)), i2, t2);
+    const int sub = lane / width;
+    const int o2 = sz == 1 ? 0 : 1, o1 = sy == 1 ? 0 : sz;
+    const int64_t o0 = sx == 1 ? 0 : (int64_t)sy * sz;
+    const double u2 = 1.0 - t2;
+#pragma unroll 2
+    for (int k = 0; k < kRows; ++k) {
+        const int r = k * (64 / width) + sub;
+        const int i0 = __shfl(ix, r), i1 = __shfl(iy, r);
+        const double t0 = __shfl(tx, r), t1 = __shfl(ty, r);
+        if (first + r >= rows || c >= dz)
+            continue;
+        float out = 0.0f;
+        if ((i0 | i1 | i2) >= 0) {
+            const float* p = src + ((int64_t)i0 * sy + i1) * sz + i2;
+            const float f[8] = {p[0],       p[o2],      p[o1],
+                                p[o1 + o2], p[o0],      p[o0 + o2],
+                                p[o0 + o1], p[o0 + o1 + o2]};
+            const double u0 = 1.0 - t0, u1 = 1.0 - t1;
+            const double w[4] = {u0 * u1, u0 * t1, t0 * u1, t0 * t1};
+            double v = 0.0;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v = v + (double)f[e] * (w[e >> 1] * (e & 1 ? t2 : u2));
+            out = (float)v;
+        }
+        dst[(first + r) * dz + c] = out;
     }
-    dst[li] = out;
 }
 
 // CT numbers to densities: a piecewise-linear calibration curve evaluated
@@ -113,39 +130,101 @@ struct CtTable {
     double hu[CH_CT_MAX_POINTS];
     double rho[CH_CT_MAX_POINTS];
     double slope[CH_CT_MAX_POINTS];
+    float at[CH_CT_MAX_POINTS];  // the least float >= hu
     float override_rho[256];  // NaN: keep the curve's density
     int n;
 };
 
-__device__ __forceinline__ float ct_density(const CtTable& c, double x)
+// Entry m of the tables in LDS serves the numbers with m nodes at or below
+// them: m = 0 and m = n are the clamps.  Comparing in FP32 with the least
+// float at or above a node decides as the FP64 comparison does.
+struct CtLds {
+    double hu[CH_CT_MAX_POINTS + 1];
+    double slope[CH_CT_MAX_POINTS + 1];
+    double rho[CH_CT_MAX_POINTS + 1];
+    float over[256];
+};
+
+template <typename T>
+__device__ __forceinline__ float ct_density(const CtTable& c, const CtLds& t,
+                                            T hu)
 {
-    if (x < c.hu[0])
-        return (float)c.rho[0];
-    if (x >= c.hu[c.n - 1])
-        return (float)c.rho[c.n - 1];
-    int j = 0;  // the last node at or below x
-    for (int k = 1; k < c.n - 1; ++k)
-        j = x >= c.hu[k] ? k : j;
-    if (x == c.hu[j])
-        return (float)c.rho[j];
-    return (float)(c.slope[j] * (x - c.hu[j]) + c.rho[j]);
+    const float xf = (float)hu;   // exact
+    int m = 0;
+    for (int k = 0; k < c.n; ++k)
+        m += xf >= c.at[k] ? 1 : 0;
+    const double x = (double)xf, h = t.hu[m], r = t.rho[m];
+    const bool flat = (m == 0 && xf == xf) || m == c.n;
+    // a NaN has m = 0 and takes the slope
+    return flat || x == h ? (float)r : (float)(t.slope[m] * (x - h) + r);
 }
+
+// kCtGroups groups of four voxels per thread, a workgroup's 256 threads side
+// by side in each: 8-byte loads of int16, 16-byte stores.  The curve and the
+// overrides are read from LDS; with the nodes searched in FP64 and the
+// entries read from the kernel arguments the kernel ran at 1.6 TB/s.
+// 512 x 512 x 120 with labels: 137 -> 49 us (4.5 TB/s).
+constexpr int kCtGroups = 4;
+template <typename T>
+struct alignas(sizeof(T)) Ct4 {
+    T v[4];
+};
+struct Label4 {
+    uint8_t v[4];
+};
+struct Rho4 {
+    float v[4];
+};
 
 template <typename T>
 __global__ __launch_bounds__(256) void ct_kernel(
     const T* __restrict__ hu, const uint8_t* __restrict__ labels, int64_t n,
     CtTable c, float* __restrict__ rho)
 {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n)
-        return;
-    float v = ct_density(c, (double)hu[i]);
-    if (labels) {
-        const float o = c.override_rho[labels[i]];
-        if (o == o)
-            v = o;
+    __shared__ CtLds t;
+    for (int m = threadIdx.x; m <= c.n; m += 256) {
+        const int j = m == 0 ? 0 : m - 1;
+        t.hu[m] = c.hu[j];
+        t.slope[m] = c.slope[j];
+        t.rho[m] = c.rho[j];
     }
-    rho[i] = v;
+    if (labels)
+        t.over[threadIdx.x] = c.override_rho[threadIdx.x];
+    __syncthreads();
+    const int64_t base = blockIdx.x * (int64_t)(1024 * kCtGroups);
+    if (base + 1024 * kCtGroups <= n) {
+        Ct4<T> x[kCtGroups];
+        Label4 l[kCtGroups] = {};
+#pragma unroll
+        for (int g = 0; g < kCtGroups; ++g) {
+            const int64_t i = base + 1024 * g + 4 * threadIdx.x;
+            x[g] = *(const Ct4<T>*)(hu + i);
+            if (labels)
+                l[g] = *(const Label4*)(labels + i);
+        }
+#pragma unroll
+        for (int g = 0; g < kCtGroups; ++g) {
+            Rho4 v;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                v.v[q] = ct_density(c, t, x[g].v[q]);
+                if (labels) {
+                    const float o = t.over[l[g].v[q]];
+                    v.v[q] = o == o ? o : v.v[q];
+                }
+            }
+            *(Rho4*)(rho + base + 1024 * g + 4 * threadIdx.x) = v;
+        }
+        return;
+    }
+    for (int64_t i = base + threadIdx.x; i < n; i += 256) {
+        float v = ct_density(c, t, hu[i]);
+        if (labels) {
+            const float o = t.over[labels[i]];
+            v = o == o ? o : v;
+        }
+        rho[i] = v;
+    }
 }
 
 static Axis axis(double origin, double spacing, int n)
@@ -153,6 +232,7 @@ static Axis axis(double origin, double spacing, int n)
     Axis a;
     a.start = origin;
     a.stop = origin + (double)n * spacing;
+    a.step = n > 1 ? (a.stop - a.start) / (double)(n - 1) : 0.0;
     a.n = n;
     return a;
 }
@@ -186,8 +266,13 @@ ch_status ch_resample_linear(const float* d_src, const int32_t src_shape[3],
                dst_shape[0], dst_shape[1]);
     const int64_t n = (int64_t)dst_shape[0] * dst_shape[1] * dst_shape[2];
     CH_REQUIRE(n < (1LL << 31), "ch_resample_linear: grid too large");
+    const int width = dst_shape[2] > 32 ? 64 : dst_shape[2] > 16 ? 32 : 16;
+    const int z_groups = (dst_shape[2] + width - 1) / width;
+    const int64_t per_group = 4 * kRows * (64 / width);
+    const int64_t groups =
+        ((int64_t)dst_shape[0] * dst_shape[1] + per_group - 1) / per_group;
     hipLaunchKernelGGL(
-        resample_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+        resample_kernel, dim3((unsigned)(groups * z_groups)), dim3(256), 0,
         (hipStream_t)stream, d_src, src_shape[0], src_shape[1], src_shape[2],
         axis(src_origin[0], src_spacing[0], src_shape[0]),
         axis(src_origin[1], src_spacing[1], src_shape[1]),
@@ -195,7 +280,8 @@ ch_status ch_resample_linear(const float* d_src, const int32_t src_shape[3],
         dst_shape[0], dst_shape[1], dst_shape[2],
         axis(dst_origin[0], dst_spacing[0], dst_shape[0]),
         axis(dst_origin[1], dst_spacing[1], dst_shape[1]),
-        axis(dst_origin[2], dst_spacing[2], dst_shape[2]), xy_swap ? 1 : 0);
+        axis(dst_origin[2], dst_spacing[2], dst_shape[2]), xy_swap ? 1 : 0,
+        width, z_groups);
     CH_HIP(hipGetLastError());
     return CH_OK;
 }
@@ -227,6 +313,9 @@ ch_status ch_ct_to_density(const void* d_ct, int32_t ct_type, int64_t n,
                    "(point %d)", k);
         c.hu[k] = curve_hu[k];
         c.rho[k] = curve_rho[k];
+        c.at[k] = (float)curve_hu[k];
+        if ((double)c.at[k] < curve_hu[k])
+            c.at[k] = nextafterf(c.at[k], INFINITY);
     }
     for (int k = 0; k + 1 < n_points; ++k)
         c.slope[k] = (c.rho[k + 1] - c.rho[k]) / (c.hu[k + 1] - c.hu[k]);
@@ -234,7 +323,8 @@ ch_status ch_ct_to_density(const void* d_ct, int32_t ct_type, int64_t n,
         c.override_rho[k] = override_rho ? override_rho[k] : NAN;
     if (n == 0)
         return CH_OK;
-    const dim3 grid((unsigned)((n + 255) / 256));
+    const dim3 grid(
+        (unsigned)((n + 1024 * kCtGroups - 1) / (1024 * kCtGroups)));
     if (ct_type == CH_CT_I16)
         hipLaunchKernelGGL(ct_kernel<int16_t>, grid, dim3(256), 0,
                            (hipStream_t)stream, (const int16_t*)d_ct,

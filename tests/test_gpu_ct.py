@@ -2,6 +2,8 @@
 numpy.interp, the routine the calibration curve is defined by, bit for bit;
 density overrides by label; and a CtPhantom through Conehead.calculate
 giving the same dose as a Phantom holding numpy's densities."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -67,6 +69,42 @@ def test_label_overrides():
     assert (got[labels == 7] == np.float32(0.25)).all()
     assert np.array_equal(got[labels == 2],
                           numpy_density(ct[labels == 2], CURVE5))
+
+
+@pytest.mark.parametrize("dtype", [np.int16, np.float32])
+@pytest.mark.parametrize("n", [1, 4095, 4096, 4097, 9000])
+def test_groups_and_remainders(n, dtype):
+    """Whole and partial workgroups at pointers of every alignment of the
+    element type, nodes between two floats, and numbers that are not finite;
+    bit for bit."""
+    curve = ((-1000.0, 0.0012), (-500.1, 0.5), (0.0, 1.0), (300.3, 1.16),
+             (1500.0, 1.82), (3000.0, 2.9))
+    rng = np.random.default_rng(n)
+    for shift in (0, 1, 3):
+        m = n + shift
+        ct = rng.integers(-1500, 4000, size=m).astype(dtype)
+        if dtype == np.float32:
+            ct[shift:] += rng.random(n).astype(np.float32)
+            near = np.float32([-500.1, 300.3, np.inf, -np.inf, np.nan])
+            near = np.concatenate([near, np.nextafter(near[:2],
+                                                      np.float32(1e9))])
+            ct[shift:shift + len(near)] = near[:n]
+        labels = rng.choice(np.array([0, 3], np.uint8), size=m)
+        d_ct, d_lab = DeviceArray.from_host(ct), DeviceArray.from_host(labels)
+        d_rho = DeviceArray((m,), np.float32, zero=True)
+        for lab in (None, d_lab):
+            # the arrays from element `shift` on
+            views = [None if d is None else SimpleNamespace(
+                shape=(n,), dtype=d.dtype,
+                ptr=d.ptr + shift * d.dtype.itemsize)
+                for d in (d_ct, lab, d_rho)]
+            ct_to_density(views[0], curve, views[1],
+                          {3: 0.26} if lab is not None else None, views[2])
+            got = d_rho.download()[shift:]
+            want = numpy_density(ct, curve,
+                                 labels if lab is not None else None,
+                                 {3: 0.26})[shift:]
+            assert np.array_equal(got, want, equal_nan=True)
 
 
 def test_bad_curves_are_refused():

@@ -56,3 +56,38 @@ def test_same_grid_is_the_reference_transpose():
     got = resample(DeviceArray.from_host(dens), dens.shape, ph.origin,
                    ph.spacing, dens.shape, ph.origin, ph.spacing).download()
     assert np.array_equal(got, dose_grid_densities(ph))
+
+
+@pytest.mark.parametrize("dz", [1, 7, 16, 17, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("swap", [True, False])
+def test_lane_layouts_match_scipy(dz, swap):
+    """Every width of a wavefront's row of lanes, ragged in z and in rows,
+    with points outside the source; one unit in the last place as above."""
+    rng = np.random.default_rng(dz)
+    dens = rng.random((9, 12, 11)).astype(np.float32) * 2
+    so, ss = np.array([-2.0, -3.0, -2.5]), np.array([0.5, 0.4, 0.55])
+    dshape = (11, 11, dz) if swap else (13, 7, dz)
+    do, ds = np.array([-2.6, -3.1, -3.0]), np.array([0.5, 0.55, 7.0 / dz])
+    want = scipy_ref(dens, so, ss, dshape, do, ds, swap)
+    got = resample(DeviceArray.from_host(dens), dens.shape, so, ss, dshape,
+                   do, ds, swap_xy=swap).download()
+    assert (want == 0).any() and (dz == 1 or (want > 0).any())
+    np.testing.assert_array_max_ulp(got, want, maxulp=1)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_axis_of_one_node(axis):
+    """A source axis of a single node serves exactly the points on it."""
+    shape = [6, 5, 4]
+    shape[axis] = 1
+    rng = np.random.default_rng(axis)
+    dens = rng.random(shape).astype(np.float32) + 1
+    o, sp = np.array([-1.0, 0.5, 2.0]), np.array([0.5, 0.5, 0.5])
+    got = resample(DeviceArray.from_host(dens), dens.shape, o, sp,
+                   dens.shape, o, sp, swap_xy=False).download()
+    assert np.array_equal(got, dens)
+    off = o.copy()
+    off[axis] += 0.25
+    got = resample(DeviceArray.from_host(dens), dens.shape, o, sp,
+                   dens.shape, off, sp, swap_xy=False).download()
+    assert (got == 0).all()
