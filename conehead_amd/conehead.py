@@ -32,15 +32,45 @@ Settings keys are the reference's (example.py:27-58).  Optional keys:
       swaps the x and y axes (conehead/conehead.py:562-567); False uses the
       densities as given.
 """
+import collections
+import threading
+
 import numpy as np
 
 from . import engine as _engine
 from .cones import ConeSet, beam_frame, default_thetas, kernel_phis
-from .batch import spectral_ok
-from .device import DeviceArray, Stream
+from .batch import DevicePool, spectral_ok
+from .device import HostPool, Stream
 from .dosegrid import DoseGrid
 from .kernel import EdkSet, merge_polar
 from .kernel2 import PolyenergeticKernel
+from .phantom import CtPhantom
+
+# The packaged kernel table, parsed once, and the cone sets of it most
+# recently asked for, by the values of their angles.  A whole call of 50^3
+# voxels and 576 cones spent 3.0 of its 3.6 ms on parsing the table, building
+# the cones and hashing their rows.
+_DEFAULT_LOCK = threading.Lock()
+_DEFAULT = {"kernel": None, "cones": collections.OrderedDict()}
+
+
+def _default_cones(thetas, phis):
+    """ConeSet of the packaged kernel (phis None: all its polar angles)."""
+    with _DEFAULT_LOCK:
+        if _DEFAULT["kernel"] is None:
+            _DEFAULT["kernel"] = PolyenergeticKernel()
+        kernel, sets = _DEFAULT["kernel"], _DEFAULT["cones"]
+        th = np.array(thetas, dtype=np.float64).ravel()
+        ph = np.array(kernel_phis(kernel) if phis is None else phis,
+                      dtype=np.float64).ravel()
+        key = (th.tobytes(), ph.tobytes())
+        cones = sets.pop(key, None)
+        if cones is None:
+            cones = ConeSet(th, ph, kernel)
+        sets[key] = cones
+        while len(sets) > 8:
+            sets.popitem(last=False)
+        return cones
 
 
 def dose_grid_densities(phantom, swap_xy=True):
@@ -66,6 +96,12 @@ class Conehead:
     def __init__(self, engine=None):
         self._engine = engine
         self._stream = None
+        # Device grids and pinned results are kept between calls: an
+        # allocation of each grid cost 0.17 ms, a download into fresh
+        # pageable memory ran at a quarter of the link.  Results view pinned
+        # buffers, which return to the pool when their last array is gone.
+        self._pool = DevicePool(max_free_bytes=1 << 30)
+        self._host = HostPool(max_free_bytes=256 << 20)
         self.dose_grid = None
 
     @property
@@ -96,39 +132,60 @@ class Conehead:
         swap = settings.get("density_xy_swap", True)
         grid = settings.get("dose_grid")
         s = self.stream
+        held = []                   # back to the pool once the stream is idle
+
+        def device(shape, dtype=np.float32):
+            held.append(self._pool.get(tuple(shape), np.dtype(dtype)))
+            return held[-1]
+
+        def upload(arr):
+            a = np.ascontiguousarray(arr)
+            return device(a.shape, a.dtype).upload(a, s)
+
+        d_dens = None
         on_device = hasattr(phantom, "device_densities")  # CtPhantom
         if grid is None and not on_device:
             self.dose_grid = DoseGrid(phantom.size, phantom.origin,
                                       phantom.spacing)
             dens = dose_grid_densities(phantom, swap)
-            d_rho = DeviceArray.from_host(dens, stream=s)
+            dens_shape = dens.shape
+            d_rho = upload(dens)
         else:
             # resampling the phantom's own grid onto itself gives every
             # node's value, i.e. dose_grid_densities bit for bit
-            from .density import resample
+            from .density import ct_to_density, resample
             self.dose_grid = DoseGrid(*grid) if grid is not None else \
                 DoseGrid(phantom.size, phantom.origin, phantom.spacing)
-            if on_device:
+            if type(phantom) is CtPhantom:
+                d_src = ct_to_density(
+                    upload(phantom.ct), phantom.curve,
+                    None if phantom.labels is None
+                    else upload(phantom.labels), phantom.overrides,
+                    device(phantom.ct.shape), stream=s)
+            elif on_device:
                 d_src = phantom.device_densities(stream=s)
             else:
-                d_src = DeviceArray.from_host(phantom.densities, stream=s)
-            d_rho = resample(d_src, tuple(phantom.size), phantom.origin,
-                             phantom.spacing, self.dose_grid.size,
-                             self.dose_grid.origin, self.dose_grid.spacing,
-                             swap_xy=swap, stream=s)
-            dens = d_rho.download(stream=s)
+                d_src = upload(phantom.densities)
+            d_rho = d_dens = resample(
+                d_src, tuple(phantom.size), phantom.origin, phantom.spacing,
+                self.dose_grid.size, self.dose_grid.origin,
+                self.dose_grid.spacing, swap_xy=swap,
+                d_dst=device(int(v) for v in self.dose_grid.size), stream=s)
+            dens_shape = d_rho.shape
         shape = tuple(int(v) for v in self.dose_grid.size)
         origin = np.asarray(self.dose_grid.origin, dtype=np.float64)
         spacing = np.asarray(self.dose_grid.spacing, dtype=np.float64)
-        if dens.shape != shape:
+        if dens_shape != shape:
             raise ValueError("densities %s do not match size %s" %
-                             (dens.shape, shape))
+                             (dens_shape, shape))
 
         semantics = settings.get("semantics", "convolve_c")
         kernel = settings.get("kernel")
         physics = semantics == "physics"
-        if semantics == "convolve_c":
-            kernel = kernel if kernel is not None else PolyenergeticKernel()
+        default = semantics == "convolve_c" and kernel is None
+        if default:
+            phis = settings.get("phis")
+        elif semantics == "convolve_c":
             phis = settings.get("phis")
             phis = kernel_phis(kernel) if phis is None else phis
         elif physics and kernel is None:
@@ -157,8 +214,9 @@ class Conehead:
         if thetas is None:
             thetas = (np.linspace(0, 360 - 360 / 12, 12, dtype=np.float32)
                       if semantics == "cuda_dose" else default_thetas(12))
-        cones = ConeSet(thetas, phis, kernel, semantics=semantics,
-                        frame=beam_frame(source) if physics else None)
+        cones = _default_cones(thetas, phis) if default else \
+            ConeSet(thetas, phis, kernel, semantics=semantics,
+                    frame=beam_frame(source) if physics else None)
 
         method = settings.get("convolution", "fft")
         if method not in ("fft", "gather"):
@@ -166,25 +224,45 @@ class Conehead:
                              "'gather'")
         # the FFT form takes axes of up to 512 voxels; beyond, the gather
         use_fft = method == "fft" and not physics and spectral_ok(shape)
-        d_terma = DeviceArray(shape, np.float32)
+        d_terma = device(shape)
         # the support box only serves the gathers, which clip to it
-        d_box = None if use_fft else DeviceArray((6,), np.int32)
+        d_box = None if use_fft else device((6,), np.int32)
         d_raster = eng.aperture(block, s)
         beam = _engine.beam_struct(source, settings, d_raster, d_rho,
                                    d_terma, d_box)
-        _engine.terma([beam], shape, origin, spacing, stream=s)
-        plan = eng.plan(shape, spacing, cones)
-        d_dose = DeviceArray(shape, np.float32)
-        if physics:
-            _engine.convolve_rad(plan, d_terma, d_rho, d_dose, d_box,
-                                 stream=s)
-        elif use_fft:
-            _engine.convolve_fft(plan, d_terma, d_dose, stream=s)
-        else:
-            _engine.convolve(plan, d_terma, d_dose, d_box, stream=s)
-        dose = d_dose.download(stream=s)
-        self.dose_grid_terma = d_terma.download(stream=s)
-        self.dose_grid_densities = dens
-        self.dose_grid.dose = dose
-        s.sync()
-        return dose
+        # queued without a wait in between; the geometry flag is read once
+        # at the end, and first where something else fails
+        _engine.terma([beam], shape, origin, spacing, stream=s, check=False)
+        results = []
+        try:
+            plan = eng.plan(shape, spacing, cones)
+            d_dose = device(shape)
+            if physics:
+                _engine.convolve_rad(plan, d_terma, d_rho, d_dose, d_box,
+                                     stream=s)
+            elif use_fft:
+                _engine.convolve_fft(plan, d_terma, d_dose, stream=s)
+            else:
+                _engine.convolve(plan, d_terma, d_dose, d_box, stream=s)
+            for d in (d_dose, d_terma, d_dens):
+                if d is not None:
+                    results.append(self._host.get(d.nbytes))
+                    d.download_async(results[-1], stream=s)
+            s.sync()
+        except Exception:
+            s.sync()
+            _engine.terma_check(s)
+            raise
+        try:
+            _engine.terma_check(s)
+        except Exception:
+            for h in results:
+                self._host.put(h)
+            raise
+        arrays = [self._host.as_array(h, shape) for h in results]
+        for d in held:
+            self._pool.put(d)
+        self.dose_grid_terma = arrays[1]
+        self.dose_grid_densities = dens if d_dens is None else arrays[2]
+        self.dose_grid.dose = arrays[0]
+        return arrays[0]

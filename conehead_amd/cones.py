@@ -78,6 +78,38 @@ def beam_aligned_direction(theta, phi, frame):
                      for k in range(3)], dtype=np.float64)
 
 
+def cone_directions(thetas, phis, semantics, frame):
+    """[n_theta * n_phi, 3] directions, theta-major: the functions above with
+    the sine and cosine of each angle taken once (libm's, as there) and the
+    products of all pairs by numpy, whose FP64 operations round like
+    Python's; the same bits."""
+    pi = PI_CONVOLVE_C if semantics == "convolve_c" else math.pi
+
+    def tables(angles):
+        rad = [float(a) * pi / 180.0 for a in angles]
+        return (np.array([math.cos(r) for r in rad], np.float64),
+                np.array([math.sin(r) for r in rad], np.float64))
+
+    c_t, s_t = (v[:, None] for v in tables(thetas))
+    c_p, s_p = (v[None, :] for v in tables(phis))
+    polar = np.broadcast_to(c_p, (len(thetas), len(phis)))
+    if semantics == "convolve_c":
+        d = [c_t * s_p, s_t * s_p, polar]
+    else:
+        d = [c_t * s_p, polar, s_t * s_p]
+    n = d[0] * d[0] + d[1] * d[1] + d[2] * d[2]
+    if semantics == "convolve_c":
+        n_inv = 1.0 / n
+        d = [np.ceil(v * n_inv * 100000) * 0.00001 for v in d]
+    else:
+        n = np.sqrt(n)
+        d = [v / n for v in d]
+        if semantics == "physics":
+            d = [d[0] * frame[0, k] + d[1] * frame[1, k] + d[2] * frame[2, k]
+                 for k in range(3)]
+    return np.ascontiguousarray(np.stack(d, axis=-1).reshape(-1, 3))
+
+
 class ConeSet:
     """n_theta x n_phi cones ordered theta-major as convolve_c loops them
     (conehead/convolve_c.pyx:88-89); cone (i, j) uses kernel row j.
@@ -99,20 +131,10 @@ class ConeSet:
         self.semantics = semantics
         self.frame = np.eye(3) if frame is None else \
             np.asarray(frame, dtype=np.float64).reshape(3, 3)
-        if semantics == "convolve_c":
-            fn = convolve_c_direction
-        elif semantics == "cuda_dose":
-            fn = cuda_dose_direction
-        else:
-            def fn(t, p):
-                return beam_aligned_direction(t, p, self.frame)
         nt, nph = len(self.thetas), len(self.phis)
-        self.dirs = np.zeros((nt * nph, 3), np.float64)
-        self.rows = np.zeros(nt * nph, np.int32)
-        for i, t in enumerate(self.thetas):
-            for j, p in enumerate(self.phis):
-                self.dirs[i * nph + j] = fn(t, p)
-                self.rows[i * nph + j] = j
+        self.dirs = cone_directions(self.thetas, self.phis, semantics,
+                                    self.frame)
+        self.rows = np.tile(np.arange(nph, dtype=np.int32), nt)
         if semantics == "convolve_c":
             self.cum = kernel_rows(kernel, self.phis)
         else:

@@ -5,10 +5,12 @@ accumulated in place with the collapsed-cone convolution of
 `dose_grid_terma`, for the cones thetas x phis (degrees) and the cumulative
 kernel tables kernel.cumulative["%.2f" % phi].  The work runs on the GPU:
 the FP64 TERMA is converted to FP32 on the device, the convolution runs in
-the FFT form (grids whose axes fit its frames) or as the deterministic
-stencil gather, and the FP32 result is added into the FP64 dose on the
-device.  Cone sets, plans and device buffers are kept between calls.
+the FFT form (grids whose axes fit its frames), whose FP32 result is added
+into the FP64 dose on the host, or as the deterministic stencil gather,
+which adds into it on the device.  Cone sets, plans, device buffers and the
+pinned target of the FP32 result are kept between calls.
 """
+import ctypes
 import threading
 
 import numpy as np
@@ -16,7 +18,7 @@ import numpy as np
 from . import _lib
 from . import engine as _engine
 from .cones import ConeSet, kernel_rows
-from .device import DeviceArray
+from .device import DeviceArray, HostBuffer
 
 _ENGINE = None
 _LOCK = threading.Lock()
@@ -75,7 +77,7 @@ def _buffers(shape):
                 "t64": DeviceArray(shape, np.float64),
                 "t": DeviceArray(shape, np.float32),
                 "part": DeviceArray(shape, np.float32),
-                "dose": DeviceArray(shape, np.float64),
+                "host": HostBuffer(4 * int(np.prod(shape))),
                 "box": DeviceArray((6,), np.int32)}
         return b
 
@@ -120,14 +122,26 @@ def _run(plan, shape, terma, dose, fft):
     b = _buffers(shape)
     b["t64"].upload(np.ascontiguousarray(terma))
     _convert(b["t"], b["t64"])
-    b["dose"].upload(np.ascontiguousarray(dose))
     if fft:
+        # the FP32 result crosses the bus once, into pinned memory, instead
+        # of the FP64 dose there and back (101 x 97 x 83 voxels: a download
+        # of the dose 0.47 ms and its upload 0.18 ms of the call's 0.94)
         plan.spectrum()
         _engine.convolve_fft(plan, b["t"], b["part"])
-        _convert(b["dose"], b["part"], accumulate=True)
-    else:
-        _engine.support_box(b["t"], shape, b["box"])
-        _engine.convolve_f64(plan, b["t"], b["dose"], b["box"])
+        part = np.ctypeslib.as_array(
+            ctypes.cast(b["host"].ptr, _lib.c_f32p), shape)
+        b["part"].download(out=part)
+        if dose.flags.c_contiguous and dose.flags.aligned:
+            _lib.check(_lib.lib().ch_host_add_f32(
+                dose.ctypes.data, part.ctypes.data, dose.size))
+        else:
+            np.add(dose, part, out=dose)
+        return
+    if "dose" not in b:
+        b["dose"] = DeviceArray(shape, np.float64)
+    b["dose"].upload(np.ascontiguousarray(dose))
+    _engine.support_box(b["t"], shape, b["box"])
+    _engine.convolve_f64(plan, b["t"], b["dose"], b["box"])
     if dose.flags.c_contiguous:
         b["dose"].download(out=dose)
     else:

@@ -141,8 +141,10 @@ def cones_digest(cones):
     d = getattr(cones, "_digest", None)
     if d is None:
         h = hashlib.sha1()
-        for part in cones.key():
-            h.update(part.encode() if isinstance(part, str) else part)
+        for part in (cones.semantics.encode(), cones.dirs, cones.rows,
+                     cones.cum):
+            h.update(part if isinstance(part, bytes)
+                     else np.ascontiguousarray(part).data)
         d = cones._digest = h.digest()
     return d
 

@@ -47,6 +47,8 @@ ch_status ch_memcpy_d2h(void* h_dst, const void* d_src, size_t bytes,
  * data is there once later work on the stream (an event) has completed. */
 ch_status ch_memcpy_d2h_async(void* h_dst, const void* d_src, size_t bytes,
                               void* stream);
+/* Host arrays: h_dst[i] += (double)h_src[i], on up to four threads. */
+ch_status ch_host_add_f32(double* h_dst, const float* h_src, int64_t n);
 /* Device-to-device copy by a kernel (16-byte aligned pointers). */
 ch_status ch_memcpy_d2d(void* d_dst, const void* d_src, size_t bytes,
                         void* stream);

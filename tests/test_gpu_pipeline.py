@@ -161,3 +161,41 @@ def test_calculate_cuda_dose_reference_settings(oracle, engine, method):
     assert ref.max() > 0
     err = np.abs(dose - ref).max() / ref.max()
     assert err < 1e-4, err
+
+
+def test_calls_do_not_share_results(engine):
+    """Device grids and result buffers are reused between calls: earlier
+    results keep their values, other shapes and default cone sets come and
+    go, and a call that fails leaves the next one as it would be alone."""
+    def case(n, seed, gantry):
+        s = 0.5
+        origin = np.array([-(n - 1) / 2 * s, s / 2, -(n - 1) / 2 * s])
+        rng = np.random.default_rng(seed)
+        dens = (1.0 + 0.3 * rng.random((n, n, n))).astype(np.float32)
+        src = Source("varian_clinac_6MV")
+        src.gantry = gantry
+        blk = Block()
+        blk.set_square(6)
+        thetas = default_thetas(4 + seed)
+        return (src, blk, Phantom(dens, origin, [s] * 3),
+                dict(SETTINGS, thetas=thetas))
+
+    cases = [case(18, 0, 0.0), case(18, 1, 30.0), case(21, 2, 0.0)]
+    alone = []
+    for c in cases:
+        ch = Conehead(engine)
+        alone.append((ch.calculate(*c).copy(), ch.dose_grid_terma.copy()))
+    one = Conehead(engine)
+    kept = []
+    for _ in range(3):
+        for i, c in enumerate(cases):
+            kept.append((i, one.calculate(*c), one.dose_grid_terma))
+        # the grid plane through the source: refused once, then not again
+        bad = case(18, 0, 0.0)
+        ph = bad[2]
+        ph.origin = np.array([-4.25, -100.0, -4.25], np.float32)
+        with pytest.raises(RuntimeError, match="within plane"):
+            one.calculate(*bad)
+    for i, dose, terma in kept:
+        assert np.array_equal(dose, alone[i][0])
+        assert np.array_equal(terma, alone[i][1])

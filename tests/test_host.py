@@ -6,7 +6,9 @@ import numpy as np
 import pytest
 
 from conehead_amd.block import Block, mlc_raster, square_bounds
-from conehead_amd.cones import ConeSet, convolve_c_direction, default_thetas
+from conehead_amd.cones import (ConeSet, beam_aligned_direction,
+                                cone_directions, convolve_c_direction,
+                                cuda_dose_direction, default_thetas)
 from conehead_amd.geometry import line_block_plane_collision
 from conehead_amd.kernel2 import PolyenergeticKernel, merged_kernel
 from conehead_amd.nist import mu_water
@@ -178,6 +180,38 @@ def test_cone_set_order_and_missing_key():
                                   convolve_c_direction(120.0, 67.5))
     with pytest.raises(KeyError):
         ConeSet([0.0], [12.0], k)
+
+
+@pytest.mark.parametrize("semantics", ["convolve_c", "cuda_dose", "physics"])
+@pytest.mark.parametrize("nt,nph", [(12, 48), (1, 1), (7, 13), (0, 3)])
+def test_cone_directions_are_the_single_ones(semantics, nt, nph):
+    """All pairs at once: the bits of the functions of one pair."""
+    rng = np.random.default_rng(nt + nph)
+    th, ph = rng.uniform(-400, 400, nt), rng.uniform(0, 180, nph)
+    if nt == 12:
+        th, ph = default_thetas(12), np.arange(48) * 3.75
+    f = np.linalg.qr(rng.normal(size=(3, 3)))[0]
+    one = {"convolve_c": convolve_c_direction,
+           "cuda_dose": cuda_dose_direction,
+           "physics": lambda t, p: beam_aligned_direction(t, p, f)}[semantics]
+    want = np.array([one(t, p) for t in th for p in ph]).reshape(-1, 3)
+    got = cone_directions(th, ph, semantics, f)
+    assert got.shape == (nt * nph, 3) and got.dtype == np.float64
+    assert got.tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("n", [0, 1, 5, (1 << 17) * 2 - 1, (1 << 17) * 3,
+                               (1 << 19) + 7])
+def test_host_add(n):
+    """FP32 added into FP64 on one to four threads."""
+    from conehead_amd import _lib
+    rng = np.random.default_rng(n)
+    d, s = rng.random(n + 2), rng.random(n).astype(np.float32)
+    want = d.copy()
+    want[1:n + 1] += s
+    _lib.check(_lib.load().ch_host_add_f32(d[1:].ctypes.data, s.ctypes.data,
+                                           n))
+    assert np.array_equal(d, want)
 
 
 def test_beam_aligned_cones():
