@@ -261,10 +261,18 @@ __device__ __forceinline__ void gather_tile(const ConvJob& j, int tile,
 }
 
 // Wavefronts (tiles) per workgroup of the direct gather: consecutive tiles
-// along z, whose rows meet at shared L1 lines.  Measured on MI355X: 8 for a
-// single grid (1.13 -> 1.09 ms at 128^3), 4 for batches (a 64-beam batch
-// took 96 ms with 8 against 79 ms with 4).
-constexpr int kGatherWaves = 8;
+// along z, whose rows meet at shared L1 lines.  The gather is bound by the
+// vector cache: a tap is a 4-byte load per lane, 5 cycles of it at best and
+// 6.4 here (64 x 56 x 560 voxels, 96 cones).  With 8 wavefronts a workgroup's
+// slots wait for the longest of 8 tiles; with 4 that costs less than the
+// lines they no longer share (96 cones, support 48 wide: 48^3 156 -> 156 us,
+// 64 x 56 x 560 346 -> 330, 96^3 420 -> 410, 128^3 704 -> 680, 200 x 200 x
+// 160 1873 -> 1752; with 2 335, 407, 697, 1755; tiles side by side in x and
+// y instead, 392).  Batches: 4 (a 64-beam batch took 96 ms with 8 against 79
+// ms with 4).  Four voxels per lane and 16-byte loads, 16 cycles each, widen
+// the tiles' ranges more than they save (64 x 56 x 560: 438 us with 8 x 32
+// tiles, 624 with 16 x 16).
+constexpr int kGatherWaves = 4;
 constexpr int kBatchWaves = 4;
 
 template <int TY, int TZ, int ACC, typename OutT>
@@ -1194,20 +1202,32 @@ static ch_status convolve_one(const ch_plan* p, const float* d_terma,
 
 // ------------------------------------------------------- support box ----
 
+// kBoxPer voxels per thread, all loads in flight before the first is used;
+// only voxels of the support are located (64 x 56 x 560 voxels: 15.4 -> 6.2
+// us, and 5.8 -> 4.7 for the eighth as many partial boxes).
+constexpr int kBoxPer = 8;
 __global__ __launch_bounds__(256) void box_kernel(const float* __restrict__ T,
                                                   int X, int Y, int Z,
                                                   int32_t* box)
 {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int64_t n = (int64_t)X * Y * Z;
+    const uint32_t n = (uint32_t)X * Y * Z;   // < 2^31
+    const uint32_t first = blockIdx.x * (256u * kBoxPer) + threadIdx.x;
     int32_t v[6] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN};
-    if (i < n && T[i] != 0.0f) {
-        const int z = (int)(i % Z);
-        const int64_t r = i / Z;
-        v[0] = v[3] = (int)(r / Y);
-        v[1] = v[4] = (int)(r % Y);
-        v[2] = v[5] = z;
-    }
+    float t[kBoxPer];
+#pragma unroll
+    for (int q = 0; q < kBoxPer; ++q)
+        t[q] = first + 256u * q < n ? T[first + 256u * q] : 0.0f;
+#pragma unroll
+    for (int q = 0; q < kBoxPer; ++q)
+        if (t[q] != 0.0f) {
+            const uint32_t i = first + 256u * q, r = i / (uint32_t)Z;
+            const int c[3] = {(int)(r / (uint32_t)Y), (int)(r % (uint32_t)Y),
+                              (int)(i - r * (uint32_t)Z)};
+            for (int a = 0; a < 3; ++a) {
+                v[a] = min(v[a], c[a]);
+                v[3 + a] = max(v[3 + a], c[a]);
+            }
+        }
     // one partial box per block; box_finalize reduces them (no atomics)
     block_box_partial(v, box);
 }
@@ -1225,7 +1245,8 @@ ch_status ch_support_box(const float* d_terma, const int32_t h_shape[3],
     const int64_t n = (int64_t)h_shape[0] * h_shape[1] * h_shape[2];
     CH_REQUIRE(n > 0 && n < (1LL << 31), "ch_support_box: grid size");
     hipStream_t s = (hipStream_t)stream;
-    const unsigned blocks = (unsigned)((n + 255) / 256);
+    const unsigned blocks =
+        (unsigned)((n + 256 * kBoxPer - 1) / (256 * kBoxPer));
     void* parts = nullptr;
     ch_status st = stream_scratch(s, kScratchBoxPartials,
                                   (size_t)blocks * kBoxStride *

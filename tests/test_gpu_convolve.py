@@ -358,3 +358,28 @@ def test_diagonal_support_uses_slab_boxes(oracle, engine, kern, tile):
         d_d = DeviceArray(shape, zero=True)
         E.convolve(plan, d_t, d_d, box)
         assert rel_err(d_d.download(), ref) < TOL
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 1, 2047), (2, 32, 32),
+                                   (3, 683, 1), (17, 11, 13), (40, 41, 5)])
+def test_support_box_remainders(engine, shape):
+    """Whole and partial workgroups, single voxels at the corners, NaN and
+    negative values, and an empty grid against numpy."""
+    from conehead_amd import engine as E
+    from conehead_amd.device import DeviceArray
+    rng = np.random.default_rng(sum(shape))
+    corners = [(0, 0, 0), tuple(n - 1 for n in shape),
+               tuple(int(rng.integers(n)) for n in shape)]
+    for n_set in range(4):
+        T = np.zeros(shape, np.float32)
+        for c, v in zip(corners[3 - n_set:] if n_set < 3 else corners,
+                        (np.nan, -1e-30, 2.0)):
+            T[c] = v
+        d_box = DeviceArray((6,), np.int32)
+        E.support_box(DeviceArray.from_host(T), shape, d_box)
+        box = d_box.download()
+        idx = np.argwhere(T != 0)
+        if len(idx):
+            assert box.tolist() == idx.min(0).tolist() + idx.max(0).tolist()
+        else:
+            assert (box[:3] > box[3:]).all()
