@@ -264,23 +264,26 @@ __device__ __forceinline__ void gather_tile(const ConvJob& j, int tile,
 // along z, whose rows meet at shared L1 lines.  The gather is bound by the
 // vector cache: a tap is a 4-byte load per lane, 5 cycles of it at best and
 // 6.4 here (64 x 56 x 560 voxels, 96 cones).  With 8 wavefronts a workgroup's
-// slots wait for the longest of 8 tiles; with 4 that costs less than the
-// lines they no longer share (96 cones, support 48 wide: 48^3 156 -> 156 us,
-// 64 x 56 x 560 346 -> 330, 96^3 420 -> 410, 128^3 704 -> 680, 200 x 200 x
-// 160 1873 -> 1752; with 2 335, 407, 697, 1755; tiles side by side in x and
-// y instead, 392).  Batches: 4 (a 64-beam batch took 96 ms with 8 against 79
-// ms with 4).  Four voxels per lane and 16-byte loads, 16 cycles each, widen
-// the tiles' ranges more than they save (64 x 56 x 560: 438 us with 8 x 32
-// tiles, 624 with 16 x 16).
-constexpr int kGatherWaves = 4;
+// slots wait for the longest of 8 tiles; with 4 it shares fewer lines.  Tiles
+// of one or two rows take 4, of four or eight rows, which read more lines
+// apiece, 8 (us with 8 and 4, 144 cones, 10 cm field; 64^3 within 1 % either
+// way):            1 x 64       2 x 32       4 x 16       8 x 8
+//   128^3       1100 1066    730  720     718  759    1038 1412
+//   160^3       2948 2669   2037 1880    1878 1852    2150 2215
+// and 64 x 56 x 560 with 2 x 32 tiles and 96 cones 346 and 330 (with 2
+// wavefronts 335, tiles side by side in x and y instead 392).  Batches: 4 (a
+// 64-beam batch took 96 ms with 8 against 79 ms with 4).  Four voxels per
+// lane and 16-byte loads, 16 cycles each, widen the tiles' ranges more than
+// they save (64 x 56 x 560: 438 us with 8 x 32 tiles, 624 with 16 x 16).
+constexpr int gather_waves(int ty) { return ty <= 2 ? 4 : 8; }
 constexpr int kBatchWaves = 4;
 
 template <int TY, int TZ, int ACC, typename OutT>
-__global__ __launch_bounds__(64 * kGatherWaves) void gather_single(
+__global__ __launch_bounds__(64 * gather_waves(TY)) void gather_single(
     ConvJob j, int n_tiles)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int tile = blockIdx.x * kGatherWaves + wave;
+    const int tile = blockIdx.x * gather_waves(TY) + wave;
     if (tile >= n_tiles)
         return;
     gather_tile<TY, TZ, ACC, OutT>(j, tile, threadIdx.x & 63);
@@ -956,8 +959,8 @@ static ch_status kernels_for(const ch_plan* p, Kernels<OutT>& k)
     if (tx == 1 && ty == TY && tz == TZ && p->accum_mode == A) {            \
         k.single = gather_single<TY, TZ, A, OutT>;                          \
         k.batch = gather_batch<TY, TZ, A, OutT>;                            \
-        k.tiles_per_block = kGatherWaves;                                   \
-        k.threads = 64 * kGatherWaves;                                      \
+        k.tiles_per_block = gather_waves(TY);                               \
+        k.threads = 64 * gather_waves(TY);                                  \
         k.batch_tiles_per_block = kBatchWaves;                              \
         k.batch_threads = 64 * kBatchWaves;                                 \
         return CH_OK;                                                       \

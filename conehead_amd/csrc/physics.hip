@@ -15,18 +15,15 @@
 // The gather keeps the direct gather's layout: a wavefront owns a 1 x 4 x 16
 // output tile and reads padded copies of the grids.  Every lane walks its
 // cone from its own voxel (R needs the whole path), loading densities only
-// up to the first tap of the tile's union range and (density, T) pairs from
+// up to the first tap of the tile's union range and densities and T from
 // there on.  A workgroup of 8 wavefronts stages each kernel row in LDS once
 // and runs the cones of that row.  R, the index and the increments are FP64;
 // the sums are FP32 with compensation.
 //
 // What bounds it is the latency of the loads and of the path sum they feed,
 // with vector issue at half of its rate, so
-//   - a workgroup's wavefronts are 4 x 2 tiles in x and y: they walk the same
-//     cone at about the same time, and what one of them reads its neighbours
-//     read a few taps later (96^3 voxels, 144 cones: 8 tiles along z 2393 us,
-//     8 along x 2069, 2 x 2 x 2 2098, 4 x 2 1976; a contiguous eighth of the
-//     workgroups per XCD 2371, the XCDs' shares are too uneven);
+//   - a workgroup's wavefronts are neighbouring tiles that walk the same cone
+//     at about the same time, so one reads what another has read (rad_tiles);
 //   - tap addresses are a scalar base per tap plus the lane's own offset, no
 //     vector arithmetic and no range check: every tap of a range lies inside
 //     the padded grids for every lane (the tile's end points are within the
@@ -40,10 +37,11 @@
 //     100 R is its slot;
 //   - a chunk whose T is 0 for the whole wavefront (the corners of an
 //     oblique beam's box) needs one lookup instead of eight;
-//   - a staged row's loads are all in flight before the first store.
-// The times above and at rad_parts are with the path sum as fused
-// multiply-adds, 2.5 % faster than the product and sum kept here, whose
-// indices are the FP64 oracle's.  96^3 voxels, 144 cones: 2540 -> 2010 us.
+//   - a staged row's loads are all in flight before the first store;
+//   - the path sum stays a product and a sum, whose indices are the FP64
+//     oracle's: fused multiply-adds were 2.5 % faster.
+// 144 cones, 96^3 voxels: 2532 -> 2078 us; 128^3 with the gantry at 0 and at
+// 20 degrees 3485 -> 3249 and 6245 -> 5590.
 #include <algorithm>
 #include <climits>
 
@@ -68,11 +66,11 @@ struct RadJob {
     double* parts;         // n_parts > 1: the sums of each part of the rows
     int32_t row_len, n_rows, n_parts;
     int32_t X, Y, Z, n_cones, accumulate, nty, ntz;
+    int32_t wx, wy, wz;    // a workgroup's tiles: wx wy wz = kRadWaves
 };
 
 constexpr int kRadTY = 4, kRadTZ = 16;   // a wavefront's y and z voxels
-constexpr int kRadWX = 4, kRadWY = 2;    // a workgroup's tiles in x and y
-constexpr int kRadWaves = kRadWX * kRadWY;
+constexpr int kRadWaves = 8;
 constexpr int kRadRow = kMaxIndex + 1;
 constexpr int kRadLead = 5;   // unused entries before a row in LDS
 
@@ -321,13 +319,14 @@ __global__ __launch_bounds__(64 * kRadWaves, 6) void gather_rad(RadJob j)
     __shared__ double s_cum[kRadRow + kRadLead];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int gy = (j.nty + kRadWY - 1) / kRadWY;
-    const int tz = blockIdx.x % j.ntz, by = blockIdx.x / j.ntz;
-    const int xw = (by / gy) * kRadWX + wave % kRadWX;
-    const int ty = (by % gy) * kRadWY + wave / kRadWX;
-    const bool live = xw < j.X && ty < j.nty;
+    const int gz = (j.ntz + j.wz - 1) / j.wz, gy = (j.nty + j.wy - 1) / j.wy;
+    const int g = blockIdx.x, gxy = g / gz, wxy = wave / j.wx;
+    const int xw = gxy / gy * j.wx + wave % j.wx;
+    const int ty = gxy % gy * j.wy + wxy % j.wy;
+    const int tz = g % gz * j.wz + wxy / j.wy;
+    const bool live = xw < j.X && ty < j.nty && tz < j.ntz;
     const int x = live ? xw : 0;
-    const int y0 = live ? ty * kRadTY : 0, z0 = tz * kRadTZ;
+    const int y0 = live ? ty * kRadTY : 0, z0 = live ? tz * kRadTZ : 0;
     const int yl = min(y0 + kRadTY - 1, j.Y - 1);
     const int zl = min(z0 + kRadTZ - 1, j.Z - 1);
     const int y = y0 + lane / kRadTZ;
@@ -376,15 +375,29 @@ __global__ __launch_bounds__(256) void rad_sum(const double* parts,
     dose[i] = (accumulate ? dose[i] : 0.0f) + (float)v;
 }
 
+// The tiles of a workgroup: 2 x 1 x 4 in x, y and z where the tiles along z
+// fill groups of four to within an eighth, 4 x 2 x 1 elsewhere (us; z rows of
+// 128, 120 and 64 voxels: 128^3 3263 and 4027, 101 x 83 x 120 1214 and 1523,
+// 64^3 814 and 888; z rows of 96 and 90: 96^3 3195 and 2193, 150 x 120 x 90
+// 10072 and 7080).  One contiguous eighth of the workgroups per XCD: 2371
+// for 1976 at 96^3, the XCDs' shares are too uneven.
+static void rad_tiles(RadJob& j)
+{
+    const bool flat = (j.ntz + 3) / 4 * 4 * 8 <= j.ntz * 9;
+    j.wx = flat ? 2 : 4;
+    j.wy = flat ? 1 : 2;
+    j.wz = flat ? 4 : 1;
+}
+
 // Parts of the kernel rows, each a grid of workgroups of its own: a launch
 // of a few workgroups per slot ends in a round of partly idle compute units
 // (and a small grid never fills them), so the rows are split until there are
-// sixteen per slot (96^3 voxels, 144 cones: 2128 us at two, 1976 at eight,
-// 1948 at sixteen, 1950 at 32).  A slot is a third of a compute unit: the
-// row in LDS.
+// four per slot (us at two, four and eight: 96^3 voxels 2265, 2147, 2145,
+// 101 x 83 x 120 1375, 1215, 1239, 128^3 3255, 3249, 3697).  A slot is a
+// third of a compute unit: the row in LDS.
 static int rad_parts(unsigned blocks, int n_rows)
 {
-    const unsigned want = 16u * 3u * (unsigned)num_cus();
+    const unsigned want = 4u * 3u * (unsigned)num_cus();
     const unsigned parts = (want + blocks - 1) / blocks;
     return (int)std::max(1u, std::min(parts, (unsigned)n_rows));
 }
@@ -413,9 +426,10 @@ ch_status ch_convolve_rad(const ch_plan* plan, const float* d_terma,
     RadJob j;
     j.nty = (plan->shape[1] + kRadTY - 1) / kRadTY;
     j.ntz = (plan->shape[2] + kRadTZ - 1) / kRadTZ;
+    rad_tiles(j);
     const int64_t groups =
-        (int64_t)((plan->shape[0] + kRadWX - 1) / kRadWX) *
-        ((j.nty + kRadWY - 1) / kRadWY) * j.ntz;
+        (int64_t)((plan->shape[0] + j.wx - 1) / j.wx) *
+        ((j.nty + j.wy - 1) / j.wy) * ((j.ntz + j.wz - 1) / j.wz);
     CH_REQUIRE(groups * kRadWaves < INT_MAX / 2,
                "ch_convolve_rad: too many tiles");
     const unsigned blocks = (unsigned)groups;

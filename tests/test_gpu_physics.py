@@ -250,7 +250,8 @@ def test_water_profiles_against_tank(engine):
 
 @pytest.mark.parametrize("n_phi", [1, 6])     # the rows whole, and in parts
 @pytest.mark.parametrize("shape", [(4, 8, 16), (5, 9, 17), (1, 1, 1),
-                                   (3, 7, 33), (8, 16, 31)])
+                                   (3, 7, 33), (8, 16, 31),
+                                   (3, 5, 61), (2, 9, 120)])
 def test_tiles_and_densities(oracle, engine, shape, n_phi):
     """Tile and workgroup remainders, boxes at the grid's faces and away
     from them, taps below index 5, negative and far out-of-range densities,
