@@ -10,6 +10,7 @@ into the FP64 dose on the host, or as the deterministic stencil gather,
 which adds into it on the device.  Cone sets, plans, device buffers and the
 pinned target of the FP32 result are kept between calls.
 """
+import collections
 import ctypes
 import threading
 
@@ -24,7 +25,13 @@ _ENGINE = None
 _LOCK = threading.Lock()
 _CALL_LOCK = threading.Lock()   # one call at a time owns the buffers
 _CONES = {}     # (thetas, phis, id(kernel)) -> (kernel rows, ConeSet)
-_BUFS = {}      # grid shape -> device buffers of one call
+_BUFS = collections.OrderedDict()   # grid shape -> device buffers of one
+_MAX_SHAPES = 5                     # call, least recently used first
+# The pinned target of FP32 results, one for all shapes: allocated per shape,
+# it made a caller that goes round six shapes of 60^3 to 80 voxels pay 0.4 ms
+# a call, more than the upload and download that it saves.
+_PINNED = {}
+_MAX_PINNED = 256 << 20             # larger results take ordinary memory
 
 
 def default_engine():
@@ -69,17 +76,32 @@ def _cones(thetas, phis, kernel):
 
 def _buffers(shape):
     with _LOCK:
-        b = _BUFS.get(shape)
+        b = _BUFS.pop(shape, None)
         if b is None:
-            if len(_BUFS) > 4:
-                _BUFS.clear()
-            b = _BUFS[shape] = {
-                "t64": DeviceArray(shape, np.float64),
-                "t": DeviceArray(shape, np.float32),
-                "part": DeviceArray(shape, np.float32),
-                "host": HostBuffer(4 * int(np.prod(shape))),
-                "box": DeviceArray((6,), np.int32)}
+            while len(_BUFS) >= _MAX_SHAPES:
+                _BUFS.popitem(last=False)
+            b = {"t64": DeviceArray(shape, np.float64),
+                 "t": DeviceArray(shape, np.float32),
+                 "part": DeviceArray(shape, np.float32),
+                 "box": DeviceArray((6,), np.int32)}
+        _BUFS[shape] = b
         return b
+
+
+def _host_result(shape):
+    """A float32 array of this shape for the result: a view of the pinned
+    target, or ordinary memory where that cannot hold it."""
+    nbytes = 4 * int(np.prod(shape))
+    if nbytes > _MAX_PINNED:
+        return np.empty(shape, np.float32)
+    buf = _PINNED.get("buf")
+    if buf is None or buf.nbytes < nbytes:
+        _PINNED.clear()
+        try:
+            buf = _PINNED["buf"] = HostBuffer(nbytes)
+        except _lib.CHError:
+            return np.empty(shape, np.float32)
+    return np.ctypeslib.as_array(ctypes.cast(buf.ptr, _lib.c_f32p), shape)
 
 
 def _convert(dst, src, accumulate=False):
@@ -128,8 +150,7 @@ def _run(plan, shape, terma, dose, fft):
         # of the dose 0.47 ms and its upload 0.18 ms of the call's 0.94)
         plan.spectrum()
         _engine.convolve_fft(plan, b["t"], b["part"])
-        part = np.ctypeslib.as_array(
-            ctypes.cast(b["host"].ptr, _lib.c_f32p), shape)
+        part = _host_result(shape)
         b["part"].download(out=part)
         if dose.flags.c_contiguous and dose.flags.aligned:
             _lib.check(_lib.lib().ch_host_add_f32(

@@ -1,0 +1,116 @@
+"""Memory kept between calls, on the CPU: the drop-in's buffers and the way
+its result reaches doses of any layout, with numpy arrays standing in for
+device and pinned memory."""
+import numpy as np
+import pytest
+
+from conehead_amd import _lib, convolve_c
+
+
+class Dev:
+    """A DeviceArray's interface on host memory."""
+
+    def __init__(self, shape, dtype=np.float32):
+        self.a = np.zeros(shape, dtype)
+        self.shape, self.dtype = self.a.shape, self.a.dtype
+        self.nbytes, self.size = self.a.nbytes, self.a.size
+
+    def upload(self, arr, stream=None):
+        self.a[...] = arr
+        return self
+
+    def download(self, out=None, stream=None):
+        out = np.empty_like(self.a) if out is None else out
+        assert out.flags.c_contiguous and out.dtype == self.dtype
+        out[...] = self.a
+        return out
+
+
+class Pinned:
+    """A HostBuffer's; `made` counts the allocations."""
+    made = 0
+    fail = False
+
+    def __init__(self, nbytes):
+        if Pinned.fail:
+            raise _lib.CHError(_lib.CH_ERR_NOMEM, "no pinned memory")
+        Pinned.made += 1
+        self.nbytes = nbytes
+        self.mem = np.zeros(nbytes, np.uint8)
+        self.ptr = self.mem.ctypes.data
+
+
+class FakePlan:
+    def spectrum(self):
+        pass
+
+
+@pytest.fixture
+def dropin(monkeypatch):
+    """convolve_c's host path with a convolution that doubles TERMA."""
+    def doubled(plan, t, part):
+        part.a[...] = 2 * t.a
+
+    def doubled64(plan, t, dose, box):
+        dose.a[...] += 2 * t.a
+
+    monkeypatch.setattr(convolve_c, "DeviceArray", Dev)
+    monkeypatch.setattr(convolve_c, "HostBuffer", Pinned)
+    monkeypatch.setattr(convolve_c, "_convert",
+                        lambda dst, src: dst.upload(src.a))
+    monkeypatch.setattr(convolve_c._engine, "convolve_fft", doubled)
+    monkeypatch.setattr(convolve_c._engine, "convolve_f64", doubled64)
+    monkeypatch.setattr(convolve_c._engine, "support_box", lambda *a: None)
+    monkeypatch.setattr(_lib, "lib", _lib.load)
+    monkeypatch.setattr(convolve_c, "_BUFS", type(convolve_c._BUFS)())
+    if hasattr(convolve_c, "_PINNED"):
+        monkeypatch.setattr(convolve_c, "_PINNED", {})
+    monkeypatch.setattr(Pinned, "made", 0)
+    monkeypatch.setattr(Pinned, "fail", False)
+
+    def call(shape, dose=None, fft=True):
+        t = np.random.default_rng(sum(shape)).random(shape)
+        dose = np.ones(shape) if dose is None else dose
+        want = dose + 2 * t.astype(np.float32)
+        convolve_c._run(FakePlan(), shape, t, dose, fft)
+        assert np.array_equal(dose, want)
+    return call
+
+
+SHAPES = [(4, 5, n) for n in (11, 3, 7, 5, 9, 2)]
+
+
+def test_dropin_pinned_target_serves_every_shape(dropin):
+    """One pinned buffer as large as the largest result, not one per shape:
+    a caller that goes round more shapes than are kept allocates none."""
+    for _ in range(3):
+        for shape in SHAPES:
+            dropin(shape)
+    assert Pinned.made == 1
+    dropin((4, 5, 12))                     # a larger one replaces it
+    assert Pinned.made == 2
+
+
+def test_dropin_gather_takes_no_pinned_memory(dropin):
+    for shape in SHAPES:
+        dropin(shape, fft=False)
+    assert Pinned.made == 0
+
+
+def test_dropin_without_pinned_memory(dropin, monkeypatch):
+    """Results past the kept size, or no pinned memory to be had: ordinary
+    memory takes its place."""
+    monkeypatch.setattr(Pinned, "fail", True)
+    dropin((4, 5, 6))
+    monkeypatch.setattr(Pinned, "fail", False)
+    monkeypatch.setattr(convolve_c, "_MAX_PINNED", 4 * 4 * 5 * 6 - 1)
+    dropin((4, 5, 6))
+    assert Pinned.made == 0
+
+
+def test_dropin_drops_the_oldest_shape(dropin):
+    for shape in SHAPES[:5]:
+        dropin(shape)
+    dropin(SHAPES[0])
+    dropin(SHAPES[5])
+    assert set(convolve_c._BUFS) == set(SHAPES) - {SHAPES[1]}
