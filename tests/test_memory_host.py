@@ -114,3 +114,37 @@ def test_dropin_drops_the_oldest_shape(dropin):
     dropin(SHAPES[0])
     dropin(SHAPES[5])
     assert set(convolve_c._BUFS) == set(SHAPES) - {SHAPES[1]}
+
+
+@pytest.mark.parametrize("layout", ["C", "F", "swapped", "step", "slice",
+                                    "reversed", "unaligned"])
+def test_dropin_dose_layouts(dropin, layout):
+    shape = (6, 5, 7)
+    dose = {"C": lambda: np.ones(shape),
+            "F": lambda: np.ones(shape, order="F"),
+            "swapped": lambda: np.ones((5, 6, 7)).transpose(1, 0, 2),
+            "step": lambda: np.ones((6, 5, 14))[:, :, ::2],
+            "slice": lambda: np.ones((6, 9, 7))[:, 2:7],
+            "reversed": lambda: np.ones(shape)[::-1, :, ::-1],
+            "unaligned": lambda: np.frombuffer(
+                bytearray(1) + bytearray(np.ones(shape).tobytes()), np.uint8)
+            [1:].view(np.float64).reshape(shape)}[layout]()
+    dropin(shape, dose)
+
+
+@pytest.mark.parametrize("order", [(0, 1, 2), (2, 1, 0), (1, 0, 2),
+                                   (0, 2, 1), (1, 2, 0)])
+def test_result_takes_the_dose_layout(order):
+    """What is added to a dose lies in memory as the dose does, so that the
+    sum runs along both (a C-ordered one under a Fortran-ordered dose costs
+    a cache line per element)."""
+    shape = (6, 5, 7)
+    part = np.random.default_rng(1).random(shape).astype(np.float32)
+    dose = np.empty([shape[a] for a in order]).transpose(np.argsort(order))
+    assert dose.shape == shape
+    got = convolve_c._laid_out_as(dose, part)
+    assert np.array_equal(got, part)
+    assert np.argsort(got.strides).tolist() == \
+        np.argsort(dose.strides).tolist()
+    if order == (0, 1, 2):
+        assert got is part
