@@ -24,13 +24,15 @@ under a caller key, both convolutions are deterministic and groups are
 chosen per request from its own beams, so a request's result is bitwise
 the same alone or inside any batch.
 """
+import collections
 import threading
 
 import numpy as np
 
 from . import _lib
 from . import engine as E
-from .device import DeviceArray, Event, HostPool, Stream, _h
+from .device import (DeviceArray, Event, HostPool, Stream, _h, drop_idle,
+                     keep_idle, take_idle)
 
 PAD_Y = 32   # kYPad of the padded TERMA copy (ch_internal.h)
 PAD_Z = 80   # kZPad
@@ -123,10 +125,11 @@ class DoseRequest:
 
 
 class DevicePool:
-    """Reusable device buffers keyed by (shape, dtype)."""
+    """Reusable device buffers keyed by (shape, dtype).  Idle ones hold at
+    most max_free_bytes; those of the key least recently used go first."""
 
     def __init__(self, max_free_bytes=64 << 30):
-        self._free = {}
+        self._free = collections.OrderedDict()
         self._bytes = 0
         self._max = max_free_bytes
         self._lock = threading.Lock()
@@ -134,29 +137,16 @@ class DevicePool:
     def get(self, shape, dtype=np.float32):
         key = (tuple(shape), np.dtype(dtype).str)
         with self._lock:
-            lst = self._free.get(key)
-            if lst:
-                a = lst.pop()
-                self._bytes -= a.nbytes
-                return a
-        return DeviceArray(tuple(shape), dtype)
+            a = take_idle(self, key)
+        return DeviceArray(tuple(shape), dtype) if a is None else a
 
     def put(self, arr):
-        key = (arr.shape, arr.dtype.str)
         with self._lock:
-            if self._bytes + arr.nbytes > self._max:
-                arr.free()
-                return
-            self._free.setdefault(key, []).append(arr)
-            self._bytes += arr.nbytes
+            keep_idle(self, (arr.shape, arr.dtype.str), arr)
 
     def clear(self):
         with self._lock:
-            for lst in self._free.values():
-                for a in lst:
-                    a.free()
-            self._free.clear()
-            self._bytes = 0
+            drop_idle(self, -1)
 
 
 class BatchHandle:

@@ -2,6 +2,7 @@
 
 The library allocates HBM itself (ch_malloc); numpy arrays are the host side.
 """
+import collections
 import ctypes
 import threading
 
@@ -197,6 +198,39 @@ class HostBuffer:
             pass
 
 
+# The idle buffers of a pool (_free: key -> list, least recently used key
+# first; _bytes: what they hold; _max: what they may), its lock held.
+
+def take_idle(pool, key):
+    lst = pool._free.get(key)
+    if not lst:
+        return None
+    buf = lst.pop()
+    pool._bytes -= buf.nbytes
+    if not lst:
+        del pool._free[key]
+    return buf
+
+
+def drop_idle(pool, limit):
+    """Frees idle buffers until they hold at most `limit` bytes."""
+    while pool._free and pool._bytes > limit:
+        key = next(iter(pool._free))
+        take_idle(pool, key).free()
+
+
+def keep_idle(pool, key, buf):
+    """Adds a buffer, making room for it: with the newest refused instead, a
+    pool full of earlier shapes would allocate every later one anew."""
+    if buf.nbytes > pool._max:
+        buf.free()
+        return
+    drop_idle(pool, pool._max - buf.nbytes)
+    pool._free.setdefault(key, []).append(buf)
+    pool._free.move_to_end(key)
+    pool._bytes += buf.nbytes
+
+
 class _PinnedView:
     """Owner of a HostBuffer while numpy arrays view it; gives the buffer
     back to its pool when the last array is dropped."""
@@ -220,30 +254,25 @@ class HostPool:
     """Reusable pinned host buffers keyed by size.  as_array() hands a buffer
     out as a numpy array that owns it: the buffer returns to the pool when
     that array (and every view of it) is gone, so results are delivered
-    without a host-side copy."""
+    without a host-side copy.
+
+    Idle buffers hold at most max_free_bytes; those of the size least
+    recently used go first."""
 
     def __init__(self, max_free_bytes=4 << 30):
-        self._free = {}
+        self._free = collections.OrderedDict()
         self._bytes = 0
         self._max = max_free_bytes
         self._lock = threading.RLock()
 
     def get(self, nbytes):
         with self._lock:
-            lst = self._free.get(int(nbytes))
-            if lst:
-                b = lst.pop()
-                self._bytes -= b.nbytes
-                return b
-        return HostBuffer(nbytes)
+            b = take_idle(self, int(nbytes))
+        return HostBuffer(nbytes) if b is None else b
 
     def put(self, buf):
         with self._lock:
-            if self._bytes + buf.nbytes > self._max:
-                buf.free()
-                return
-            self._free.setdefault(buf.nbytes, []).append(buf)
-            self._bytes += buf.nbytes
+            keep_idle(self, buf.nbytes, buf)
 
     def as_array(self, buf, shape, dtype=np.float32):
         if int(np.prod(shape)) * np.dtype(dtype).itemsize > buf.nbytes:
@@ -253,8 +282,4 @@ class HostPool:
 
     def clear(self):
         with self._lock:
-            for lst in self._free.values():
-                for b in lst:
-                    b.free()
-            self._free.clear()
-            self._bytes = 0
+            drop_idle(self, -1)

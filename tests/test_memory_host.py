@@ -1,10 +1,10 @@
-"""Memory kept between calls, on the CPU: the drop-in's buffers and the way
-its result reaches doses of any layout, with numpy arrays standing in for
-device and pinned memory."""
+"""Memory kept between calls, on the CPU: the drop-in's buffers, the way its
+result reaches doses of any layout, and the pools, with numpy arrays standing
+in for device and pinned memory."""
 import numpy as np
 import pytest
 
-from conehead_amd import _lib, convolve_c
+from conehead_amd import _lib, batch, convolve_c, device
 
 
 class Dev:
@@ -148,3 +148,55 @@ def test_result_takes_the_dose_layout(order):
         np.argsort(dose.strides).tolist()
     if order == (0, 1, 2):
         assert got is part
+
+
+class Block:
+    """A pooled buffer of either kind; `live` holds those not freed."""
+    live = []
+
+    def __init__(self, shape, dtype=np.uint8):
+        self.shape = shape if isinstance(shape, tuple) else (shape,)
+        self.dtype = np.dtype(dtype)
+        self.nbytes = int(np.prod(self.shape)) * self.dtype.itemsize
+        Block.live.append(self)
+
+    def free(self):
+        Block.live.remove(self)
+
+
+@pytest.fixture(params=["device", "host"])
+def pool(request, monkeypatch):
+    """(pool of at most 100 idle bytes, its buffer of n bytes)"""
+    monkeypatch.setattr(Block, "live", [])
+    if request.param == "device":
+        monkeypatch.setattr(batch, "DeviceArray", Block)
+        p = batch.DevicePool(max_free_bytes=100)
+        return p, lambda n: p.get((n,), np.uint8)
+    monkeypatch.setattr(device, "HostBuffer", Block)
+    p = device.HostPool(max_free_bytes=100)
+    return p, p.get
+
+
+def test_full_pool_keeps_the_shape_in_use(pool):
+    """Buffers of shapes that are gone make room: a pool filled by earlier
+    shapes keeps the present one's."""
+    p, get = pool
+    old = [get(n) for n in (30, 31, 32)]
+    for b in old:
+        p.put(b)
+    a, b = get(40), get(40)
+    p.put(a)                               # the two oldest go
+    p.put(b)
+    assert Block.live == [a, b] and p._bytes == 80
+    assert {get(40), get(40)} == {a, b} and p._bytes == 0
+    c = get(101)                           # larger than the pool
+    for x in (a, c, b):
+        p.put(x)
+    assert Block.live == [a, b]
+    p.put(get(19))                         # fits beside them
+    assert get(40) is b                    # the size is in use again
+    p.put(b)
+    p.put(get(20))                         # so the 19 bytes go
+    assert sorted(x.nbytes for x in Block.live) == [20, 40, 40]
+    p.clear()
+    assert Block.live == [] and p._bytes == 0 and not p._free
