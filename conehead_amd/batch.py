@@ -32,7 +32,7 @@ import numpy as np
 from . import _lib
 from . import engine as E
 from .device import (DeviceArray, Event, HostPool, Stream, _h, drop_idle,
-                     keep_idle, take_idle)
+                     keep_idle, register_pool, take_idle)
 
 PAD_Y = 32   # kYPad of the padded TERMA copy (ch_internal.h)
 PAD_Z = 80   # kZPad
@@ -133,6 +133,7 @@ class DevicePool:
         self._bytes = 0
         self._max = max_free_bytes
         self._lock = threading.Lock()
+        register_pool(self)
 
     def get(self, shape, dtype=np.float32):
         key = (tuple(shape), np.dtype(dtype).str)

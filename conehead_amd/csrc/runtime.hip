@@ -31,6 +31,9 @@ void set_error(const char* fmt, ...)
 ch_status hip_fail(hipError_t e, const char* what, const char* file, int line)
 {
     set_error("%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
+    // reported here: a launch checked later must not report it again, as
+    // after an allocation that is tried once more
+    (void)hipGetLastError();
     return e == hipErrorOutOfMemory ? CH_ERR_NOMEM : CH_ERR_HIP;
 }
 

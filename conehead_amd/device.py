@@ -5,10 +5,36 @@ The library allocates HBM itself (ch_malloc); numpy arrays are the host side.
 import collections
 import ctypes
 import threading
+import weakref
 
 import numpy as np
 
 from . import _lib
+
+
+_POOLS = weakref.WeakSet()   # the pools alive, for trim_pools
+
+
+def register_pool(pool):
+    _POOLS.add(pool)
+
+
+def trim_pools():
+    """Frees what every pool of this process holds idle; returns its size."""
+    freed = 0
+    for pool in list(_POOLS):
+        freed += pool._bytes
+        pool.clear()
+    return freed
+
+
+def allocate(call):
+    """Checks the status of `call`, which allocates; where memory is short it
+    is called again without the idle buffers of the pools."""
+    st = call()
+    if st == _lib.CH_ERR_NOMEM and trim_pools() > 0:
+        st = call()
+    return _lib.check(st)
 
 
 class Stream:
@@ -96,7 +122,8 @@ class DeviceArray:
         self.nbytes = int(np.prod(self.shape, dtype=np.int64)) * \
             self.dtype.itemsize
         p = ctypes.c_void_p()
-        _lib.check(_lib.lib().ch_malloc(ctypes.byref(p), self.nbytes))
+        L = _lib.lib()
+        allocate(lambda: L.ch_malloc(ctypes.byref(p), self.nbytes))
         self.ptr = p.value
         if zero:
             self.zero(stream)
@@ -183,7 +210,8 @@ class HostBuffer:
     def __init__(self, nbytes):
         self.nbytes = int(nbytes)
         p = ctypes.c_void_p()
-        _lib.check(_lib.lib().ch_host_alloc(ctypes.byref(p), self.nbytes))
+        L = _lib.lib()
+        allocate(lambda: L.ch_host_alloc(ctypes.byref(p), self.nbytes))
         self.ptr = p.value
 
     def free(self):
@@ -264,6 +292,7 @@ class HostPool:
         self._bytes = 0
         self._max = max_free_bytes
         self._lock = threading.RLock()
+        register_pool(self)
 
     def get(self, nbytes):
         with self._lock:

@@ -16,7 +16,7 @@ import numpy as np
 
 from . import _lib
 from .cones import ConeSet
-from .device import DeviceArray, Stream, _h
+from .device import DeviceArray, Stream, _h, allocate
 from .nist import mu_water
 
 SETTINGS_KEYS = ("sPri", "sAnn", "zAnn", "rInner", "rOuter", "zExp", "sExp",
@@ -41,7 +41,7 @@ class Plan:
         rows = np.ascontiguousarray(cones.rows, dtype=np.int32)
         cum = np.ascontiguousarray(cones.cum, dtype=np.float64)
         h = ctypes.c_void_p()
-        _lib.check(L.ch_plan_create(
+        allocate(lambda: L.ch_plan_create(
             shp, vs, len(rows), dirs.ctypes.data_as(_lib.c_f64p),
             rows.ctypes.data_as(_lib.c_i32p), cum.shape[0], cum.shape[1],
             cum.ctypes.data_as(_lib.c_f64p), SEMANTICS[cones.semantics],
@@ -94,7 +94,8 @@ class Plan:
     def spectrum(self, stream=None):
         """Builds the kernel spectrum the FFT convolution needs (once);
         returns (frame lengths, half-spectrum pitch, work bytes per beam)."""
-        _lib.check(_lib.lib().ch_plan_spectrum(self.handle, _h(stream)))
+        L = _lib.lib()
+        allocate(lambda: L.ch_plan_spectrum(self.handle, _h(stream)))
         f = (ctypes.c_int32 * 3)()
         pitch = ctypes.c_int32()
         work = ctypes.c_int64()

@@ -199,3 +199,18 @@ def test_calls_do_not_share_results(engine):
     for i, dose, terma in kept:
         assert np.array_equal(dose, alone[i][0])
         assert np.array_equal(terma, alone[i][1])
+
+
+def test_failed_allocation_is_reported_once(engine):
+    """An allocation larger than the card fails as such, and the launches
+    after it are not blamed for it."""
+    from conehead_amd import _lib
+    from conehead_amd import engine as E
+    from conehead_amd.device import DeviceArray
+    with pytest.raises(_lib.CHError) as e:
+        DeviceArray((1 << 42,), np.uint8)
+    assert e.value.status == _lib.CH_ERR_NOMEM
+    t = DeviceArray.from_host(np.ones((3, 4, 5), np.float32))
+    box = DeviceArray((6,), np.int32)
+    E.support_box(t, (3, 4, 5), box)
+    assert box.download().tolist() == [0, 0, 0, 2, 3, 4]

@@ -200,3 +200,40 @@ def test_full_pool_keeps_the_shape_in_use(pool):
     assert sorted(x.nbytes for x in Block.live) == [20, 40, 40]
     p.clear()
     assert Block.live == [] and p._bytes == 0 and not p._free
+
+
+def test_short_memory_empties_the_pools(monkeypatch):
+    """An allocation that fails for want of memory is tried again without
+    the idle buffers of every pool, and fails when none are left."""
+    class Lib:
+        room = 100
+
+        def ch_malloc(self, p, nbytes):
+            if nbytes > Lib.room:
+                return _lib.CH_ERR_NOMEM
+            Lib.room -= nbytes
+            p._obj.value = 1 + nbytes
+            return _lib.CH_OK
+
+        def ch_free(self, ptr):
+            Lib.room += ptr - 1
+            return _lib.CH_OK
+
+        ch_host_alloc, ch_host_free = ch_malloc, ch_free
+
+    one = Lib()
+    monkeypatch.setattr(_lib, "lib", lambda: one)
+    monkeypatch.setattr(device, "_POOLS", type(device._POOLS)())
+    pools = batch.DevicePool(), device.HostPool()
+    a, h = pools[0].get((40,), np.uint8), pools[1].get(30)
+    pools[0].put(a)
+    pools[1].put(h)
+    assert Lib.room == 30
+    b = device.DeviceArray((80,), np.uint8)
+    assert Lib.room == 20 and pools[0]._bytes == pools[1]._bytes == 0
+    with pytest.raises(_lib.CHError) as e:
+        device.HostBuffer(21)
+    assert e.value.status == _lib.CH_ERR_NOMEM
+    b.free()
+    assert Lib.room == 100
+    monkeypatch.undo()       # the freed buffers above end on the fake library
