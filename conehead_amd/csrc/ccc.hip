@@ -1124,16 +1124,23 @@ static ch_status pad_into(const float* T, float* P, const ch_plan* p,
 }
 
 ch_status pad_rad(const ch_plan* p, const float* terma, const float* density,
-                  int32_t n_parts, hipStream_t s, const float** grids,
+                  int32_t* n_parts, hipStream_t s, const float** grids,
                   double** parts)
 {
     std::lock_guard<std::mutex> lock(g_ws_mu);
     Workspace* w = nullptr;
     const size_t n = padded_elems(p);
-    // the sums first, 8-byte aligned
-    const size_t np =
-        (size_t)n_parts * p->shape[0] * p->shape[1] * p->shape[2];
+    const size_t voxels = (size_t)p->shape[0] * p->shape[1] * p->shape[2];
+    // the sums first, 8-byte aligned; none where the workspace may not grow
+    // for them (during a capture, with a live graph on the stream) or the
+    // memory is short
+    size_t np = *n_parts > 1 ? *n_parts * voxels : 0;
     ch_status st = workspace(s, 2 * np + 2 * n, 0, &w);
+    if (st != CH_OK && np > 0) {
+        *n_parts = 1;
+        np = 0;
+        st = workspace(s, 2 * n, 0, &w);
+    }
     if (st != CH_OK)
         return st;
     float* r = w->pad + 2 * np;

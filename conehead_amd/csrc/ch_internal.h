@@ -235,9 +235,10 @@ ch_status stage_table(hipStream_t s, const void* h_src, size_t bytes,
 void release_stage_tables(hipStream_t s);
 // Pads densities and T of plan p's shape into the stream's gather workspace
 // (the layout the gathers read), T right after the densities.  Returns their
-// start and room for n_parts dose grids of FP64 sums.
+// start and, for n_parts > 1, room for n_parts dose grids of FP64 sums;
+// n_parts becomes 1 where there is no room.
 ch_status pad_rad(const ch_plan* p, const float* terma, const float* density,
-                  int32_t n_parts, hipStream_t s, const float** grids,
+                  int32_t* n_parts, hipStream_t s, const float** grids,
                   double** parts);
 
 // Support box of T != 0 from per-block partial boxes: kernels write

@@ -434,8 +434,7 @@ ch_status ch_convolve_rad(const ch_plan* plan, const float* d_terma,
                "ch_convolve_rad: too many tiles");
     const unsigned blocks = (unsigned)groups;
     j.n_parts = rad_parts(blocks, plan->n_rows);
-    ch_status st = pad_rad(plan, d_terma, d_density,
-                           j.n_parts > 1 ? j.n_parts : 0, s, &j.grids,
+    ch_status st = pad_rad(plan, d_terma, d_density, &j.n_parts, s, &j.grids,
                            &j.parts);
     if (st != CH_OK)
         return st;

@@ -282,3 +282,37 @@ def test_tiles_and_densities(oracle, engine, shape, n_phi):
                 d = gpu_rad(engine, shape, vs, cs, T, rho, box=box)
                 err = float(np.abs(d - ref).max())
                 assert err <= TOL * np.abs(ref).max(), (kind, box, err)
+
+
+def test_row_parts_within_a_warmed_workspace(engine, edk):
+    """The partial sums of the kernel rows are no reason to refuse a call:
+    on a stream whose workspace holds the padded grids and may not grow
+    (during a capture, or with a live graph on it) the rows run whole."""
+    from conehead_amd.device import Stream
+    shape, vs = (9, 10, 11), (0.5, 0.5, 0.5)
+    phis, cum = edk
+    src = Source("varian_clinac_6MV")
+    one = ConeSet(default_thetas(6), phis[:1], cum[:1], semantics="physics",
+                  frame=beam_frame(src))
+    cs = physics_cones(edk, 0.0)
+    T, rho = heterogeneous(shape, 8)
+    ref = gpu_rad(engine, shape, vs, cs, T, rho, box=False)
+    s = Stream()
+    d_t, d_r = DeviceArray.from_host(T), DeviceArray.from_host(rho)
+    d_d = DeviceArray(shape)
+    E.convolve_rad(engine.plan(shape, vs, one), d_t, d_r, d_d, stream=s)
+    plan = engine.plan(shape, vs, cs)
+    with E.Graph.capture(s) as cap:
+        E.convolve_rad(plan, d_t, d_r, d_d, stream=s)
+    for _ in range(3):
+        d_d.zero(s)
+        s.sync()
+        cap.graph.launch(s)
+        assert rel_err(d_d.download(stream=s), ref) < TOL
+        d_d.zero(s)
+        E.convolve_rad(plan, d_t, d_r, d_d, stream=s)
+        assert rel_err(d_d.download(stream=s), ref) < TOL
+    cap.graph.close()
+    E.convolve_rad(plan, d_t, d_r, d_d, stream=s)   # and may grow again
+    assert np.array_equal(d_d.download(stream=s), ref)
+    s.close()
