@@ -1,8 +1,7 @@
 // dda_core.h -- FP64 3D-DDA step shared by the trace, plan and TERMA kernels.
 //
 // Same operations as conehead/dda_3d_c.pyx:33-99: step sign from d < 0,
-// |d| in place, t = (s/2)/|d| and dt = s/|d| (1e9 for a zero component;
-// halving is exact, so t is taken as dt/2, the same bits from one division),
+// |d| in place, t = (s/2)/|d| and dt = s/|d| (1e9 for a zero component),
 // then repeated t += dt (never a closed form) and the tie rules
 //   t_x < t_y && t_x < t_z -> x;  t_x < t_y -> z;  t_y < t_z -> y;  else z.
 // Files including this header are compiled with -ffp-contract=off.
@@ -19,6 +18,18 @@ struct Dda {
 
     __device__ __forceinline__ void init(double d0, double d1, double d2,
                                          double v0, double v1, double v2)
+    {
+        init_unit(d0, d1, d2, v0, v1, v2);
+        if (d0 != 0.0) t0 = (v0 / 2) / fabs(d0);
+        if (d1 != 0.0) t1 = (v1 / 2) / fabs(d1);
+        if (d2 != 0.0) t2 = (v2 / 2) / fabs(d2);
+    }
+
+    // For a direction of length 1 with no component near the ends of the
+    // double range: halving is exact while s/|d| neither overflows nor is
+    // subnormal, so t is dt/2, the same bits from one division.
+    __device__ __forceinline__ void init_unit(double d0, double d1, double d2,
+                                              double v0, double v1, double v2)
     {
         s0 = d0 < 0 ? -1 : 1;
         s1 = d1 < 0 ? -1 : 1;

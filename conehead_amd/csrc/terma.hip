@@ -108,7 +108,8 @@ __global__ __launch_bounds__(256) void terma_rays_kernel(
     dirs[3 * r + 1] = dir[1];
     dirs[3 * r + 2] = dir[2];
     Dda d;
-    d.init(dir[0], dir[1], dir[2], P.spacing[0], P.spacing[1], P.spacing[2]);
+    d.init_unit(dir[0], dir[1], dir[2], P.spacing[0], P.spacing[1],
+                P.spacing[2]);
     int32_t m = 0;
     while (c0 >= 0 && c0 < P.X && c1 >= 0 && c1 < P.Y && c2 >= 0 &&
            c2 < P.Z) {
@@ -959,8 +960,8 @@ __device__ __forceinline__ float terma_brick(const TermaParams& P,
             ray_to_source(P, x, y, z, pos2, rv, mag, dir);
             const double r0 = rv[0], r1 = rv[1], r2 = rv[2];
             Dda d;
-            d.init(dir[0], dir[1], dir[2], P.spacing[0], P.spacing[1],
-                   P.spacing[2]);
+            d.init_unit(dir[0], dir[1], dir[2], P.spacing[0], P.spacing[1],
+                        P.spacing[2]);
             const float de =
                 depth_walk(P.density, P.X, P.Y, P.Z, x, y, z, d);
 

@@ -125,3 +125,14 @@ def test_terma_rays_bitwise(oracle):
             assert cnt[i] == len(ot)
             assert np.array_equal(vox[i, :cnt[i]], ov)
             assert np.array_equal(bits(t[i, :cnt[i]]), bits(ot))
+
+
+def test_quotients_past_the_double_range(oracle):
+    """s / |d| overflows where (s / 2) / |d| does not: the crossings are the
+    reference's own operations."""
+    from conehead_amd.dda_3d_c import dda_3d_c
+    for d in ([1e-308] * 3, [1e-308, -1e-308, 1.2e-308]):
+        want = oracle.dda_3d(np.array(d), (9, 10, 11), (4, 5, 6), [2.0] * 3)
+        got = dda_3d_c(np.array(d), (9, 10, 11), (4, 5, 6), [2.0] * 3)
+        assert np.array_equal(got[0], want[0])
+        assert np.array_equal(bits(got[1]), bits(want[1]))
