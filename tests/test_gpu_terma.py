@@ -267,11 +267,16 @@ def test_repeated_calls_keep_their_counters(engine):
     ((24, 21, 40), 5, "mlc", 90.0),       # more lanes than a wavefront holds
     ((20, 22, 24), 2, "narrow", 305.0),   # closed leaf interiors, thin leaves
     ((33, 18, 30), 3, "two", 17.0),       # two rectangles
+    # edges through most voxels of a brick: samples in rounds of lanes
+    ((26, 20, 24), 3, "square", 33.0),
+    ((12, 14, 26), 8, "square", 70.0),
+    ((9, 8, 16), 16, "mlc", 45.0),        # four voxels per round
 ])
 def test_brick_remainders_and_sample_counts(oracle, engine, shape, samples,
                                             aperture, gantry):
     """Grids that end inside a brick, sub-sample counts on both sides of
-    one lane per plane of a voxel's samples, and leaf tables whose rows are
+    one lane per plane of a voxel's samples, rounds of such lanes, and leaf
+    tables whose rows are
     open, closed, interior and edge: the blocked fraction stays bitwise the
     oracle's and the raster gives the same TERMA as the analytic aperture
     (compare)."""
