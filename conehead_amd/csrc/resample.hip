@@ -145,26 +145,37 @@ struct CtLds {
     float over[256];
 };
 
-template <typename T>
-__device__ __forceinline__ float ct_density(const CtTable& c, const CtLds& t,
-                                            T hu)
+// Nodes at or below x (exact for both types of CT numbers).
+__device__ __forceinline__ int ct_nodes(const CtTable& c, float x)
 {
-    const float xf = (float)hu;   // exact
     int m = 0;
     for (int k = 0; k < c.n; ++k)
-        m += xf >= c.at[k] ? 1 : 0;
-    const double x = (double)xf, h = t.hu[m], r = t.rho[m];
+        m += x >= c.at[k] ? 1 : 0;
+    return m;
+}
+// The density with m nodes at or below xf, from entry m of the tables.
+__device__ __forceinline__ float ct_density(const CtTable& c, float xf, int m,
+                                            double h, double slope, double r)
+{
+    const double x = (double)xf;
     const bool flat = (m == 0 && xf == xf) || m == c.n;
     // a NaN has m = 0 and takes the slope
-    return flat || x == h ? (float)r : (float)(t.slope[m] * (x - h) + r);
+    return flat || x == h ? (float)r : (float)(slope * (x - h) + r);
+}
+__device__ __forceinline__ float ct_density(const CtTable& c, const CtLds& t,
+                                            float xf)
+{
+    const int m = ct_nodes(c, xf);
+    return ct_density(c, xf, m, t.hu[m], t.slope[m], t.rho[m]);
 }
 
-// kCtGroups groups of four voxels per thread, a workgroup's 256 threads side
-// by side in each: 8-byte loads of int16, 16-byte stores.  The curve and the
-// overrides are read from LDS; with the nodes searched in FP64 and the
-// entries read from the kernel arguments the kernel ran at 1.6 TB/s.
-// 512 x 512 x 120 with labels: 137 -> 49 us (4.5 TB/s).
-constexpr int kCtGroups = 4;
+// G groups of four voxels per thread, a workgroup's 256 threads side by side
+// in each: 8-byte loads of int16, 16-byte stores.  The curve and the overrides
+// are read from LDS; with the nodes searched in FP64 and the entries read from
+// the kernel arguments the kernel ran at 1.6 TB/s.  512 x 512 x 120 with
+// labels: 137 -> 49 us (4.5 TB/s).  G = 0: a voxel per thread, its entry of
+// the tables read from the arguments, for series too small to fill the chip,
+// where filling LDS and several voxels in a row are latency (ct_groups).
 template <typename T>
 struct alignas(sizeof(T)) Ct4 {
     T v[4];
@@ -177,6 +188,21 @@ struct Rho4 {
 };
 
 template <typename T>
+__global__ __launch_bounds__(256) void ct_small_kernel(
+    const T* __restrict__ hu, const uint8_t* __restrict__ labels, int64_t n,
+    CtTable c, float* __restrict__ rho)
+{
+    const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (i >= n)
+        return;
+    const T x = hu[i];
+    const float o = labels ? c.override_rho[labels[i]] : NAN;
+    const int m = ct_nodes(c, (float)x), j = m == 0 ? 0 : m - 1;
+    const float v = ct_density(c, (float)x, m, c.hu[j], c.slope[j], c.rho[j]);
+    rho[i] = o == o ? o : v;
+}
+
+template <typename T, int G>
 __global__ __launch_bounds__(256) void ct_kernel(
     const T* __restrict__ hu, const uint8_t* __restrict__ labels, int64_t n,
     CtTable c, float* __restrict__ rho)
@@ -191,23 +217,23 @@ __global__ __launch_bounds__(256) void ct_kernel(
     if (labels)
         t.over[threadIdx.x] = c.override_rho[threadIdx.x];
     __syncthreads();
-    const int64_t base = blockIdx.x * (int64_t)(1024 * kCtGroups);
-    if (base + 1024 * kCtGroups <= n) {
-        Ct4<T> x[kCtGroups];
-        Label4 l[kCtGroups] = {};
+    const int64_t base = blockIdx.x * (int64_t)(1024 * G);
+    if (base + 1024 * G <= n) {
+        Ct4<T> x[G];
+        Label4 l[G] = {};
 #pragma unroll
-        for (int g = 0; g < kCtGroups; ++g) {
+        for (int g = 0; g < G; ++g) {
             const int64_t i = base + 1024 * g + 4 * threadIdx.x;
             x[g] = *(const Ct4<T>*)(hu + i);
             if (labels)
                 l[g] = *(const Label4*)(labels + i);
         }
 #pragma unroll
-        for (int g = 0; g < kCtGroups; ++g) {
+        for (int g = 0; g < G; ++g) {
             Rho4 v;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                v.v[q] = ct_density(c, t, x[g].v[q]);
+                v.v[q] = ct_density(c, t, (float)x[g].v[q]);
                 if (labels) {
                     const float o = t.over[l[g].v[q]];
                     v.v[q] = o == o ? o : v.v[q];
@@ -218,13 +244,37 @@ __global__ __launch_bounds__(256) void ct_kernel(
         return;
     }
     for (int64_t i = base + threadIdx.x; i < n; i += 256) {
-        float v = ct_density(c, t, hu[i]);
+        float v = ct_density(c, t, (float)hu[i]);
         if (labels) {
             const float o = t.over[labels[i]];
             v = o == o ? o : v;
         }
         rho[i] = v;
     }
+}
+
+// us for G = 0, 1 and 4, int16 with labels (the FP64 search took 2.7 at 2^15
+// voxels, 3.0 at 2^18, 7.6 at 1.6 M and 37 at 8 M):
+//   2^15   2.4  3.4  7.7     1 M     4.9  4.3  8.2     8 M     29  17  19
+//   2^18   2.7  3.6  7.8     1.6 M   6.7  5.6  8.8     31 M   105  49  47
+static int ct_groups(int64_t n)
+{
+    return n <= 1 << 19 ? 0 : n <= 1 << 24 ? 1 : 4;
+}
+template <typename T>
+static void ct_launch(const T* d_ct, const uint8_t* d_labels, int64_t n,
+                      const CtTable& c, float* d_rho, hipStream_t s)
+{
+    const int g = ct_groups(n);
+    const int64_t per = g == 0 ? 256 : 1024 * g;
+    void (*kernel)(const T*, const uint8_t*, int64_t, CtTable, float*) =
+        ct_small_kernel<T>;
+    if (g == 1)
+        kernel = ct_kernel<T, 1>;
+    else if (g == 4)
+        kernel = ct_kernel<T, 4>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((n + per - 1) / per)),
+                       dim3(256), 0, s, d_ct, d_labels, n, c, d_rho);
 }
 
 static Axis axis(double origin, double spacing, int n)
@@ -323,16 +373,12 @@ ch_status ch_ct_to_density(const void* d_ct, int32_t ct_type, int64_t n,
         c.override_rho[k] = override_rho ? override_rho[k] : NAN;
     if (n == 0)
         return CH_OK;
-    const dim3 grid(
-        (unsigned)((n + 1024 * kCtGroups - 1) / (1024 * kCtGroups)));
     if (ct_type == CH_CT_I16)
-        hipLaunchKernelGGL(ct_kernel<int16_t>, grid, dim3(256), 0,
-                           (hipStream_t)stream, (const int16_t*)d_ct,
-                           d_labels, n, c, d_rho);
+        ct_launch((const int16_t*)d_ct, d_labels, n, c, d_rho,
+                  (hipStream_t)stream);
     else
-        hipLaunchKernelGGL(ct_kernel<float>, grid, dim3(256), 0,
-                           (hipStream_t)stream, (const float*)d_ct, d_labels,
-                           n, c, d_rho);
+        ct_launch((const float*)d_ct, d_labels, n, c, d_rho,
+                  (hipStream_t)stream);
     CH_HIP(hipGetLastError());
     return CH_OK;
 }

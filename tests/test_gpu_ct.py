@@ -107,6 +107,23 @@ def test_groups_and_remainders(n, dtype):
             assert np.array_equal(got, want, equal_nan=True)
 
 
+@pytest.mark.parametrize("dtype", [np.int16, np.float32])
+@pytest.mark.parametrize("n", [1 << 19, (1 << 19) + 1, (1 << 19) + 1023,
+                               1 << 24, (1 << 24) + 1])
+def test_sizes_on_both_sides_of_each_kernel(n, dtype):
+    """One voxel per thread, one and four groups of four: last sizes and
+    first ones, with numbers on nodes and not finite, bit for bit."""
+    rng = np.random.default_rng(n)
+    ct = rng.integers(-1500, 4000, size=n).astype(dtype)
+    if dtype == np.float32:
+        ct[-4:] = [np.nan, np.inf, -np.inf, -1000.0]
+    labels = rng.integers(0, 4, size=n).astype(np.uint8)
+    got = ct_to_density(DeviceArray.from_host(ct), CURVE5,
+                        DeviceArray.from_host(labels), {3: 0.26}).download()
+    assert np.array_equal(got, numpy_density(ct, CURVE5, labels, {3: 0.26}),
+                          equal_nan=True)
+
+
 def test_bad_curves_are_refused():
     d = DeviceArray.from_host(np.zeros(8, np.int16))
     for curve in [((0.0, 1.0), (0.0, 2.0)), ((10.0, 1.0), (-10.0, 2.0)),
