@@ -11,6 +11,8 @@
 // outside [node_0, node_{n-1}] give 0, and the eight corner weights are
 // products of (1 - t) and t accumulated corner by corner in
 // itertools.product order.
+#include <algorithm>
+
 #include "ch_internal.h"
 
 #include <cmath>
@@ -65,11 +67,10 @@ __device__ __forceinline__ void locate(const Axis& a, double x, int& i,
 // so they are shared: a wavefront's lanes lie along z, `width` of them on a
 // row, and take kRows rows one after the other.  A lane finds its own z once;
 // lane r finds x and y of the wavefront's r-th row, and the others fetch them
-// from it.  The width is 64, or 32 or 16 for dose grids of few slices, where
-// the lanes of a wavefront lie on two or four rows at a time.
+// from it.  The width is 64, or down to 4 for dose grids of few slices, where
+// the lanes of a wavefront lie on up to 16 rows at a time.
 // 512 x 512 x 120 onto 160 x 160 x 128: 82 -> 19 us.
-constexpr int kRows = 8;
-
+template <int kRows>
 __global__ __launch_bounds__(256) void resample_kernel(
     const float* __restrict__ src, int sx, int sy, int sz, Axis ax, Axis ay,
     Axis az, float* __restrict__ dst, int dx, int dy, int dz, Axis bx,
@@ -95,7 +96,7 @@ __global__ __launch_bounds__(256) void resample_kernel(
     const int o2 = sz == 1 ? 0 : 1, o1 = sy == 1 ? 0 : sz;
     const int64_t o0 = sx == 1 ? 0 : (int64_t)sy * sz;
     const double u2 = 1.0 - t2;
-#pragma unroll 2
+#pragma unroll (kRows > 1 ? 2 : 1)
     for (int k = 0; k < kRows; ++k) {
         const int r = k * (64 / width) + sub;
         const int i0 = __shfl(ix, r), i1 = __shfl(iy, r);
@@ -287,6 +288,28 @@ static Axis axis(double origin, double spacing, int n)
     return a;
 }
 
+// Rows a lane takes, by the lanes its z row and the others' fill (lanes): more
+// rows share more searches, fewer fill the chip.  us for 8, 4, 2 and 1 rows,
+// and for three searches per voxel:
+//   50^3 onto itself         160 K lanes   5.7  4.7  4.7  5.2     5.5
+//   64^3 onto 32^3            32 K         6.3  5.0  4.3  4.0     4.7
+//   512 x 512 x 120 onto 40^3 102 K        6.6  5.4  4.7  5.0     5.2
+//   128^3 onto 64^3          262 K         6.8  5.5  5.4  6.6     9.0
+//   256 x 256 x 60 onto 128 x 128 x 20
+//                            524 K         7.5  6.5  7.4 10.2    10.6
+//   80^3 onto itself         819 K         7.2  8.3 10.1 14.4
+// Narrow rows (width 4 or 8) take at most two: 512 x 512 x 120 onto one slice
+// of 512 x 512 (1 M lanes) 13.8 us with four, 13.2 with two, 18.7 with one
+// (15.2 with three searches per voxel; 20 with the width kept at 16).
+static int resample_rows(int64_t lanes, int width)
+{
+    const int kr = lanes < 1 << 16   ? 1
+                   : lanes < 1 << 17 ? 2
+                   : lanes < 600000  ? 4
+                                     : 8;
+    return width < 16 ? std::min(kr, 2) : kr;
+}
+
 }  // namespace ch
 
 using namespace ch;
@@ -316,13 +339,23 @@ ch_status ch_resample_linear(const float* d_src, const int32_t src_shape[3],
                dst_shape[0], dst_shape[1]);
     const int64_t n = (int64_t)dst_shape[0] * dst_shape[1] * dst_shape[2];
     CH_REQUIRE(n < (1LL << 31), "ch_resample_linear: grid too large");
-    const int width = dst_shape[2] > 32 ? 64 : dst_shape[2] > 16 ? 32 : 16;
+    int width = 4;
+    while (width < 64 && width < dst_shape[2])
+        width *= 2;
     const int z_groups = (dst_shape[2] + width - 1) / width;
-    const int64_t per_group = 4 * kRows * (64 / width);
-    const int64_t groups =
-        ((int64_t)dst_shape[0] * dst_shape[1] + per_group - 1) / per_group;
+    const int64_t rows = (int64_t)dst_shape[0] * dst_shape[1];
+    const int kr = resample_rows(rows * z_groups * width, width);
+    const int64_t per_group = 4 * kr * (64 / width);
+    const int64_t groups = (rows + per_group - 1) / per_group;
+    auto kernel = resample_kernel<1>;
+    if (kr == 2)
+        kernel = resample_kernel<2>;
+    else if (kr == 4)
+        kernel = resample_kernel<4>;
+    else if (kr == 8)
+        kernel = resample_kernel<8>;
     hipLaunchKernelGGL(
-        resample_kernel, dim3((unsigned)(groups * z_groups)), dim3(256), 0,
+        kernel, dim3((unsigned)(groups * z_groups)), dim3(256), 0,
         (hipStream_t)stream, d_src, src_shape[0], src_shape[1], src_shape[2],
         axis(src_origin[0], src_spacing[0], src_shape[0]),
         axis(src_origin[1], src_spacing[1], src_shape[1]),

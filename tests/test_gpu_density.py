@@ -75,6 +75,25 @@ def test_lane_layouts_match_scipy(dz, swap):
     np.testing.assert_array_max_ulp(got, want, maxulp=1)
 
 
+@pytest.mark.parametrize("dshape", [
+    (181, 181, 2), (250, 250, 3),      # narrow rows, one and two per lane
+    (64, 65, 16), (90, 91, 17),        # rows of 16 and 32 lanes: 2 and 4
+    (100, 100, 70), (97, 103, 63)])    # 8 rows, a ragged and a full width
+def test_rows_per_lane_match_scipy(dshape):
+    """Every count of rows per lane on grids large enough for it, ragged in
+    rows; one unit in the last place as above."""
+    rng = np.random.default_rng(sum(dshape))
+    dens = rng.random((19, 22, 21)).astype(np.float32) * 2
+    so, ss = np.array([-2.0, -3.0, -2.5]), np.array([0.5, 0.4, 0.55])
+    do = np.array([-2.6, -3.1, -2.4])    # z inside the source
+    ds = np.array([11.0, 9.5, 9.0]) / dshape
+    want = scipy_ref(dens, so, ss, dshape, do, ds, False)
+    got = resample(DeviceArray.from_host(dens), dens.shape, so, ss, dshape,
+                   do, ds, swap_xy=False).download()
+    assert (want == 0).any() and (want > 0).any()
+    np.testing.assert_array_max_ulp(got, want, maxulp=1)
+
+
 @pytest.mark.parametrize("axis", [0, 1, 2])
 def test_axis_of_one_node(axis):
     """A source axis of a single node serves exactly the points on it."""
