@@ -1212,23 +1212,23 @@ static ch_status convolve_one(const ch_plan* p, const float* d_terma,
 
 // ------------------------------------------------------- support box ----
 
-// kBoxPer voxels per thread, all loads in flight before the first is used;
-// only voxels of the support are located (64 x 56 x 560 voxels: 15.4 -> 6.2
-// us, and 5.8 -> 4.7 for the eighth as many partial boxes).
-constexpr int kBoxPer = 8;
+// kPer voxels per thread, all loads in flight before the first is used; only
+// voxels of the support are located (64 x 56 x 560 voxels: 15.4 -> 6.2 us, and
+// 5.8 -> 4.7 for the eighth as many partial boxes).
+template <int kPer>
 __global__ __launch_bounds__(256) void box_kernel(const float* __restrict__ T,
                                                   int X, int Y, int Z,
                                                   int32_t* box)
 {
     const uint32_t n = (uint32_t)X * Y * Z;   // < 2^31
-    const uint32_t first = blockIdx.x * (256u * kBoxPer) + threadIdx.x;
+    const uint32_t first = blockIdx.x * (256u * kPer) + threadIdx.x;
     int32_t v[6] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN};
-    float t[kBoxPer];
+    float t[kPer];
 #pragma unroll
-    for (int q = 0; q < kBoxPer; ++q)
+    for (int q = 0; q < kPer; ++q)
         t[q] = first + 256u * q < n ? T[first + 256u * q] : 0.0f;
 #pragma unroll
-    for (int q = 0; q < kBoxPer; ++q)
+    for (int q = 0; q < kPer; ++q)
         if (t[q] != 0.0f) {
             const uint32_t i = first + 256u * q, r = i / (uint32_t)Z;
             const int c[3] = {(int)(r / (uint32_t)Y), (int)(r % (uint32_t)Y),
@@ -1240,6 +1240,16 @@ __global__ __launch_bounds__(256) void box_kernel(const float* __restrict__ T,
         }
     // one partial box per block; box_finalize reduces them (no atomics)
     block_box_partial(v, box);
+}
+
+// Voxels per thread: more leave fewer partial boxes but make a small grid wait
+// for one thread after the other.  us with the reduction, for 1, 2 and 8, half
+// of the voxels lit (1 voxel, with 64-bit divisions, before: 5.5, 5.8, 7.2):
+//   16^3  5.6  5.7  6.7     48^3  6.1  5.9  7.1     80^3   9.0  7.3  7.2
+//   32^3  5.7  5.8  7.1     64^3  7.1  6.2  7.1     128^3 20.9 12.8  8.2
+static int box_per(int64_t n)
+{
+    return n <= 1 << 16 ? 1 : n <= 1 << 18 ? 2 : 8;
 }
 
 }  // namespace ch
@@ -1255,16 +1265,23 @@ ch_status ch_support_box(const float* d_terma, const int32_t h_shape[3],
     const int64_t n = (int64_t)h_shape[0] * h_shape[1] * h_shape[2];
     CH_REQUIRE(n > 0 && n < (1LL << 31), "ch_support_box: grid size");
     hipStream_t s = (hipStream_t)stream;
-    const unsigned blocks =
-        (unsigned)((n + 256 * kBoxPer - 1) / (256 * kBoxPer));
+    const int per = box_per(n);
+    const unsigned blocks = (unsigned)((n + 256 * per - 1) / (256 * per));
+    // scratch for one voxel per thread, so that a stream warmed by a grid
+    // serves every smaller one in a capture
     void* parts = nullptr;
     ch_status st = stream_scratch(s, kScratchBoxPartials,
-                                  (size_t)blocks * kBoxStride *
+                                  (size_t)((n + 255) / 256) * kBoxStride *
                                       sizeof(int32_t),
                                   &parts);
     if (st != CH_OK)
         return st;
-    hipLaunchKernelGGL(box_kernel, dim3(blocks), dim3(256), 0, s, d_terma,
+    auto kernel = box_kernel<1>;
+    if (per == 2)
+        kernel = box_kernel<2>;
+    else if (per == 8)
+        kernel = box_kernel<8>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, d_terma,
                        h_shape[0], h_shape[1], h_shape[2], (int32_t*)parts);
     CH_HIP(hipGetLastError());
     launch_box_finalize((const int32_t*)parts, (int)blocks, d_box, 0,

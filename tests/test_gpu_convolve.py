@@ -361,7 +361,9 @@ def test_diagonal_support_uses_slab_boxes(oracle, engine, kern, tile):
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 1), (1, 1, 2047), (2, 32, 32),
-                                   (3, 683, 1), (17, 11, 13), (40, 41, 5)])
+                                   (3, 683, 1), (17, 11, 13), (40, 41, 5),
+                                   (32, 64, 32), (5, 29, 452),  # 2^16, + 4
+                                   (64, 64, 64), (5, 13, 4033)])  # 2^18, + 1
 def test_support_box_remainders(engine, shape):
     """Whole and partial workgroups, single voxels at the corners, NaN and
     negative values, and an empty grid against numpy."""
