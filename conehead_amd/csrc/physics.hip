@@ -38,10 +38,13 @@
 //   - a chunk whose T is 0 for the whole wavefront (the corners of an
 //     oblique beam's box) needs one lookup instead of eight;
 //   - a staged row's loads are all in flight before the first store;
+//   - the ends of a path and of a range go in chunks of four taps with wide
+//     scalar loads of their table entries (rad_chunk): short ranges, in thin
+//     grids, are mostly ends (chunks of eight 2 to 5 % slower);
 //   - the path sum stays a product and a sum, whose indices are the FP64
 //     oracle's: fused multiply-adds were 2.5 % faster.
-// 144 cones, 96^3 voxels: 2532 -> 2078 us; 128^3 with the gantry at 0 and at
-// 20 degrees 3485 -> 3249 and 6245 -> 5590.
+// 144 cones, 96^3 voxels with the gantry at 0 and at 20 degrees: 1359 -> 1195
+// and 2498 -> 1928 us; 128^3 at 0 3448 -> 3040.
 #include <algorithm>
 #include <climits>
 
@@ -123,28 +126,31 @@ __device__ __forceinline__ float tap_load(const char* base, int64_t tap,
     return *(g_float*)((g_char*)p + voff);
 }
 
-// Densities and T of kUnroll taps from tap t; LAST: the ones at or past the
-// range end uhi take tap uhi - 1 (with path length 0 and T = 0 in rad_step).
-template <bool LAST>
-__device__ __forceinline__ void rad_load(const char* rho, uint32_t voff,
-                                         uint32_t toff, const c_i32* ml,
-                                         int t, int uhi, float (&v)[kUnroll],
-                                         float (&y)[kUnroll])
+// N taps from tap t of the range that ends at uhi: densities into the path sum
+// R, T times the rows' increments into the compensated sum (acc, ac).  LAST:
+// taps at or past uhi take the address of tap uhi - 1, path length 0 and T =
+// 0.  Their table entries are read all the same (a cone's taps are followed by
+// kTapPad unused ones), so the chunk's entries come in wide scalar loads; one
+// load each, with the index held below uhi, cost 3 to 6 % of the gather.
+template <bool LAST, int N>
+__device__ __forceinline__ void rad_chunk(const char* rho, uint32_t voff,
+                                          uint32_t toff, const c_i32* ml,
+                                          const c_f64* ms,
+                                          const double* s_cum, int t, int uhi,
+                                          double& R, double& cprev,
+                                          float& acc, float& ac)
 {
+    static_assert(N <= kTapPad, "entries read past the range");
+    float v[N], y[N];
+    int idx[N];
+    const int32_t last = LAST ? ml[uhi - 1] : 0;
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-        const int q = LAST ? min(t + u, uhi - 1) : t + u;
-        v[u] = tap_load(rho, ml[q], voff);
-        y[u] = tap_load(rho, ml[q], toff);
+    for (int u = 0; u < N; ++u) {
+        const int32_t o = ml[t + u];
+        const int32_t tap = LAST && t + u >= uhi ? last : o;
+        v[u] = tap_load(rho, tap, voff);
+        y[u] = tap_load(rho, tap, toff);
     }
-}
-template <bool LAST>
-__device__ __forceinline__ void rad_step(const c_f64* ms, int t, int uhi,
-                                         const float (&v)[kUnroll],
-                                         double& R,
-                                         int (&idx)[kUnroll],
-                                         float (&y)[kUnroll], bool& lit)
-{
     // For x = 100 R >= 5 the subtraction of 5 is exact (the difference is a
     // multiple of ulp(x) below x), so the slot |floor(x - 5)| + 5, clamped,
     // is min(trunc(x), kMaxIndex + 5); a chunk with a tap below 5 (or NaN,
@@ -153,33 +159,66 @@ __device__ __forceinline__ void rad_step(const c_f64* ms, int t, int uhi,
     int least = kMaxIndex;
     int any = 0;
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
+    for (int u = 0; u < N; ++u) {
         if (LAST)
             y[u] = t + u < uhi ? y[u] : 0.0f;
         any |= __float_as_int(y[u]);
-        const int q = LAST ? min(t + u, uhi - 1) : t + u;
-        const double seg = ms[q] * (LAST && t + u >= uhi ? 0.0 : 1.0);
-        R = R + (double)v[u] * seg;
+        const double g = ms[t + u];
+        R = R + (double)v[u] * (LAST && t + u >= uhi ? 0.0 : g);
         idx[u] = min(trunc_sat(R * 100.0), kMaxIndex + kRadLead);
         least = min(least, idx[u]);
     }
-    lit = __builtin_amdgcn_ballot_w64(any != 0) != 0;
+    const bool lit = __builtin_amdgcn_ballot_w64(any != 0) != 0;
     if (__builtin_amdgcn_ballot_w64(least < kRadLead) != 0) {
         // a real branch: R passes through an empty asm here, so the compiler
         // cannot hoist this work onto every chunk
         double r = R0;
         asm volatile("" : "+v"(r));
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const int q = LAST ? min(t + u, uhi - 1) : t + u;
-            const double seg = ms[q] * (LAST && t + u >= uhi ? 0.0 : 1.0);
-            r = r + (double)v[u] * seg;
+        for (int u = 0; u < N; ++u) {
+            const double g = ms[t + u];
+            r = r + (double)v[u] * (LAST && t + u >= uhi ? 0.0 : g);
             idx[u] = rad_index_of(r * 100.0) + kRadLead;
         }
     }
+    if (!lit) {
+        cprev = s_cum[idx[N - 1]];
+        return;
+    }
+    float some = 0.0f;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const double cv = s_cum[idx[u]];
+        const float k = (float)(cv - cprev);
+        cprev = cv;
+        some = fmaf(k, y[u], some);
+    }
+    rad_kahan(acc, ac, some);
+}
+
+// R along N taps, those at or past the end without length (LAST).
+template <bool LAST, int N>
+__device__ __forceinline__ void rad_path(const char* rho, uint32_t voff,
+                                         const c_i32* ml, const c_f64* ms,
+                                         int t, int end, double& R)
+{
+    float v[N];
+    double g[N];
+    const int32_t last = LAST ? ml[end - 1] : 0;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const int32_t o = ml[t + u];
+        const double s = ms[t + u];
+        v[u] = tap_load(rho, LAST && t + u >= end ? last : o, voff);
+        g[u] = LAST && t + u >= end ? 0.0 : s;
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+        R = R + (double)v[u] * g[u];
 }
 
 constexpr int kRadAhead = 2;   // chunks of densities in flight
+constexpr int kRadTail = 4;    // taps per chunk at the end of a range
 constexpr int kRadStage = (kRadRow + 64 * kRadWaves - 1) / (64 * kRadWaves);
 
 // The lane's sum over every kernel row (all wavefronts of the workgroup call
@@ -257,57 +296,23 @@ __device__ __forceinline__ void rad_rows(const RadJob& j, double* s_cum,
                 // densities only (every source there is outside the box)
                 double R = 0.0;
                 int t = 0;
-                for (; t + kRadAhead * kUnroll <= ulo;
-                     t += kRadAhead * kUnroll) {
-                    float v[kRadAhead * kUnroll];
-#pragma unroll
-                    for (int u = 0; u < kRadAhead * kUnroll; ++u)
-                        v[u] = tap_load(rho, ml[t + u], voff);
-#pragma unroll
-                    for (int u = 0; u < kRadAhead * kUnroll; ++u)
-                        R = R + (double)v[u] * ms[t + u];
+                constexpr int far = kRadAhead * kUnroll;
+                for (; t + far <= ulo; t += far)
+                    rad_path<false, far>(rho, voff, ml, ms, t, ulo, R);
+                if (t + kUnroll <= ulo) {
+                    rad_path<false, kUnroll>(rho, voff, ml, ms, t, ulo, R);
+                    t += kUnroll;
                 }
-                for (; t < ulo; t += kUnroll) {
-                    float v[kUnroll];
-                    double sg[kUnroll];
-#pragma unroll
-                    for (int u = 0; u < kUnroll; ++u) {
-                        const int q = min(t + u, ulo - 1);
-                        v[u] = tap_load(rho, ml[q], voff);
-                        sg[u] = ms[q] * (t + u >= ulo ? 0.0 : 1.0);
-                    }
-#pragma unroll
-                    for (int u = 0; u < kUnroll; ++u)
-                        R = R + (double)v[u] * sg[u];
-                }
+                for (; t < ulo; t += kRadTail)
+                    rad_path<true, kRadTail>(rho, voff, ml, ms, t, ulo, R);
                 double cprev = ulo > 0 ? rad_at(s_cum, R) : 0.0;
                 float acc = 0.0f, ac = 0.0f;
-                for (t = ulo; t < uhi; t += kUnroll) {
-                    float v[kUnroll];
-                    int idx[kUnroll];
-                    float y[kUnroll];
-                    bool lit;
-                    if (t + kUnroll <= uhi) {
-                        rad_load<false>(rho, voff, toff, ml, t, uhi, v, y);
-                        rad_step<false>(ms, t, uhi, v, R, idx, y, lit);
-                    } else {
-                        rad_load<true>(rho, voff, toff, ml, t, uhi, v, y);
-                        rad_step<true>(ms, t, uhi, v, R, idx, y, lit);
-                    }
-                    if (!lit) {
-                        cprev = s_cum[idx[kUnroll - 1]];
-                        continue;
-                    }
-                    float some = 0.0f;
-#pragma unroll
-                    for (int u = 0; u < kUnroll; ++u) {
-                        const double cv = s_cum[idx[u]];
-                        const float k = (float)(cv - cprev);
-                        cprev = cv;
-                        some = fmaf(k, y[u], some);
-                    }
-                    rad_kahan(acc, ac, some);
-                }
+                for (t = ulo; t + kUnroll <= uhi; t += kUnroll)
+                    rad_chunk<false, kUnroll>(rho, voff, toff, ml, ms, s_cum,
+                                              t, uhi, R, cprev, acc, ac);
+                for (; t < uhi; t += kRadTail)
+                    rad_chunk<true, kRadTail>(rho, voff, toff, ml, ms, s_cum,
+                                              t, uhi, R, cprev, acc, ac);
                 rad_kahan(sum, comp, acc);
             }
         }
@@ -375,31 +380,48 @@ __global__ __launch_bounds__(256) void rad_sum(const double* parts,
     dose[i] = (accumulate ? dose[i] : 0.0f) + (float)v;
 }
 
-// The tiles of a workgroup: 2 x 1 x 4 in x, y and z where the tiles along z
-// fill groups of four to within an eighth, 4 x 2 x 1 elsewhere (us; z rows of
-// 128, 120 and 64 voxels: 128^3 3263 and 4027, 101 x 83 x 120 1214 and 1523,
-// 64^3 814 and 888; z rows of 96 and 90: 96^3 3195 and 2193, 150 x 120 x 90
-// 10072 and 7080).  One contiguous eighth of the workgroups per XCD: 2371
-// for 1976 at 96^3, the XCDs' shares are too uneven.
+// The tiles of a workgroup in x, y and z, by the tiles along z: 2 x 1 x 4
+// where they fill groups of four to within an eighth, 2 x 2 x 2 where there
+// are two, 4 x 2 x 1 elsewhere, 2 x 4 x 1 for grids of at most 12 slices (us,
+// 144 cones, the last 72; gantry 0 but where given; consecutive: the eight
+// tiles along z, then y, of range-checked loads and whole rows that this
+// replaced):
+//                          here   4 x 2 x 1  consecutive
+//   128^3                  3040   3783       3448
+//   101 x 83 x 120         1233              1236
+//   64^3                    420    482        529
+//   96^3, 20 degrees              1928       2498
+//   128 x 128 x 20         1028   1210       999
+//   64 x 64 x 30            281    369        548
+//   128 x 128 x 10          712    772        701
+//   64 x 200 x 24           894    975        926
+// One contiguous eighth of the workgroups per XCD: 2371 for 1976 at 96^3, the
+// XCDs' shares are too uneven.
 static void rad_tiles(RadJob& j)
 {
     const bool flat = (j.ntz + 3) / 4 * 4 * 8 <= j.ntz * 9;
-    j.wx = flat ? 2 : 4;
-    j.wy = flat ? 1 : 2;
-    j.wz = flat ? 4 : 1;
+    const bool thin = j.Z <= 12;
+    j.wx = flat || j.ntz == 2 || thin ? 2 : 4;
+    j.wy = flat ? 1 : thin ? 4 : 2;
+    j.wz = flat ? 4 : j.ntz == 2 ? 2 : 1;
 }
 
 // Parts of the kernel rows, each a grid of workgroups of its own: a launch
 // of a few workgroups per slot ends in a round of partly idle compute units
 // (and a small grid never fills them), so the rows are split until there are
-// four per slot (us at two, four and eight: 96^3 voxels 2265, 2147, 2145,
-// 101 x 83 x 120 1375, 1215, 1239, 128^3 3255, 3249, 3697).  A slot is a
-// third of a compute unit: the row in LDS.
-static int rad_parts(unsigned blocks, int n_rows)
+// four per slot (us at two, four and eight, before the tails of ranges took
+// chunks of four: 96^3 voxels 2265, 2147, 2145, 101 x 83 x 120 1375, 1215,
+// 1239, 128^3 3255, 3249, 3697).  Grids two tiles deep that fill the slots
+// keep their rows whole: walks are short there, and a part costs more than
+// the idle slots (128 x 128 x 20 1028 us whole, 1072 in two parts, 1118 in
+// three).  A slot is a third of a compute unit: the row in LDS.
+static int rad_parts(const RadJob& j, unsigned blocks)
 {
-    const unsigned want = 4u * 3u * (unsigned)num_cus();
-    const unsigned parts = (want + blocks - 1) / blocks;
-    return (int)std::max(1u, std::min(parts, (unsigned)n_rows));
+    const unsigned slots = 3u * (unsigned)num_cus();
+    if (j.wz == 2 && blocks >= slots)
+        return 1;
+    const unsigned parts = (4 * slots + blocks - 1) / blocks;
+    return (int)std::max(1u, std::min(parts, (unsigned)j.n_rows));
 }
 
 }  // namespace ch
@@ -424,6 +446,10 @@ ch_status ch_convolve_rad(const ch_plan* plan, const float* d_terma,
                "ch_convolve_rad: plan has no kernel rows");
     hipStream_t s = (hipStream_t)stream;
     RadJob j;
+    j.X = plan->shape[0];
+    j.Y = plan->shape[1];
+    j.Z = plan->shape[2];
+    j.n_rows = plan->n_rows;
     j.nty = (plan->shape[1] + kRadTY - 1) / kRadTY;
     j.ntz = (plan->shape[2] + kRadTZ - 1) / kRadTZ;
     rad_tiles(j);
@@ -433,7 +459,7 @@ ch_status ch_convolve_rad(const ch_plan* plan, const float* d_terma,
     CH_REQUIRE(groups * kRadWaves < INT_MAX / 2,
                "ch_convolve_rad: too many tiles");
     const unsigned blocks = (unsigned)groups;
-    j.n_parts = rad_parts(blocks, plan->n_rows);
+    j.n_parts = rad_parts(j, blocks);
     ch_status st = pad_rad(plan, d_terma, d_density, &j.n_parts, s, &j.grids,
                            &j.parts);
     if (st != CH_OK)
@@ -449,10 +475,6 @@ ch_status ch_convolve_rad(const ch_plan* plan, const float* d_terma,
     j.row_begin = plan->d_row_begin;
     j.cum = plan->d_cum;
     j.row_len = plan->row_len;
-    j.n_rows = plan->n_rows;
-    j.X = plan->shape[0];
-    j.Y = plan->shape[1];
-    j.Z = plan->shape[2];
     j.n_cones = plan->n_cones;
     j.accumulate = accumulate;
     LaunchTimer timer(s);

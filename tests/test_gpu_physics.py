@@ -284,6 +284,21 @@ def test_tiles_and_densities(oracle, engine, shape, n_phi):
                 assert err <= TOL * np.abs(ref).max(), (kind, box, err)
 
 
+@pytest.mark.parametrize("shape", [(130, 96, 17), (40, 44, 12),
+                                   (41, 9, 13), (6, 70, 32)])
+def test_tiles_by_slices(oracle, edk, engine, shape):
+    """Grids two tiles deep that fill the chip (rows whole) and that do not,
+    and the last of the thin ones and the first past them, ragged in x and
+    y, ranges from one tap up; the tolerance of this file."""
+    cs = physics_cones(edk, 30.0, n_theta=3)
+    vs = (0.4, 0.5, 0.3)
+    T, rho = heterogeneous(shape, sum(shape))
+    ref = np.zeros(shape)
+    oracle.convolve_rad(T, rho, ref, vs, cs.dirs, cs.rows, cs.cum,
+                        radiological=True, n_threads=8)
+    assert rel_err(gpu_rad(engine, shape, vs, cs, T, rho), ref) <= TOL
+
+
 def test_row_parts_within_a_warmed_workspace(engine, edk):
     """The partial sums of the kernel rows are no reason to refuse a call:
     on a stream whose workspace holds the padded grids and may not grow
