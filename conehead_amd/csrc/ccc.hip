@@ -264,26 +264,57 @@ __device__ __forceinline__ void gather_tile(const ConvJob& j, int tile,
 // along z, whose rows meet at shared L1 lines.  The gather is bound by the
 // vector cache: a tap is a 4-byte load per lane, 5 cycles of it at best and
 // 6.4 here (64 x 56 x 560 voxels, 96 cones).  With 8 wavefronts a workgroup's
-// slots wait for the longest of 8 tiles; with 4 it shares fewer lines.  Tiles
-// of one or two rows take 4, of four or eight rows, which read more lines
-// apiece, 8 (us with 8 and 4, 144 cones, 10 cm field; 64^3 within 1 % either
-// way):            1 x 64       2 x 32       4 x 16       8 x 8
-//   128^3       1100 1066    730  720     718  759    1038 1412
-//   160^3       2948 2669   2037 1880    1878 1852    2150 2215
-// and 64 x 56 x 560 with 2 x 32 tiles and 96 cones 346 and 330 (with 2
-// wavefronts 335, tiles side by side in x and y instead 392).  Batches: 4 (a
-// 64-beam batch took 96 ms with 8 against 79 ms with 4).  Four voxels per
-// lane and 16-byte loads, 16 cycles each, widen the tiles' ranges more than
-// they save (64 x 56 x 560: 438 us with 8 x 32 tiles, 624 with 16 x 16).
-constexpr int gather_waves(int ty) { return ty <= 2 ? 4 : 8; }
+// slots wait for the longest of 8 tiles; with 4 it shares fewer lines, which
+// quad_block makes up for.  Tiles of one or two rows take 4, but
+//   - tiles of four or eight rows, which read more lines apiece, take 8;
+//   - grids past 2.2 M voxels take 8: where T fills them their rows no longer
+//     stay in L2;
+//   - 16 tiles along z, or a multiple, take 8: groups of four then lie alike in
+//     every row, and those at the lit slices all land on the same CUs;
+//   - fewer than 2800 tiles take 8: the chip is not full with either.
+// us with 8 and 4 (96 cones, 2 x 32 tiles; lit: a 10 cm field; full: T
+// everywhere):
+//                     lit          full                      lit          full
+//   48^3           167  169    180  183     128^3         633  595   3338 3190
+//   64^3           200  190    262  244     150^3        1142 1034   9944 9248
+//   100^3          407  393   1553 1505     140 x 90 x 200            5113 5273
+//   64 x 56 x 560  300  286   2475 2287     50 x 50 x 500 250  322   1212 1234
+// with 1 x 64 tiles 150^3 1559 1433 and 9343 11322; 4 x 16 and 8 x 8 tiles at
+// 128^3 718 759 and 1038 1412.  Batches: 4 (a 64-beam batch took 96 ms with 8
+// against 79 ms with 4).  Four voxels per lane and 16-byte loads, 16 cycles
+// each, widen the tiles' ranges more than they save (64 x 56 x 560: 438 us
+// with 8 x 32 tiles, 624 with 16 x 16).
+constexpr int kGatherWaves = 8;   // at most
+static int gather_waves(const ch_plan* p)
+{
+    const int64_t X = p->shape[0], Y = p->shape[1], Z = p->shape[2];
+    const int ty = p->tile[1];
+    const int64_t ntz = (Z + p->tile[2] - 1) / p->tile[2];
+    const int64_t tiles = X * ((Y + ty - 1) / ty) * ntz;
+    return ty <= 2 && tiles >= 2800 && X * Y * Z <= 2200000 && ntz % 16 != 0
+               ? 4
+               : kGatherWaves;
+}
 constexpr int kBatchWaves = 4;
 
+// Workgroups of four tiles: four consecutive ones on each XCD in turn, so
+// that neighbouring rows meet in one L2 (workgroups go to the eight XCDs round
+// robin).
+__device__ __forceinline__ unsigned quad_block()
+{
+    const unsigned b = blockIdx.x, first = b / 32 * 32, r = b % 32;
+    if (first + 32 > gridDim.x)
+        return b;
+    return first + r % 8 * 4 + r / 8;
+}
+
 template <int TY, int TZ, int ACC, typename OutT>
-__global__ __launch_bounds__(64 * gather_waves(TY)) void gather_single(
+__global__ __launch_bounds__(64 * kGatherWaves) void gather_single(
     ConvJob j, int n_tiles)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int tile = blockIdx.x * gather_waves(TY) + wave;
+    const int tile = blockDim.x == 256 ? (int)quad_block() * 4 + wave
+                                       : (int)blockIdx.x * 8 + wave;
     if (tile >= n_tiles)
         return;
     gather_tile<TY, TZ, ACC, OutT>(j, tile, threadIdx.x & 63);
@@ -959,8 +990,8 @@ static ch_status kernels_for(const ch_plan* p, Kernels<OutT>& k)
     if (tx == 1 && ty == TY && tz == TZ && p->accum_mode == A) {            \
         k.single = gather_single<TY, TZ, A, OutT>;                          \
         k.batch = gather_batch<TY, TZ, A, OutT>;                            \
-        k.tiles_per_block = gather_waves(TY);                               \
-        k.threads = 64 * gather_waves(TY);                                  \
+        k.tiles_per_block = gather_waves(p);                                \
+        k.threads = 64 * k.tiles_per_block;                                 \
         k.batch_tiles_per_block = kBatchWaves;                              \
         k.batch_threads = 64 * kBatchWaves;                                 \
         return CH_OK;                                                       \

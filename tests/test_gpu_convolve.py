@@ -141,6 +141,30 @@ def test_tiles_and_accumulation_modes(oracle, engine, kern, tile, accum):
     plan.set_accum(2)
 
 
+@pytest.mark.parametrize("shape", [
+    (61, 60, 70), (64, 60, 65),            # groups of four, 32 at a time
+    (57, 49, 63),                          # the first with enough tiles
+    (20, 20, 512),                         # 16 tiles along z: eight
+    (131, 130, 130)])                      # past the size for four
+@pytest.mark.parametrize("tile", [(1, 1, 64), (1, 2, 32)])
+def test_workgroups_take_every_tile_once(engine, kern, shape, tile):
+    """Four or eight tiles per workgroup, in the order that the dispatch
+    picks, ragged at the end: the bits of the batched gather's own order, on
+    a dose full of other values."""
+    from conehead_amd import engine as E
+    from conehead_amd.device import DeviceArray
+    rng = np.random.default_rng(sum(shape))
+    cs, _ = cones(kern, 3, 2)
+    plan = engine.plan(shape, (0.3, 0.3, 0.3), cs, tile=tile)
+    d_t = DeviceArray.from_host(
+        (rng.random(shape) * (rng.random(shape) < 0.3)).astype(np.float32))
+    d_d = DeviceArray.from_host(np.full(shape, np.nan, np.float32))
+    E.convolve(plan, d_t, d_d, None)
+    got = d_d.download()
+    E.convolve_batch([(plan, d_t, d_d, None, False)])
+    assert np.isfinite(got).all() and np.array_equal(got, d_d.download())
+
+
 def test_batch_equals_single_bitwise(engine, kern):
     """Deterministic gather: a job gives the same bits alone and inside a
     batch of jobs with other shapes and cone sets."""
