@@ -54,7 +54,9 @@ def default_tile(plan):
 
 
 def _shape_key(plan):
-    return "%dx%dx%d/%d" % (plan.shape + (plan.n_cones,))
+    # "tile2": workgroups of four tiles on some grids; tiles timed with eight
+    # everywhere are not read
+    return "tile2/%dx%dx%d/%d" % (plan.shape + (plan.n_cones,))
 
 
 def _load_cache():

@@ -1,6 +1,6 @@
-"""Memory kept between calls, on the CPU: the drop-in's buffers, the way its
-result reaches doses of any layout, and the pools, with numpy arrays standing
-in for device and pinned memory."""
+"""What is kept between calls, on the CPU: the drop-in's buffers, the way its
+result reaches doses of any layout, the pools and the tuned tiles, with numpy
+arrays standing in for device and pinned memory."""
 import numpy as np
 import pytest
 
@@ -237,3 +237,28 @@ def test_short_memory_empties_the_pools(monkeypatch):
     b.free()
     assert Lib.room == 100
     monkeypatch.undo()       # the freed buffers above end on the fake library
+
+
+def test_tiles_of_earlier_workgroups_are_not_read(tmp_path, monkeypatch):
+    """Tiles timed when the gather's workgroups were others stay in the cache
+    file; tuning times anew."""
+    import json
+    from types import SimpleNamespace
+    from conehead_amd import autotune
+
+    class Timed(Exception):
+        pass
+
+    def timing(*a):
+        raise Timed
+
+    path = tmp_path / "tiles.json"
+    path.write_text(json.dumps({"10x11x12/6": {
+        "tile": [1, 1, 64], "ms": {"1x1x64": 1.0}}}))
+    monkeypatch.setattr(autotune, "CACHE_PATH", str(path))
+    monkeypatch.setattr(autotune, "_memo", {})
+    monkeypatch.setattr(autotune, "Stream", timing)
+    plan = SimpleNamespace(shape=(10, 11, 12), n_cones=6,
+                           set_tile=lambda *t: None)
+    with pytest.raises(Timed):
+        autotune.tune(plan)
