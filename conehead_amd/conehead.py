@@ -100,8 +100,10 @@ class Conehead:
         # allocation of each grid cost 0.17 ms, a download into fresh
         # pageable memory ran at a quarter of the link.  Results view pinned
         # buffers, which return to the pool when their last array is gone.
+        # A caller that keeps its results gets ordinary memory once the
+        # pinned results alive and idle would pass max_bytes.
         self._pool = DevicePool(max_free_bytes=1 << 30)
-        self._host = HostPool(max_free_bytes=256 << 20)
+        self._host = HostPool(max_free_bytes=512 << 20, max_bytes=1 << 30)
         self.dose_grid = None
 
     @property
@@ -121,6 +123,11 @@ class Conehead:
 
     def calculate(self, source, block, phantom, settings):
         """TERMA and dose of one beam; returns the FP32 dose grid.
+
+        The returned arrays are the caller's, as numpy's are.  Up to 1 GiB of
+        results still referenced they lie in pinned memory, which goes to a
+        later call when the last view of them is dropped; results past that
+        lie in ordinary memory.
 
         The dose grid is the phantom's own (conehead/conehead.py:536) unless
         settings['dose_grid'] = (size, origin, spacing) names another one;
@@ -246,8 +253,9 @@ class Conehead:
                 _engine.convolve(plan, d_terma, d_dose, d_box, stream=s)
             for d in (d_dose, d_terma, d_dens):
                 if d is not None:
-                    results.append(self._host.get(d.nbytes))
-                    d.download_async(results[-1], stream=s)
+                    results.append((d, self._host.try_get(d.nbytes)))
+                    if results[-1][1] is not None:
+                        d.download_async(results[-1][1], stream=s)
             s.sync()
         except Exception:
             s.sync()
@@ -256,10 +264,12 @@ class Conehead:
         try:
             _engine.terma_check(s)
         except Exception:
-            for h in results:
-                self._host.put(h)
+            for _, h in results:
+                if h is not None:
+                    self._host.put(h)
             raise
-        arrays = [self._host.as_array(h, shape) for h in results]
+        arrays = [d.download(stream=s) if h is None
+                  else self._host.as_array(h, shape) for d, h in results]
         for d in held:
             self._pool.put(d)
         self.dose_grid_terma = arrays[1]

@@ -285,19 +285,40 @@ class HostPool:
     without a host-side copy.
 
     Idle buffers hold at most max_free_bytes; those of the size least
-    recently used go first."""
+    recently used go first.  max_bytes bounds all buffers of the pool, handed
+    out or idle, for try_get."""
 
-    def __init__(self, max_free_bytes=4 << 30):
+    def __init__(self, max_free_bytes=4 << 30, max_bytes=None):
         self._free = collections.OrderedDict()
         self._bytes = 0
         self._max = max_free_bytes
+        self._max_alive = max_bytes
+        self._alive = weakref.WeakSet()
         self._lock = threading.RLock()
         register_pool(self)
 
     def get(self, nbytes):
         with self._lock:
             b = take_idle(self, int(nbytes))
-        return HostBuffer(nbytes) if b is None else b
+        if b is None:
+            b = HostBuffer(nbytes)
+            self._alive.add(b)
+        return b
+
+    def try_get(self, nbytes):
+        """A buffer, or None where it would take the pool past max_bytes
+        (idle buffers make room) or no pinned memory is to be had."""
+        with self._lock:
+            if self._max_alive is not None and int(nbytes) not in self._free:
+                out = sum(b.nbytes for b in self._alive if b.ptr) - \
+                    self._bytes
+                if out + nbytes > self._max_alive:
+                    return None
+                drop_idle(self, self._max_alive - out - nbytes)
+        try:
+            return self.get(nbytes)
+        except _lib.CHError:
+            return None
 
     def put(self, buf):
         with self._lock:

@@ -214,3 +214,33 @@ def test_failed_allocation_is_reported_once(engine):
     box = DeviceArray((6,), np.int32)
     E.support_box(t, (3, 4, 5), box)
     assert box.download().tolist() == [0, 0, 0, 2, 3, 4]
+
+
+def test_kept_results_leave_pinned_memory(engine):
+    """A caller that keeps every result: pinned ones up to the bound, then
+    ordinary arrays, the same values; dropping them makes room again."""
+    n, s = 18, 0.5
+    origin = np.array([-(n - 1) / 2 * s, s / 2, -(n - 1) / 2 * s])
+    rng = np.random.default_rng(4)
+    dens = (1.0 + 0.3 * rng.random((n, n, n))).astype(np.float32)
+    src = Source("varian_clinac_6MV")
+    blk = Block()
+    blk.set_square(6)
+    args = (src, blk, Phantom(dens, origin, [s] * 3),
+            dict(SETTINGS, thetas=default_thetas(4)))
+    one = Conehead(engine)
+    one._host._max_alive = 5 * 4 * n ** 3
+    kept = []
+    for _ in range(4):
+        kept.append((one.calculate(*args), one.dose_grid_terma))
+    pinned = [not a.flags.owndata for pair in kept for a in pair]
+    assert pinned == [True] * 5 + [False] * 3
+    for dose, terma in kept:
+        assert np.array_equal(dose, kept[0][0])
+        assert np.array_equal(terma, kept[0][1])
+        dose *= 2.0                      # each is the caller's own
+        dose *= 0.5
+    ref = kept[0][0].copy()
+    del kept, dose, terma
+    assert not one.calculate(*args).flags.owndata
+    assert np.array_equal(one.dose_grid.dose, ref)

@@ -153,6 +153,7 @@ def test_result_takes_the_dose_layout(order):
 class Block:
     """A pooled buffer of either kind; `live` holds those not freed."""
     live = []
+    ptr = 1
 
     def __init__(self, shape, dtype=np.uint8):
         self.shape = shape if isinstance(shape, tuple) else (shape,)
@@ -162,6 +163,7 @@ class Block:
 
     def free(self):
         Block.live.remove(self)
+        self.ptr = None
 
 
 @pytest.fixture(params=["device", "host"])
@@ -200,6 +202,31 @@ def test_full_pool_keeps_the_shape_in_use(pool):
     assert sorted(x.nbytes for x in Block.live) == [20, 40, 40]
     p.clear()
     assert Block.live == [] and p._bytes == 0 and not p._free
+
+
+def test_pinned_bytes_are_bounded(monkeypatch):
+    """try_get counts what is handed out: buffers that callers keep end the
+    pinned memory of a pool, idle ones of other sizes make room, and what is
+    dropped can be had again."""
+    monkeypatch.setattr(Block, "live", [])
+    monkeypatch.setattr(device, "HostBuffer", Block)
+    p = device.HostPool(max_free_bytes=60, max_bytes=100)
+    kept = [p.try_get(40), p.try_get(40)]
+    assert None not in kept and p.try_get(40) is None
+    p.put(kept.pop())
+    assert p.try_get(60) is not None         # the idle 40 bytes are freed
+    assert sorted(b.nbytes for b in Block.live) == [40, 60]
+    assert p.try_get(1) is None
+    p.put(kept.pop())
+    idle = p.try_get(40)
+    assert idle is not None and p.try_get(40) is None
+
+    def none(nbytes):
+        raise _lib.CHError(_lib.CH_ERR_NOMEM, "no pinned memory")
+
+    monkeypatch.setattr(device, "HostBuffer", none)
+    p.put(idle)
+    assert p.try_get(30) is None and p.try_get(40) is None
 
 
 def test_short_memory_empties_the_pools(monkeypatch):
