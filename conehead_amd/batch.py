@@ -149,6 +149,11 @@ class DevicePool:
         with self._lock:
             drop_idle(self, -1)
 
+    def close(self):
+        """Frees the idle buffers, and those given back later."""
+        self._max = -1
+        self.clear()
+
 
 class BatchHandle:
     """A launched batch: its completion event and device outputs."""

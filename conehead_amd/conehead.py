@@ -96,14 +96,7 @@ class Conehead:
     def __init__(self, engine=None):
         self._engine = engine
         self._stream = None
-        # Device grids and pinned results are kept between calls: an
-        # allocation of each grid cost 0.17 ms, a download into fresh
-        # pageable memory ran at a quarter of the link.  Results view pinned
-        # buffers, which return to the pool when their last array is gone.
-        # A caller that keeps its results gets ordinary memory once the
-        # pinned results alive and idle would pass max_bytes.
-        self._pool = DevicePool(max_free_bytes=1 << 30)
-        self._host = HostPool(max_free_bytes=512 << 20, max_bytes=1 << 30)
+        self._pools = None
         self.dose_grid = None
 
     @property
@@ -113,6 +106,28 @@ class Conehead:
         if self._stream is None:
             self._stream = Stream()
         return self._stream
+
+    def _pool_pair(self):
+        """(device grids, pinned results) kept between calls: an allocation
+        of each grid cost 0.17 ms, a download into fresh pageable memory ran
+        at a quarter of the link.  Results view pinned buffers, which return
+        to the pool when their last array is gone.  A caller that keeps its
+        results gets ordinary memory once the pinned ones alive and idle
+        would pass max_bytes."""
+        if self._pools is None:
+            self._pools = (DevicePool(max_free_bytes=1 << 30),
+                           HostPool(max_free_bytes=512 << 20,
+                                    max_bytes=1 << 30))
+        return self._pools
+
+    def close(self):
+        """Frees the device grids and pinned buffers kept between calls (not
+        the results handed out: their memory goes with their last view).  A
+        later calculate() keeps its own again."""
+        if self._pools is not None:
+            for pool in self._pools:
+                pool.close()
+            self._pools = None
 
     @property
     def engine(self):
@@ -139,10 +154,11 @@ class Conehead:
         swap = settings.get("density_xy_swap", True)
         grid = settings.get("dose_grid")
         s = self.stream
+        grids, pinned = self._pool_pair()
         held = []                   # back to the pool once the stream is idle
 
         def device(shape, dtype=np.float32):
-            held.append(self._pool.get(tuple(shape), np.dtype(dtype)))
+            held.append(grids.get(tuple(shape), np.dtype(dtype)))
             return held[-1]
 
         def upload(arr):
@@ -253,7 +269,7 @@ class Conehead:
                 _engine.convolve(plan, d_terma, d_dose, d_box, stream=s)
             for d in (d_dose, d_terma, d_dens):
                 if d is not None:
-                    results.append((d, self._host.try_get(d.nbytes)))
+                    results.append((d, pinned.try_get(d.nbytes)))
                     if results[-1][1] is not None:
                         d.download_async(results[-1][1], stream=s)
             s.sync()
@@ -266,12 +282,12 @@ class Conehead:
         except Exception:
             for _, h in results:
                 if h is not None:
-                    self._host.put(h)
+                    pinned.put(h)
             raise
         arrays = [d.download(stream=s) if h is None
-                  else self._host.as_array(h, shape) for d, h in results]
+                  else pinned.as_array(h, shape) for d, h in results]
         for d in held:
-            self._pool.put(d)
+            grids.put(d)
         self.dose_grid_terma = arrays[1]
         self.dose_grid_densities = dens if d_dens is None else arrays[2]
         self.dose_grid.dose = arrays[0]

@@ -333,3 +333,8 @@ class HostPool:
     def clear(self):
         with self._lock:
             drop_idle(self, -1)
+
+    def close(self):
+        """Frees the idle buffers, and those given back later."""
+        self._max = -1
+        self.clear()

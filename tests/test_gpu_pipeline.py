@@ -229,7 +229,7 @@ def test_kept_results_leave_pinned_memory(engine):
     args = (src, blk, Phantom(dens, origin, [s] * 3),
             dict(SETTINGS, thetas=default_thetas(4)))
     one = Conehead(engine)
-    one._host._max_alive = 5 * 4 * n ** 3
+    one._pool_pair()[1]._max_alive = 5 * 4 * n ** 3
     kept = []
     for _ in range(4):
         kept.append((one.calculate(*args), one.dose_grid_terma))
@@ -242,5 +242,18 @@ def test_kept_results_leave_pinned_memory(engine):
         dose *= 0.5
     ref = kept[0][0].copy()
     del kept, dose, terma
-    assert not one.calculate(*args).flags.owndata
-    assert np.array_equal(one.dose_grid.dose, ref)
+    dose = one.calculate(*args)
+    assert not dose.flags.owndata
+    assert np.array_equal(dose, ref)
+    # and an instance gives back what it keeps, not what it handed out
+    grids, pinned = one._pool_pair()
+    assert grids._bytes > 0
+    one.close()
+    assert grids._bytes == 0 and pinned._bytes == 0
+    assert np.array_equal(dose, ref)
+    del dose
+    one.dose_grid = one.dose_grid_terma = None
+    assert pinned._bytes == 0                 # freed, not kept
+    assert np.array_equal(one.calculate(*args), ref)
+    one.close()
+    one.close()

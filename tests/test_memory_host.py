@@ -289,3 +289,13 @@ def test_tiles_of_earlier_workgroups_are_not_read(tmp_path, monkeypatch):
                            set_tile=lambda *t: None)
     with pytest.raises(Timed):
         autotune.tune(plan)
+
+
+def test_unused_instances_can_be_copied():
+    """A Conehead that has not computed holds nothing of the process."""
+    import copy
+    import pickle
+    from conehead_amd.conehead import Conehead
+    for one in (copy.deepcopy(Conehead()),
+                pickle.loads(pickle.dumps(Conehead()))):
+        assert one.dose_grid is None
