@@ -132,21 +132,26 @@ def test_accumulate_and_direct_gather(engine, kern):
     assert rel_err(both - base, gather) < TOL
 
 
-def test_zero_support_leaves_no_stale_values(engine, kern):
+@pytest.mark.parametrize("shape", [
+    (24, 17, 20),                  # odd y: an unpaired line; general passes
+    (40, 37, 44),                  # the same through the two-stage passes
+    (40, 37, 20)])                 # two-stage x and y, general z
+def test_zero_support_leaves_no_stale_values(engine, kern, shape):
     """The forward passes skip zero line pairs and zero slabs of T (support
     flags behind the work grid) and leave those parts of the work grid
     unwritten.  A sparse T convolved right after dense ones on the same
     work grid must give the same bits whatever the dense T was, agree with
     the gather, and an all-zero T must give a dose of exact zeros."""
     rng = np.random.default_rng(17)
-    shape, vs = (24, 17, 20), (0.35, 0.3, 0.4)   # odd y: an unpaired line
+    vs = (0.35, 0.3, 0.4)
     cs = cone_set(kern, 6, 4)
     plan = engine.plan(shape, vs, cs)
     dense = (0.5 + rng.random(shape)).astype(np.float32)
     sparse = np.zeros(shape, np.float32)
     sparse[3] = 1.0 + rng.random(shape[1:])        # a full slab
     sparse[11, 4:9] = 1.0 + rng.random((5, shape[2]))
-    sparse[11, 16] = 2.0                            # the unpaired line only
+    sparse[11, -1] = 2.0                            # its unpaired line
+    sparse[15, -1] = 2.0                            # the unpaired line only
     sparse[19, 0:2, 7] = 3.0                        # one line pair, one z
     after_a = (run_fft(plan, dense), run_fft(plan, sparse))[1]
     after_b = (run_fft(plan, 3.0 * dense), run_fft(plan, sparse))[1]
@@ -332,13 +337,19 @@ def test_two_stage_passes(engine, kern, frame):
             assert spectral_frame(shape)[0][axis] == frame
             plan = E.Plan(shape, (0.3, 0.3, 0.3), cs)
             plan.spectrum()
-            T = rng.random(shape).astype(np.float32)
+            dense = (0.5 + rng.random(shape)).astype(np.float32)
+            T = dense.copy()
             T[: shape[0] // 3] = 0.0
-            T[:, shape[1] // 2] = 0.0
+            pair = shape[1] // 4 * 2
+            T[:, pair:pair + 2] = 0.0
+            T[-1, :-1] = 0.0            # an unpaired line where y is odd
             d_t = DeviceArray.from_host(T)
             d_g = DeviceArray(shape, np.float32)
             E.convolve(plan, d_t, d_g)
             ref = run_fft(plan, T)
+            for scale in (1.0, -3.0):
+                run_fft(plan, np.float32(scale) * dense)
+                assert np.array_equal(run_fft(plan, T), ref), (axis, n)
             assert rel_err(ref, d_g.download()) < TOL, (axis, n)
             outs = [DeviceArray(shape, np.float32) for _ in range(3)]
             for w in (2, 4, 8, 16):
@@ -350,10 +361,11 @@ def test_two_stage_passes(engine, kern, frame):
 
 
 def test_frame_lengths_agree(engine, kern):
-    """The frame of ch_plan_spectrum is spectral_frame's, from one voxel
-    past the two-stage lengths."""
+    """The frame of ch_plan_spectrum is spectral_frame's for every axis
+    length up to past the two-stage ones, on each axis in turn."""
     cs = cone_set(kern, 3, 4)
-    for n in list(range(1, 70, 3)) + [32, 33, 36, 37, 41, 63, 68, 113, 122,
-                                      125, 126, 188, 200, 201, 260]:
-        plan = E.Plan((n, 3, 2), (0.3, 0.3, 0.3), cs)
-        assert plan.spectrum()[0] == spectral_frame((n, 3, 2))[0], n
+    for n in list(range(1, 206)) + [260, 313, 400, 486, 512]:
+        shape = [3, 2, 1]
+        shape[n % 3] = n
+        plan = E.Plan(shape, (0.3, 0.3, 0.3), cs)
+        assert plan.spectrum()[0] == spectral_frame(shape)[0], n
