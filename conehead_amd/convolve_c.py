@@ -118,12 +118,11 @@ def _laid_out_as(dose, part):
     return like
 
 
-def _convert(dst, src, accumulate=False):
+def _convert(dst, src):
     types = {np.dtype(np.float32): _lib.CH_F32,
              np.dtype(np.float64): _lib.CH_F64}
     _lib.check(_lib.lib().ch_convert(dst.ptr, types[dst.dtype], src.ptr,
-                                     types[src.dtype], dst.size,
-                                     1 if accumulate else 0, None))
+                                     types[src.dtype], dst.size, 0, None))
 
 
 def convolve_c(dose_grid_terma, dose_grid_dose, dose_grid_dim, thetas, phis,

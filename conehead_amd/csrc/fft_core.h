@@ -234,52 +234,6 @@ __device__ __forceinline__ void dft(float2 (&v)[9])
     }
 }
 
-// 25 = 5 x 5: DFT5 over n1 of x[5 n1 + n2], twiddle W25^(n2 k1), DFT5 over
-// n2, output k1 + 5 k2.
-template <bool INV, bool H = false>
-__device__ __forceinline__ void dft(float2 (&v)[25])
-{
-    static_assert(!H, "odd length");
-    // W25^m = (cos, -sin) forward, (cos, sin) inverse, at m = n2 k1
-    constexpr float c[17] = {
-        1.0f, 0.96858316112863108f, 0.87630668004386358f,
-        0.72896862742141155f, 0.53582679497899655f, 0.30901699437494745f,
-        0.062790519529313527f, -0.1873813145857246f, -0.42577929156507272f,
-        -0.63742398974868975f, -0.80901699437494734f, -0.92977648588825135f,
-        -0.99211470131447776f, -0.99211470131447788f, -0.92977648588825146f,
-        -0.80901699437494778f, -0.63742398974868952f};
-    constexpr float s[17] = {
-        0.0f, 0.24868988716485479f, 0.48175367410171532f,
-        0.68454710592868862f, 0.84432792550201508f, 0.95105651629515353f,
-        0.99802672842827156f, 0.98228725072868872f, 0.90482705246601947f,
-        0.77051324277578925f, 0.58778525229247325f, 0.36812455268467814f,
-        0.12533323356430454f, -0.12533323356430429f, -0.36812455268467792f,
-        -0.58778525229247269f, -0.77051324277578936f};
-    float2 t[5][5];
-#pragma unroll
-    for (int n2 = 0; n2 < 5; ++n2) {
-        float2 u[5];
-#pragma unroll
-        for (int n1 = 0; n1 < 5; ++n1)
-            u[n1] = v[5 * n1 + n2];
-        dft<INV>(u);
-#pragma unroll
-        for (int k1 = 0; k1 < 5; ++k1) {
-            const int m = n2 * k1;
-            t[k1][n2] = m == 0 ? u[k1]
-                               : cmul(u[k1], make_float2(c[m], INV ? s[m]
-                                                                   : -s[m]));
-        }
-    }
-#pragma unroll
-    for (int k1 = 0; k1 < 5; ++k1) {
-        dft<INV>(t[k1]);
-#pragma unroll
-        for (int k2 = 0; k2 < 5; ++k2)
-            v[k1 + 5 * k2] = t[k1][k2];
-    }
-}
-
 // N = A B with A and B coprime: the index maps n = B a + A b and k = (k mod A,
 // k mod B) turn the DFT into A- and B-point ones without twiddles.  Zero
 // inputs given as constants fold away (the two-stage passes are compiled

@@ -88,8 +88,8 @@ __global__ void zero_kernel(uint8_t* p, size_t n)
         p[j] = 0;
 }
 
-// Elementwise conversion between FP32 and FP64 grids, dst = src or
-// dst += src (the sum rounded once in the destination type).
+// Elementwise conversion between FP32 and FP64 grids, dst = src or dst += src,
+// src rounded to the destination type first.
 template <typename D, typename S>
 __global__ void convert_kernel(D* __restrict__ dst, const S* __restrict__ src,
                                size_t n, int accumulate)
@@ -518,7 +518,7 @@ ch_status ch_host_add_f32(double* h_dst, const float* h_src, int64_t n)
 {
     CH_REQUIRE(n >= 0 && (n == 0 || (h_dst && h_src)),
                "ch_host_add_f32: bad arguments");
-    // 16 bytes read and 8 written per element: one thread reaches a quarter
+    // 12 bytes read and 8 written per element: one thread reaches a quarter
     // of what four do; below 2^17 elements each, starting them costs more
     const int parts = (int)std::min<int64_t>(4, std::max<int64_t>(1, n >> 17));
     auto add = [=](int p) {

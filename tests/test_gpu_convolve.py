@@ -409,3 +409,23 @@ def test_support_box_remainders(engine, shape):
             assert box.tolist() == idx.min(0).tolist() + idx.max(0).tolist()
         else:
             assert (box[:3] > box[3:]).all()
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 1000])
+@pytest.mark.parametrize("to,of", [("f4", "f8"), ("f8", "f4"), ("f4", "f4"),
+                                   ("f8", "f8")])
+def test_convert(engine, to, of, n):
+    """ch_convert between the element types, assigned and accumulated (in
+    the destination type), bit for bit."""
+    from conehead_amd import _lib
+    from conehead_amd.device import DeviceArray
+    types = {"f4": _lib.CH_F32, "f8": _lib.CH_F64}
+    rng = np.random.default_rng(n)
+    src, base = rng.random(n).astype(of), rng.random(n).astype(to)
+    d_src = DeviceArray.from_host(src)
+    for accumulate in (0, 1):
+        d = DeviceArray.from_host(base)
+        _lib.check(_lib.lib().ch_convert(d.ptr, types[to], d_src.ptr,
+                                         types[of], n, accumulate, None))
+        want = base + src.astype(to) if accumulate else src.astype(to)
+        assert np.array_equal(d.download(), want)
