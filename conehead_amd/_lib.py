@@ -138,6 +138,8 @@ SIGNATURES = {
     "ch_memcpy_d2h": (ctypes.c_int32, [c_vp, c_vp, c_size, c_vp]),
     "ch_memcpy_d2h_async": (ctypes.c_int32, [c_vp, c_vp, c_size, c_vp]),
     "ch_host_add_f32": (ctypes.c_int32, [c_vp, c_vp, ctypes.c_int64]),
+    "ch_host_add_f32_strided": (ctypes.c_int32, [c_vp, c_vp, c_i64p, c_i64p,
+                                                 c_i64p]),
     "ch_memcpy_d2d": (ctypes.c_int32, [c_vp, c_vp, c_size, c_vp]),
     "ch_zero": (ctypes.c_int32, [c_vp, c_size, c_vp]),
     "ch_host_alloc": (ctypes.c_int32, [c_vpp, c_size]),

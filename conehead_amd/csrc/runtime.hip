@@ -420,6 +420,34 @@ void release_stage_tables(hipStream_t s)
 
 }  // namespace ch
 
+namespace ch {
+
+// work(first, last) over [0, n) in up to four parts, each in a thread of its
+// own while threads can be had; below 2^17 elements each, starting them costs
+// more.
+template <typename F>
+static void host_parts(int64_t n, int64_t elements, const F& work)
+{
+    const int parts = (int)std::min<int64_t>(
+        {4, n, std::max<int64_t>(1, elements >> 17)});
+    std::thread t[3];
+    int started = 0;
+    try {
+        for (; started < parts - 1; ++started)
+            t[started] = std::thread(work, n * (started + 1) / parts,
+                                     n * (started + 2) / parts);
+    } catch (...) {
+        // no more threads: the rest is done here
+    }
+    work((int64_t)0, parts > 0 ? n / parts : 0);
+    for (int p = started + 1; p < parts; ++p)
+        work(n * p / parts, n * (p + 1) / parts);
+    for (int p = 0; p < started; ++p)
+        t[p].join();
+}
+
+}  // namespace ch
+
 using namespace ch;
 
 extern "C" {
@@ -519,28 +547,47 @@ ch_status ch_host_add_f32(double* h_dst, const float* h_src, int64_t n)
     CH_REQUIRE(n >= 0 && (n == 0 || (h_dst && h_src)),
                "ch_host_add_f32: bad arguments");
     // 12 bytes read and 8 written per element: one thread reaches a quarter
-    // of what four do; below 2^17 elements each, starting them costs more
-    const int parts = (int)std::min<int64_t>(4, std::max<int64_t>(1, n >> 17));
-    auto add = [=](int p) {
-        const int64_t end = n * (p + 1) / parts;
-        for (int64_t i = n * p / parts; i < end; ++i)
+    // of what four do
+    ch::host_parts(n, n, [=](int64_t i, int64_t end) {
+        for (; i < end; ++i)
             h_dst[i] += (double)h_src[i];
-    };
-    std::thread t[3];
-    int started = 0;
-    try {
-        while (started < parts - 1) {
-            t[started] = std::thread(add, started + 1);
-            ++started;
-        }
-    } catch (...) {
-        // no more threads: the rest is added here
-    }
-    add(0);
-    for (int p = started + 1; p < parts; ++p)
-        add(p);
-    for (int p = 0; p < started; ++p)
-        t[p].join();
+    });
+    return CH_OK;
+}
+
+ch_status ch_host_add_f32_strided(double* h_dst, const float* h_src,
+                                  const int64_t shape[3],
+                                  const int64_t dst_strides[3],
+                                  const int64_t src_strides[3])
+{
+    CH_REQUIRE(shape && dst_strides && src_strides,
+               "ch_host_add_f32_strided: null pointer");
+    const int64_t n0 = shape[0], n1 = shape[1], n2 = shape[2];
+    CH_REQUIRE(n0 >= 0 && n1 >= 0 && n2 >= 0,
+               "ch_host_add_f32_strided: negative shape");
+    if (n0 == 0 || n1 == 0 || n2 == 0)
+        return CH_OK;
+    CH_REQUIRE(h_dst && h_src, "ch_host_add_f32_strided: null array");
+    const int64_t d0 = dst_strides[0], d1 = dst_strides[1],
+                  d2 = dst_strides[2];
+    const int64_t s0 = src_strides[0], s1 = src_strides[1],
+                  s2 = src_strides[2];
+    // Tiles of a cache line of each side (8 doubles along axis 1, 16 floats
+    // along axis 2): where both axes step over powers of two, a line is gone
+    // from its set before the next row comes back to it.
+    ch::host_parts(n0, n0 * n1 * n2, [=](int64_t i, int64_t end) {
+        for (; i < end; ++i)
+            for (int64_t k = 0; k < n2; k += 16)
+                for (int64_t j = 0; j < n1; j += 8) {
+                    double* d = h_dst + i * d0 + j * d1 + k * d2;
+                    const float* s = h_src + i * s0 + j * s1 + k * s2;
+                    const int64_t nk = std::min<int64_t>(16, n2 - k);
+                    const int64_t nj = std::min<int64_t>(8, n1 - j);
+                    for (int64_t z = 0; z < nk; ++z)
+                        for (int64_t x = 0; x < nj; ++x)
+                            d[z * d2 + x * d1] += (double)s[z * s2 + x * s1];
+                }
+    });
     return CH_OK;
 }
 

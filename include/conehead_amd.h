@@ -49,6 +49,13 @@ ch_status ch_memcpy_d2h_async(void* h_dst, const void* d_src, size_t bytes,
                               void* stream);
 /* Host arrays: h_dst[i] += (double)h_src[i], on up to four threads. */
 ch_status ch_host_add_f32(double* h_dst, const float* h_src, int64_t n);
+/* The same for arrays of three axes with strides in elements (of any sign; the
+ * elements of h_dst must not overlap), in tiles over axes 1 and 2: fastest
+ * where h_dst is contiguous along axis 1 and h_src along axis 2. */
+ch_status ch_host_add_f32_strided(double* h_dst, const float* h_src,
+                                  const int64_t shape[3],
+                                  const int64_t dst_strides[3],
+                                  const int64_t src_strides[3]);
 /* Device-to-device copy by a kernel (16-byte aligned pointers). */
 ch_status ch_memcpy_d2d(void* d_dst, const void* d_src, size_t bytes,
                         void* stream);

@@ -133,21 +133,40 @@ def test_dropin_dose_layouts(dropin, layout):
 
 
 @pytest.mark.parametrize("order", [(0, 1, 2), (2, 1, 0), (1, 0, 2),
-                                   (0, 2, 1), (1, 2, 0)])
-def test_result_takes_the_dose_layout(order):
-    """What is added to a dose lies in memory as the dose does, so that the
-    sum runs along both (a C-ordered one under a Fortran-ordered dose costs
-    a cache line per element)."""
-    shape = (6, 5, 7)
-    part = np.random.default_rng(1).random(shape).astype(np.float32)
-    dose = np.empty([shape[a] for a in order]).transpose(np.argsort(order))
-    assert dose.shape == shape
-    got = convolve_c._laid_out_as(dose, part)
-    assert np.array_equal(got, part)
-    assert np.argsort(got.strides).tolist() == \
-        np.argsort(dose.strides).tolist()
-    if order == (0, 1, 2):
-        assert got is part
+                                   (0, 2, 1), (1, 2, 0), (2, 0, 1)])
+@pytest.mark.parametrize("shape", [(6, 5, 7), (8, 16, 16), (1, 17, 9),
+                                   (33, 1, 40), (70, 65, 130)])
+def test_sum_into_any_axis_order(monkeypatch, order, shape):
+    """Tiles and remainders, one and four threads, axes reversed and of
+    every other element: numpy's sum, and nothing beside the dose's own
+    elements."""
+    monkeypatch.setattr(_lib, "lib", _lib.load)
+    rng = np.random.default_rng(sum(shape))
+    part = rng.random(shape).astype(np.float32)
+    for step in (slice(None), slice(None, None, -1), slice(None, None, 2)):
+        n = 2 if step.step == 2 else 1
+        whole = rng.random([n * shape[a] for a in order])
+        before = whole.copy()
+        view = [a.transpose(np.argsort(order))[step, step, step]
+                for a in (whole, before)]
+        assert view[0].shape == shape
+        convolve_c._add(view[0], part)
+        view[1] += part
+        assert np.array_equal(whole, before)
+
+
+def test_sum_into_overlapping_elements(monkeypatch):
+    """Doses whose elements share memory stay numpy's."""
+    monkeypatch.setattr(_lib, "lib", _lib.load)
+    part = np.ones((4, 5, 6), np.float32)
+    for strides in ((8, 8, 8), (8, 0, 16), (16, 8, 40), (8, 16, 8)):
+        base = np.zeros(400)
+        want = base.copy()
+        dose, ref = [np.lib.stride_tricks.as_strided(b, (4, 5, 6), strides)
+                     for b in (base, want)]
+        convolve_c._add(dose, part)
+        np.add(ref, part, out=ref)
+        assert np.array_equal(base, want)
 
 
 class Block:
