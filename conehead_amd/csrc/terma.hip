@@ -569,8 +569,8 @@ __device__ __forceinline__ double sample_sums(const TermaParams& P,
 //
 // 17 VALU instructions per step, against 28 when the steps left were
 // counted per axis and the sum was FP32 with Kahan compensation (FP64 runs
-// at the FP32 rate here, so the FP64 sum needs two instructions where the
-// compensated one needs seven); the 128^3 beam 127.4 -> 125.8 us, 24 MLC
+// at 0.9 of the FP32 rate here, so the FP64 sum needs two instructions where
+// the compensated one needs seven); the 128^3 beam 127.4 -> 125.8 us, 24 MLC
 // beams 4439 -> 4217 us.  What bounds the walk are its loads: each touches
 // one line per (x, y) row the wavefront's lanes stand on.
 constexpr int kWalkBatch = 8;
