@@ -302,7 +302,8 @@ class HostPool:
             b = take_idle(self, int(nbytes))
         if b is None:
             b = HostBuffer(nbytes)
-            self._alive.add(b)
+            with self._lock:
+                self._alive.add(b)
         return b
 
     def try_get(self, nbytes):
