@@ -73,13 +73,14 @@ struct PairFns {
 // The launches of frame length F; false when it has no pair of radices.
 bool fft_pair(int F, PairFns* out);
 
-// Their definitions, by translation unit (fft_pair_*.hip).
-PairFns pair_fns_72(), pair_fns_80(), pair_fns_90(), pair_fns_96(),
-    pair_fns_100(), pair_fns_108(), pair_fns_120(), pair_fns_128(),
-    pair_fns_144(), pair_fns_150(), pair_fns_160(), pair_fns_162(),
-    pair_fns_180(), pair_fns_192(), pair_fns_200(), pair_fns_216(),
-    pair_fns_240(), pair_fns_256(), pair_fns_270(), pair_fns_288(),
-    pair_fns_300(), pair_fns_320(), pair_fns_324(), pair_fns_360(),
-    pair_fns_384(), pair_fns_400();
+// The frame lengths (batch.PAIR_FRAMES has them too), X(F) for each; their
+// radices and launches are defined by translation unit (fft_pair_*.hip).
+#define CH_PAIR_FRAMES(X)                                                   \
+    X(72) X(80) X(90) X(96) X(100) X(108) X(120) X(128) X(144) X(150)       \
+    X(160) X(162) X(180) X(192) X(200) X(216) X(240) X(256) X(270) X(288)   \
+    X(300) X(320) X(324) X(360) X(384) X(400)
+#define CH_PAIR_DECLARE(F) PairFns pair_fns_##F();
+CH_PAIR_FRAMES(CH_PAIR_DECLARE)
+#undef CH_PAIR_DECLARE
 
 }  // namespace ch

@@ -1409,32 +1409,9 @@ static BeamIO table_io(void* d, int32_t nb)
 bool fft_pair(int F, PairFns* out)
 {
     switch (F) {
-    case 72: *out = pair_fns_72(); return true;
-    case 80: *out = pair_fns_80(); return true;
-    case 90: *out = pair_fns_90(); return true;
-    case 96: *out = pair_fns_96(); return true;
-    case 100: *out = pair_fns_100(); return true;
-    case 108: *out = pair_fns_108(); return true;
-    case 120: *out = pair_fns_120(); return true;
-    case 128: *out = pair_fns_128(); return true;
-    case 144: *out = pair_fns_144(); return true;
-    case 150: *out = pair_fns_150(); return true;
-    case 160: *out = pair_fns_160(); return true;
-    case 162: *out = pair_fns_162(); return true;
-    case 180: *out = pair_fns_180(); return true;
-    case 192: *out = pair_fns_192(); return true;
-    case 200: *out = pair_fns_200(); return true;
-    case 216: *out = pair_fns_216(); return true;
-    case 240: *out = pair_fns_240(); return true;
-    case 256: *out = pair_fns_256(); return true;
-    case 270: *out = pair_fns_270(); return true;
-    case 288: *out = pair_fns_288(); return true;
-    case 300: *out = pair_fns_300(); return true;
-    case 320: *out = pair_fns_320(); return true;
-    case 324: *out = pair_fns_324(); return true;
-    case 360: *out = pair_fns_360(); return true;
-    case 384: *out = pair_fns_384(); return true;
-    case 400: *out = pair_fns_400(); return true;
+#define CH_PAIR_CASE(F) case F: *out = pair_fns_##F(); return true;
+        CH_PAIR_FRAMES(CH_PAIR_CASE)
+#undef CH_PAIR_CASE
     default: return false;
     }
 }

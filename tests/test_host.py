@@ -268,3 +268,23 @@ def test_convolve_c_dropin_argument_errors():
         convolve_c(t, np.zeros((4, 4, 5)), dims, default_thetas(2), phis, k)
     with pytest.raises(KeyError):
         convolve_c(t, d, dims, default_thetas(2), [12.0], k)
+
+
+def test_two_stage_frames_are_listed_once():
+    """batch.PAIR_FRAMES are the lengths that the library's list expands to,
+    and each has its radices in one fft_pair_*.hip."""
+    import glob
+    import os
+    import re
+    from conehead_amd import batch
+    csrc = os.path.join(os.path.dirname(batch.__file__), "csrc")
+    with open(os.path.join(csrc, "fft_pair.h")) as f:
+        listed = [int(n) for n in re.findall(r" X\((\d+)\)", f.read())]
+    pairs = []
+    for path in glob.glob(os.path.join(csrc, "fft_pair_?.hip")):
+        with open(path) as f:
+            pairs += [tuple(map(int, m)) for m in re.findall(
+                r"CH_PAIR\((\d+), (\d+), (\d+)\)", f.read())]
+    assert tuple(listed) == batch.PAIR_FRAMES
+    assert sorted(p[0] for p in pairs) == listed
+    assert all(f == a * b and a % 2 == 0 for f, a, b in pairs)
